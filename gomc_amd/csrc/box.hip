@@ -404,207 +404,6 @@ __global__ void __launch_bounds__(kBlock) BoxInterKernel(const BoxInterArgs a) {
   FinishPartials(part, a.partials, a.counter, a.result);
 }
 
-// ------------------------------------------------------ structure factor --
-// S(k) = sum_j q_j (cos, sin)(k . r_j) over all charged atoms
-// (Ewald.cpp:193-274), then the per-k energy prefact (Re^2 + Im^2)
-// (Ewald.cpp:375-406).
-//
-// The k list comes in GOMC's x, y, z loop order, so it is made of runs of
-// consecutive nz at fixed (nx, ny).  KSegmentsKernel cuts it into segments:
-// pieces of a run of at most kSeg vectors.  Along a segment the phase of an
-// atom advances by one complex product, e^{i k_{n+1} . r} =
-// e^{i k_n . r} e^{i dz z}, with dz = 2 pi / L_z for every segment, so a
-// segment costs one sincos per atom (its first vector; the step's phase is
-// made once per atom) and one complex product per vector.  The first pass
-// takes one segment per thread and one chunk of atoms per work item
-// (per-chunk sums into part[chunk][k][2]); the second adds the chunks in
-// order, one k per thread.  Both passes read the segment count from device
-// memory, so a launch never waits on the host.
-struct SumsArgs {
-  const double *x, *y, *z, *q;
-  const int *mol;  // may be null: every atom counts
-  int natoms, K;
-  const double *kx, *ky, *kz, *pref;
-  const int *kseg;   // segment starts [nseg + 1], kseg[nseg] = K
-  const int *nseg;   // device
-  double cx, cy, cz;  // KVectorsOrth's spacings 2 pi / L_d (cz: every segment's nz step)
-  int nmax[3];        // KVectorsOrth's |n_d| bounds: the phase tables' ranges
-  int tabAtoms;       // atoms per LDS tile (their phase tables fill the dynamic LDS)
-  double *sumR, *sumI;
-  double *part;      // [chunks][K][2]
-  Partial4 *partials;
-  unsigned *counter;
-  double *result;
-};
-
-__device__ __forceinline__ bool RunStart(const double *kx, const double *ky, const double *kz,
-                                         int k) {
-  return k == 0 || kx[k] != kx[k - 1] || ky[k] != ky[k - 1] || !(kz[k] > kz[k - 1]);
-}
-
-// One workgroup of kSegThreads: each thread takes a contiguous range of the
-// K vectors; a max-scan carries the run start in effect into each range, a
-// sum-scan places each range's segments.
-__global__ void __launch_bounds__(kSegThreads) KSegmentsKernel(const double *kx, const double *ky,
-                                                               const double *kz, int K, int *kseg,
-                                                               int *nseg) {
-  __shared__ int sRun[kSegThreads], sCnt[kSegThreads];
-  const int t = threadIdx.x;
-  const int per = (K + kSegThreads - 1) / kSegThreads;
-  const int lo = min(K, t * per), hi = min(K, lo + per);
-  int last = -1;
-  for (int k = lo; k < hi; ++k)
-    if (RunStart(kx, ky, kz, k)) last = k;
-  sRun[t] = last;
-  __syncthreads();
-  for (int off = 1; off < kSegThreads; off <<= 1) {  // inclusive max-scan
-    const int v = t >= off ? sRun[t - off] : -1;
-    __syncthreads();
-    sRun[t] = max(sRun[t], v);
-    __syncthreads();
-  }
-  const int runAtLo = t > 0 ? sRun[t - 1] : -1;
-  int run = runAtLo, cnt = 0;
-  for (int k = lo; k < hi; ++k) {
-    if (RunStart(kx, ky, kz, k)) run = k;
-    if ((k - run) % kSeg == 0) ++cnt;
-  }
-  sCnt[t] = cnt;
-  __syncthreads();
-  for (int off = 1; off < kSegThreads; off <<= 1) {  // inclusive sum-scan
-    const int v = t >= off ? sCnt[t - off] : 0;
-    __syncthreads();
-    sCnt[t] += v;
-    __syncthreads();
-  }
-  int out = sCnt[t] - cnt;
-  run = runAtLo;
-  for (int k = lo; k < hi; ++k) {
-    if (RunStart(kx, ky, kz, k)) run = k;
-    if ((k - run) % kSeg == 0) kseg[out++] = k;
-  }
-  if (t == kSegThreads - 1) {
-    kseg[sCnt[t]] = K;
-    *nseg = sCnt[t];
-  }
-}
-
-constexpr int kSumsTabBytes = 48 * 1024;  // dynamic LDS of the phase tables
-constexpr int kSumsTabMaxAtoms = 64;
-
-__host__ __device__ inline int SumsTabEntries(const int nmax[3]) {
-  return nmax[0] + nmax[1] + nmax[2] + 3;
-}
-
-__global__ void __launch_bounds__(kBlock) RecipSumsPartKernel(const SumsArgs a) {
-  // per atom of the tile: e^{i n c_d r_d} for n = 0..nmax_d on each axis (a
-  // negative n is the conjugate), so the first phase of a segment at
-  // (nx, ny, nz0) is two complex products instead of a sincos; the nz step
-  // is the z table's n = 1
-  extern __shared__ double2 tab[];
-  __shared__ double sq[kSumsTabMaxAtoms];
-  const int nseg = *a.nseg;
-  const int segBlocks = max(1, (nseg + kBlock - 1) / kBlock);
-  const int chunks = SumsChunks(nseg, a.natoms, a.K);
-  const int aChunk = (a.natoms + chunks - 1) / chunks;
-  const int E = SumsTabEntries(a.nmax), oy = a.nmax[0] + 1, oz = oy + a.nmax[1] + 1;
-  const int T = a.tabAtoms;
-  for (int item = blockIdx.x; item < segBlocks * chunks; item += gridDim.x) {
-    const int seg = (item % segBlocks) * kBlock + threadIdx.x, chunk = item / segBlocks;
-    const bool active = seg < nseg;
-    const int k0 = active ? a.kseg[seg] : 0;
-    const int len = active ? a.kseg[seg + 1] - k0 : 0;
-    // the segment's integer triple (k = c n, one rounding, so rint recovers n)
-    const int nx = active ? min(a.nmax[0], max(0, int(rint(a.kx[k0] / a.cx)))) : 0;
-    const int ny = active ? min(a.nmax[1], max(-a.nmax[1], int(rint(a.ky[k0] / a.cy)))) : 0;
-    const int nz = active ? min(a.nmax[2], max(-a.nmax[2], int(rint(a.kz[k0] / a.cz)))) : 0;
-    const double syn = ny < 0 ? -1.0 : 1.0, szn = nz < 0 ? -1.0 : 1.0;
-    const int iy = oy + abs(ny), iz = oz + abs(nz);
-    double sR[kSeg], sI[kSeg];
-#pragma unroll
-    for (int i = 0; i < kSeg; ++i) sR[i] = sI[i] = 0.0;
-    const int a0 = min(a.natoms, chunk * aChunk), a1 = min(a.natoms, a0 + aChunk);
-    for (int tile = a0; tile < a1; tile += T) {
-      const int tn = min(T, a1 - tile);
-      __syncthreads();
-      if (int(threadIdx.x) < tn) {
-        const int j = tile + threadIdx.x;
-        sq[threadIdx.x] = (!a.mol || a.mol[j] >= 0) ? a.q[j] : 0.0;  // reservoir adds nothing
-      }
-      // each (atom, axis) table by one thread: n = 1 by sincos, then one
-      // complex product per n
-      for (int w = threadIdx.x; w < 3 * tn; w += kBlock) {
-        const int at = w / 3, ax = w - 3 * at, j = tile + at;
-        const double r = ax == 0 ? a.x[j] : (ax == 1 ? a.y[j] : a.z[j]);
-        const double c = ax == 0 ? a.cx : (ax == 1 ? a.cy : a.cz);
-        const int o = ax == 0 ? 0 : (ax == 1 ? oy : oz), n1 = a.nmax[ax];
-        double2 *t = tab + size_t(at) * E + o;
-        double s1, c1;
-        sincos(c * r, &s1, &c1);
-        t[0] = make_double2(1.0, 0.0);
-        double re = c1, im = s1;
-        for (int n = 1; n <= n1; ++n) {
-          t[n] = make_double2(re, im);
-          const double nr = fma(re, c1, -(im * s1));
-          im = fma(re, s1, im * c1);
-          re = nr;
-        }
-      }
-      __syncthreads();
-      if (active)
-        for (int jj = 0; jj < tn; ++jj) {
-          const double qj = sq[jj];
-          if (fabs(qj) < 0.000000001) continue;
-          const double2 *t = tab + size_t(jj) * E;
-          const double2 ex = t[nx], ey = t[iy], ez = t[iz], st = t[oz + 1];
-          const double eyi = syn * ey.y, ezi = szn * ez.y;
-          const double pr = fma(ex.x, ey.x, -(ex.y * eyi)), pi = fma(ex.x, eyi, ex.y * ey.x);
-          double re = fma(pr, ez.x, -(pi * ezi)), im = fma(pr, ezi, pi * ez.x);
-          const double ss = st.y, cs = st.x;
-#pragma unroll
-          for (int i = 0; i < kSeg; ++i) {
-            if (i < len) {
-              sR[i] = fma(qj, re, sR[i]);
-              sI[i] = fma(qj, im, sI[i]);
-            }
-            const double nr = fma(re, cs, -(im * ss));
-            im = fma(re, ss, im * cs);
-            re = nr;
-          }
-        }
-    }
-    if (active) {
-      double *out = a.part + (size_t(chunk) * a.K + k0) * 2;
-#pragma unroll
-      for (int i = 0; i < kSeg; ++i)
-        if (i < len) {
-          out[2 * i] = sR[i];
-          out[2 * i + 1] = sI[i];
-        }
-    }
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) RecipSumsKernel(const SumsArgs a) {
-  __shared__ double red[kBlock / kWave];
-  const int k = blockIdx.x * kBlock + threadIdx.x;
-  const bool active = k < a.K;
-  const int chunks = SumsChunks(*a.nseg, a.natoms, a.K);
-  double sR = 0.0, sI = 0.0, e = 0.0;
-  if (active) {
-    for (int c = 0; c < chunks; ++c) {
-      sR += a.part[(size_t(c) * a.K + k) * 2];
-      sI += a.part[(size_t(c) * a.K + k) * 2 + 1];
-    }
-    a.sumR[k] = sR;
-    a.sumI[k] = sI;
-    e = (sR * sR + sI * sI) * a.pref[k];
-  }
-  Partial4 part{0, 0, 0, 0};
-  part.recip = BlockSum(e, red);
-  FinishPartials(part, a.partials, a.counter, a.result);
-}
-
 // Insertion (+) or removal (-) of one molecule: SwapDestRecip /
 // SwapSourceRecip (Ewald.cpp:478-531, 657-710).
 struct SwapArgs {
@@ -1115,159 +914,6 @@ int BoxInter(gomc_box *b, double *lj, double *real) {
   return GOMC_OK;
 }
 
-// Both passes on stream s.  a carries the arrays: the segments of the k
-// list, part [SumsChunks(nseg) x K x 2], partials [ceil(K / kBlock)],
-// counter (zero, re-armed by the last block) and result [4] (result[2]
-// receives the energy).
-hipError_t LaunchRecipSums(const SumsArgs &a, hipStream_t s) {
-  const size_t tabBytes = size_t(a.tabAtoms) * SumsTabEntries(a.nmax) * sizeof(double2);
-  hipLaunchKernelGGL(RecipSumsPartKernel, dim3(kSumsGrid), dim3(kBlock), tabBytes, s, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int nblocks = std::max(1, (a.K + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL(RecipSumsKernel, dim3(nblocks), dim3(kBlock), 0, s, a);
-  return hipGetLastError();
-}
-
-int BuildKSegments(gomc_box *b) {
-  if (b->K + 1 > b->ksegCap) {
-    if (b->kseg) (void)hipFree(b->kseg);
-    b->kseg = nullptr;
-    b->ksegCap = 0;
-    HIP_TRY(b, hipMalloc(&b->kseg, sizeof(int) * (b->K + 1)));
-    b->ksegCap = b->K + 1;
-  }
-  if (!b->nsegDev) HIP_TRY(b, hipMalloc(&b->nsegDev, sizeof(int)));
-  hipLaunchKernelGGL(KSegmentsKernel, dim3(1), dim3(kSegThreads), 0, b->stream, b->kx, b->ky,
-                     b->kz, b->K, b->kseg, b->nsegDev);
-  HIP_TRY(b, hipGetLastError());
-  HIP_TRY(b, hipMemcpyAsync(&b->nseg, b->nsegDev, sizeof(int), hipMemcpyDeviceToHost, b->stream));
-  return Sync(b);
-}
-
-// The box's arrays for the two structure-factor passes; the scratch
-// (part, partials, counter) is filled in by the caller.
-static SumsArgs BoxSumsArgs(const gomc_box *b) {
-  SumsArgs a;
-  a.x = b->x;
-  a.y = b->y;
-  a.z = b->z;
-  a.q = b->q;
-  a.mol = b->mol;
-  a.natoms = b->natoms;
-  a.K = b->K;
-  a.kx = b->kx;
-  a.ky = b->ky;
-  a.kz = b->kz;
-  a.pref = b->pref;
-  a.kseg = b->kseg;
-  a.nseg = b->nsegDev;
-  a.cx = (1.0 / b->geom.L[0]) * (2.0 * M_PI);  // KVectorsOrth's spacings and ranges
-  a.cy = (1.0 / b->geom.L[1]) * (2.0 * M_PI);
-  a.cz = (1.0 / b->geom.L[2]) * (2.0 * M_PI);
-  for (int i = 0; i < 3; ++i) a.nmax[i] = int(b->recipRcut * b->geom.L[i] / (2.0 * M_PI)) + 1;
-  a.tabAtoms = std::max(1, std::min(kSumsTabMaxAtoms, kSumsTabBytes / int(SumsTabEntries(a.nmax) *
-                                                                           sizeof(double2))));
-  a.sumR = b->sumRnew;
-  a.sumI = b->sumInew;
-  a.result = b->devRes;
-  return a;
-}
-
-// BoxReciprocalSums into the "new" sums; returns the reciprocal energy.
-int RecipSums(gomc_box *b, double *erecip) {
-  if (!b->recipReady) return Fail(b, GOMC_ERR_STATE, "k-vectors not initialised");
-  SumsArgs a = BoxSumsArgs(b);
-  const int nblocks = std::max(1, (b->K + kBlock - 1) / kBlock);
-  int rc = EnsurePartials(b, nblocks);
-  if (rc) return rc;
-  a.partials = b->partials;
-  a.counter = b->counter;
-  const size_t need = size_t(SumsChunks(b->nseg, b->natoms, b->K)) * size_t(b->K) * 2;
-  if (need > b->sumPartCap) {
-    if (b->sumPart) (void)hipFree(b->sumPart);
-    b->sumPart = nullptr;
-    b->sumPartCap = 0;
-    HIP_TRY(b, hipMalloc(&b->sumPart, sizeof(double) * need));
-    b->sumPartCap = need;
-  }
-  a.part = b->sumPart;
-  HIP_TRY(b, LaunchRecipSums(a, b->stream));
-  rc = Sync(b);
-  if (rc) return rc;
-  *erecip = b->hostRes[2];
-  return GOMC_OK;
-}
-
-// ------------------------------------------- allocation-free variant --
-// gomc_recip_sums_noalloc runs the same two passes as RecipSums with its
-// scratch -- the block counter, the second pass's per-block partials and
-// the first pass's per-chunk sums -- in `scratch`, one file-scope device
-// array that each GPU holds until the process ends.  Layout: counter at
-// byte 0, partials at byte 256 (kNoAllocMaxK / kBlock entries), per-chunk
-// sums after them (SumsChunks keeps chunks x K within kSumsPartCap, so
-// 2 kSumsPartCap doubles hold them for K up to kNoAllocMaxK).  Every call on
-// one GPU shares the array: calls that overlap on one GPU race.
-constexpr int kNoAllocMaxK = 1 << 20;
-constexpr size_t kNoAllocPartialsOff = 256;
-constexpr size_t kNoAllocPartOff =
-    kNoAllocPartialsOff + sizeof(Partial4) * size_t(kNoAllocMaxK / kBlock);
-constexpr size_t kNoAllocPartDoubles = 2 * kSumsPartCap;
-constexpr size_t kScratchBytes = kNoAllocPartOff + sizeof(double) * kNoAllocPartDoubles;
-static_assert(kNoAllocPartOff % 256 == 0, "per-chunk sums must stay 256-byte aligned");
-
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
-
-constexpr int kScratchDevices = 64;
-static std::mutex gScratchMu;
-static unsigned char *gScratch[kScratchDevices] = {};
-
-// Device address of this GPU's `scratch`, looked up once per device with
-// that device current (the array's host-side name is not a device address).
-static int ScratchBase(gomc_box *b, unsigned char **base) {
-  if (b->device < 0 || b->device >= kScratchDevices)
-    return Fail(b, GOMC_ERR_ARG, "device index beyond the scratch table");
-  std::lock_guard<std::mutex> lock(gScratchMu);
-  if (!gScratch[b->device]) {
-    void *p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !p)
-      return Fail(b, GOMC_ERR_HIP,
-                  std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-    gScratch[b->device] = static_cast<unsigned char *>(p);
-  }
-  *base = gScratch[b->device];
-  return GOMC_OK;
-}
-
-// The block counter must read zero when the second pass starts; a fill
-// kernel, not a memset, so that a captured stream replays it.
-__global__ void ZeroCounterKernel(unsigned *counter) { *counter = 0u; }
-
-int RecipSumsNoAlloc(gomc_box *b, double *erecip) {
-  if (!b->recipReady) return Fail(b, GOMC_ERR_STATE, "k-vectors not initialised");
-  if (b->K > kNoAllocMaxK)
-    return Fail(b, GOMC_ERR_ARG,
-                "gomc_recip_sums_noalloc takes at most 1048576 k-vectors (use gomc_recip_sums)");
-  const size_t need = size_t(SumsChunks(b->nseg, b->natoms, b->K)) * size_t(b->K) * 2;
-  if (need > kNoAllocPartDoubles)
-    return Fail(b, GOMC_ERR_ARG, "structure-factor chunks exceed the scratch array");
-  unsigned char *base = nullptr;
-  int rc = ScratchBase(b, &base);
-  if (rc) return rc;
-  SumsArgs a = BoxSumsArgs(b);
-  a.counter = reinterpret_cast<unsigned *>(base);
-  a.partials = reinterpret_cast<Partial4 *>(base + kNoAllocPartialsOff);
-  a.part = reinterpret_cast<double *>(base + kNoAllocPartOff);
-  hipLaunchKernelGGL(ZeroCounterKernel, dim3(1), dim3(1), 0, b->stream, a.counter);
-  HIP_TRY(b, hipGetLastError());
-  HIP_TRY(b, LaunchRecipSums(a, b->stream));
-  rc = Sync(b);
-  if (rc) return rc;
-  *erecip = b->hostRes[2];
-  return GOMC_OK;
-}
-
 static double BoxHostMinImage(double d, int axis, const gomc_box *b) {
   const double ax = b->geom.L[axis], half = b->geom.half[axis];
   if (d > half)
@@ -1323,9 +969,10 @@ static void FreeAll(gomc_box *b) {
                   b->tSigSq,   b->tEpsCn,  b->tNHalf,   b->tEpsCn6,  b->tNOver6, b->cellCount,
                   b->cellCursor, b->cellStart, b->cellVec, b->atomCell, b->nbr,   b->kx,
                   b->ky,       b->kz,      b->pref,     b->sumRref,  b->sumIref, b->sumRnew,
-                  b->sumInew,  b->partials, b->counter, b->kseg, b->nsegDev};
+                  b->sumInew,  b->partials, b->counter, b->forcePart};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
+  FreeKPlan(b->kp);
   MPFree(b);
   DevFree(b);
   if (b->trialBuf) (void)hipFree(b->trialBuf);

@@ -23,28 +23,29 @@ struct DevDriver;  // buffers of the device move loop (gcmc_dev.hip)
 constexpr int kMaxMolAtoms = 16;   // atoms per molecule in a trial launch
 constexpr int kBlock = 256;        // threads per workgroup, plain kernels
 
-// Structure factors and reciprocal forces walk the k list in segments:
-// pieces of at most kSeg consecutive-nz vectors of one (nx, ny) run, built
-// on the device by one workgroup of kSegThreads (box.hip).
-constexpr int kSeg = 16;
-constexpr int kSegThreads = 1024;
-// First structure-factor pass: a fixed grid of kSumsGrid workgroups loops
-// over (segment block, atom chunk) items; chunks x K stays within
-// kSumsPartCap so the per-chunk sums fit a bounded buffer.
-constexpr int kSumsGrid = 1024;
+// Structure factors: per-chunk sums of every k-vector, chunks x K within
+// this many (so a bounded buffer holds them).
 constexpr size_t kSumsPartCap = size_t(1) << 21;
 
-// Atom chunks of the first structure-factor pass: about kSumsGrid items
-// over the segment blocks, chunks of at least 32 atoms, within the cap.
-__host__ __device__ inline int SumsChunks(int nseg, int natoms, int K) {
-  const int segBlocks = nseg > kBlock ? (nseg + kBlock - 1) / kBlock : 1;
-  int c = (kSumsGrid + segBlocks - 1) / segBlocks;
-  const int byAtoms = natoms > 32 ? (natoms + 31) / 32 : 1;
-  if (c > byAtoms) c = byAtoms;
-  const int byCap = K > 0 ? int(kSumsPartCap / size_t(K)) : 1;
-  if (c > byCap) c = byCap;
-  return c > 1 ? c : 1;
-}
+// The k-vectors as columns (every nz at one (nx, ny)), longest first, and the
+// work units of the structure-factor and force products (recip.hip): device
+// array `buf` holds the columns {index of nz = 0, nx, ny, m}, the units and
+// the force groups' first steps.
+struct KPlan {
+  int *buf = nullptr;
+  size_t cap = 0, unitOff = 0, fstartOff = 0;
+  int nx = 0, ny = 0, nz = 0;   // largest |n| of a k-vector per axis
+  int nB = 0;                   // unit blocks of eight
+  int ngrp = 0, steps = 0;      // force groups of four columns, their steps in all
+  double *coef = nullptr;       // force coefficients of the last sums
+  size_t coefCap = 0;
+};
+
+// Per-atom k-space forces in parts [chunks][xyz][natoms], to be added.
+struct RecipParts {
+  const double *part = nullptr;
+  int chunks = 0;
+};
 
 // CellList::PositionToCell (src/CellList.h:88-101), on the host and the
 // device alike: both sides of the trial cell table must put a position in
@@ -132,8 +133,6 @@ struct MPState {
   int nchunks = 0, maxChunks = 0;
   double *wpart = nullptr;                              // per-block products
   unsigned *wcounter = nullptr;
-  double *fpart = nullptr;  // per-k-chunk reciprocal forces [chunk][xyz][natoms]
-  size_t fpartCap = 0;
   double *spart = nullptr;  // per-slice pair forces [slice][xyz][natoms]
   size_t spartCap = 0;
 };
@@ -236,10 +235,10 @@ struct gomc_box {
   // per-chunk structure factors of RecipSums [chunks][K][2]
   double *sumPart = nullptr;
   size_t sumPartCap = 0;
-  // k segments (box.hip): starts [nseg + 1] and the count, on the device;
-  // nseg also on the host for launch shapes
-  int *kseg = nullptr, *nsegDev = nullptr;
-  int ksegCap = 0, nseg = 0;
+  // per-chunk reciprocal forces [chunk][xyz][natoms]
+  double *forcePart = nullptr;
+  size_t forcePartCap = 0;
+  gomc::KPlan kp;
 
   // ---- GCMC (ensemble 1): box 0 interacts, box 1 is the reservoir ----
   // Reservoir atoms carry molecule id -1 on the device and are skipped by
@@ -281,8 +280,12 @@ int LaunchTrial(gomc_box *b, int mol, const double *ox, const double *oy, const 
                 bool doRecip, double out[4]);
 void HostCorrectionSelfLRC(gomc_box *b, double &self, double &corr, double &lrc);
 int RecipSums(gomc_box *b, double *erecip);
-// Cuts the box's k list into segments (after the k-vectors change).
-int BuildKSegments(gomc_box *b);
+// The k list's columns and work units (after the k-vectors change).
+int BuildKPlan(gomc_box *b, const std::vector<double> &kx, const std::vector<double> &ky,
+               const std::vector<double> &kz);
+void FreeKPlan(KPlan &p);
+int RecipSumsNoAlloc(gomc_box *b, double *erecip);
+int RecipForceParts(gomc_box *b, const double *sumR, const double *sumI, RecipParts *out);
 int BoxInter(gomc_box *b, double *lj, double *real);
 int EnsurePartials(gomc_box *b, int nblocks);
 int Sync(gomc_box *b);

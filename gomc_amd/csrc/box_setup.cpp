@@ -84,7 +84,7 @@ int RecipInitImpl(gomc_box *b, double *erecip) {
   HIP_TRY(b, hipMemcpyAsync(b->ky, ky.data(), n, hipMemcpyHostToDevice, b->stream));
   HIP_TRY(b, hipMemcpyAsync(b->kz, kz.data(), n, hipMemcpyHostToDevice, b->stream));
   HIP_TRY(b, hipMemcpyAsync(b->pref, pref.data(), n, hipMemcpyHostToDevice, b->stream));
-  int rc = BuildKSegments(b);
+  int rc = BuildKPlan(b, kx, ky, kz);
   if (rc) return rc;
   b->recipReady = true;
   rc = RecipSums(b, erecip);

@@ -271,125 +271,27 @@ __global__ void __launch_bounds__(kChunk) PairForceSumKernel(const PairForceArgs
 }
 
 // ------------------------------------------------------ reciprocal force --
-// Ewald::BoxForceReciprocal (Ewald.cpp:1496-1596), one atom per thread:
-// the k-space force F_j = sum_k 2 q_j prefact_k (sin ReS - cos ImS) k over
-// the current structure factors, walked segment by segment (pieces of at
-// most kSeg consecutive-nz k-vectors, built with the box's k-vectors): one
-// sincos per run of consecutive nz (a segment continuing a run starts at
-// the phase the previous segment rotated to; the nz step's phase is the
-// atom's own), then one complex product and six FMAs per vector against
-// pref S_R k and pref S_I k, staged per tile of segments in LDS; the 2 q
-// factor is applied once at the end.  Then the intramolecular erf correction is subtracted and
-// the chunks added in order.
-constexpr int kForceSegTile = 32;  // segments per LDS tile (at most 512 k)
-
+// Ewald::BoxForceReciprocal (Ewald.cpp:1496-1596): the k-space force of
+// every atom comes in parts from the matrix product of recip.hip; here, one
+// atom per thread, the intramolecular erf correction is subtracted and the
+// parts are added in order.
 struct RecipForceArgs {
   BoxGeom g;
   const double *x, *y, *z, *q;
   const int *mol, *molStart;
-  int natoms, K;
-  const double *kx, *ky, *kz, *pref, *sumR, *sumI;
-  const int *kseg;  // segment starts [nseg + 1]
-  int nseg;
-  double cz;  // the nz step of every segment, 2 pi / L_z
+  int natoms;
   double *fx, *fy, *fz;
-  // segment chunks: RecipForcePartKernel writes chunk c's k-space force of
-  // every atom (segments [c segChunk, (c + 1) segChunk)) to
-  // part[c][xyz][natoms]; RecipForceKernel adds the chunks in order after
-  // the intramolecular term.
-  int segChunk, kChunks;
-  double *part;
+  RecipParts k;
 };
 
-__global__ void __launch_bounds__(kBlock) RecipForcePartKernel(const RecipForceArgs a) {
-  // per k of the tile: pref S_R k_d and pref S_I k_d (d = x, y, z); per
-  // segment: its first k-vector
-  __shared__ double2 sk[3][kForceSegTile * kSeg];  // (pref S_R k_d, pref S_I k_d), one 16-byte read
-  __shared__ double sf[3][kForceSegTile];
-  __shared__ int ss[kForceSegTile + 1];
-  const int chunk = blockIdx.x % a.kChunks;
-  const int p = blockIdx.x / a.kChunks * kBlock + threadIdx.x;
-  const bool active = p < a.natoms;
-  double xp = 0.0, yp = 0.0, zp = 0.0, qp = 0.0;
-  if (active) {
-    xp = a.x[p];
-    yp = a.y[p];
-    zp = a.z[p];
-    qp = a.q[p];
-  }
-  const bool on = active && !(fabs(qp) < 0.000000001);
-  double X = 0.0, Y = 0.0, Z = 0.0;
-  // the atom's phase step e^{i c_z z}, the same for every segment
-  double sn = 0.0, cn = 1.0;
-  if (on) sincos(a.cz * zp, &sn, &cn);
-  const int s0 = min(a.nseg, chunk * a.segChunk), s1 = min(a.nseg, s0 + a.segChunk);
-  // a segment that continues the previous one's run (same nx, ny after a
-  // full segment) starts at the phase the previous one rotated to
-  double im = 0.0, re = 1.0, pkx = 0.0, pky = 0.0;
-  int plen = 0;
-  for (int t = s0; t < s1; t += kForceSegTile) {
-    const int tn = min(kForceSegTile, s1 - t);
-    const int kA = a.kseg[t], kn = a.kseg[t + tn] - kA;
-    __syncthreads();
-    for (int i = threadIdx.x; i <= tn; i += kBlock) {
-      const int k = a.kseg[t + i];
-      ss[i] = k - kA;
-      if (i < tn) {
-        sf[0][i] = a.kx[k];
-        sf[1][i] = a.ky[k];
-        sf[2][i] = a.kz[k];
-      }
-    }
-    for (int i = threadIdx.x; i < kn; i += kBlock) {
-      const int k = kA + i;
-      const double pr = a.pref[k] * a.sumR[k], pi = a.pref[k] * a.sumI[k];
-      sk[0][i] = make_double2(pr * a.kx[k], pi * a.kx[k]);
-      sk[1][i] = make_double2(pr * a.ky[k], pi * a.ky[k]);
-      sk[2][i] = make_double2(pr * a.kz[k], pi * a.kz[k]);
-    }
-    __syncthreads();
-    if (on)
-      for (int j = 0; j < tn; ++j) {
-        const int k0 = ss[j], len = ss[j + 1] - k0;
-        const double kx0 = sf[0][j], ky0 = sf[1][j];
-        if (!(plen == kSeg && kx0 == pkx && ky0 == pky))
-          sincos(xp * kx0 + yp * ky0 + zp * sf[2][j], &im, &re);
-        pkx = kx0;
-        pky = ky0;
-        plen = len;
-#pragma unroll
-        for (int i = 0; i < kSeg; ++i) {
-          if (i < len) {
-            const int k = k0 + i;
-            const double2 vx = sk[0][k], vy = sk[1][k], vz = sk[2][k];
-            X = fma(im, vx.x, X);
-            X = fma(-re, vx.y, X);
-            Y = fma(im, vy.x, Y);
-            Y = fma(-re, vy.y, Y);
-            Z = fma(im, vz.x, Z);
-            Z = fma(-re, vz.y, Z);
-          }
-          const double nr = fma(re, cn, -(im * sn));
-          im = fma(re, sn, im * cn);
-          re = nr;
-        }
-      }
-  }
-  if (active) {
-    const double q2 = 2.0 * qp;
-    a.part[(size_t(chunk) * 3 + 0) * a.natoms + p] = q2 * X;
-    a.part[(size_t(chunk) * 3 + 1) * a.natoms + p] = q2 * Y;
-    a.part[(size_t(chunk) * 3 + 2) * a.natoms + p] = q2 * Z;
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) RecipForceKernel(const RecipForceArgs a) {
-  const int p = blockIdx.x * kBlock + threadIdx.x;
+__global__ void __launch_bounds__(kWave) RecipForceKernel(const RecipForceArgs a) {
+  const int p = blockIdx.x * kWave + threadIdx.x;
   if (p >= a.natoms) return;
   double X = 0.0, Y = 0.0, Z = 0.0;
   const double xp = a.x[p], yp = a.y[p], zp = a.z[p], qp = a.q[p];
   if (!(fabs(qp) < 0.000000001)) {
-    const int m = a.mol[p], s = a.molStart[m], e = a.molStart[m + 1];
+    const int m = a.mol[p];  // < 0: a reservoir atom, no intramolecular term
+    const int s = m < 0 ? p : a.molStart[m], e = m < 0 ? p : a.molStart[m + 1];
     const double constValue = a.g.alpha * M_2_SQRTPI;
     const double alphaSq = a.g.alpha * a.g.alpha;
     for (int j = s; j < e; ++j) {
@@ -408,10 +310,12 @@ __global__ void __launch_bounds__(kBlock) RecipForceKernel(const RecipForceArgs 
       Z -= intraForce * dz;
     }
   }
-  for (int c = 0; c < a.kChunks; ++c) {
-    X += a.part[(size_t(c) * 3 + 0) * a.natoms + p];
-    Y += a.part[(size_t(c) * 3 + 1) * a.natoms + p];
-    Z += a.part[(size_t(c) * 3 + 2) * a.natoms + p];
+#pragma unroll 4
+  for (int c = 0; c < a.k.chunks; ++c) {
+    const double *part = a.k.part + size_t(c) * 3 * a.natoms + p;
+    X += part[0];
+    Y += part[a.natoms];
+    Z += part[2 * size_t(a.natoms)];
   }
   a.fx[p] = X;
   a.fy[p] = Y;
@@ -639,7 +543,7 @@ namespace gomc {
 void MPFree(gomc_box *b) {
   MPState &mp = b->mp;
   std::vector<void *> ptrs = {mp.xn, mp.yn, mp.zn, mp.inRange, mp.fail, mp.chunks, mp.wpart,
-                              mp.wcounter, mp.fpart, mp.spart};
+                              mp.wcounter, mp.spart};
   for (int s = 0; s < 2; ++s)
     for (int d = 0; d < 3; ++d) {
       ptrs.push_back(mp.com[s][d]);
@@ -799,6 +703,8 @@ int MPRecipForce(gomc_box *b, int set) {
     return Sync(b);
   }
   RecipForceArgs a;
+  int rc = RecipForceParts(b, b->sumRnew, b->sumInew, &a.k);
+  if (rc) return rc;
   a.g = b->geom;
   a.x = b->x;
   a.y = b->y;
@@ -807,37 +713,11 @@ int MPRecipForce(gomc_box *b, int set) {
   a.mol = b->mol;
   a.molStart = mp.molStart;
   a.natoms = b->natoms;
-  a.K = b->K;
-  a.kx = b->kx;
-  a.ky = b->ky;
-  a.kz = b->kz;
-  a.pref = b->pref;
-  a.sumR = b->sumRnew;
-  a.sumI = b->sumInew;
   a.fx = mp.aFR[set][0];
   a.fy = mp.aFR[set][1];
   a.fz = mp.aFR[set][2];
-  a.kseg = b->kseg;
-  a.cz = (1.0 / b->geom.L[2]) * (2.0 * M_PI);  // KVectorsOrth's z spacing
-  a.nseg = b->nseg;
-  const int g = (b->natoms + kBlock - 1) / kBlock;
-  // segment chunks, about 1024 workgroups in the first pass
-  int chunks = std::min(std::max(1, b->nseg), std::max(1, (1024 + g - 1) / g));
-  a.segChunk = std::max(1, (b->nseg + chunks - 1) / chunks);
-  chunks = std::max(1, (b->nseg + a.segChunk - 1) / a.segChunk);
-  a.kChunks = chunks;
-  const size_t need = size_t(chunks) * 3 * size_t(std::max(b->natoms, 1));
-  if (need > mp.fpartCap) {
-    if (mp.fpart) (void)hipFree(mp.fpart);
-    mp.fpart = nullptr;
-    mp.fpartCap = 0;
-    HIP_TRY(b, hipMalloc(&mp.fpart, sizeof(double) * need));
-    mp.fpartCap = need;
-  }
-  a.part = mp.fpart;
-  hipLaunchKernelGGL(RecipForcePartKernel, dim3(g * chunks), dim3(kBlock), 0, b->stream, a);
-  HIP_TRY(b, hipGetLastError());
-  hipLaunchKernelGGL(RecipForceKernel, dim3(g), dim3(kBlock), 0, b->stream, a);
+  hipLaunchKernelGGL(RecipForceKernel, dim3((b->natoms + kWave - 1) / kWave), dim3(kWave), 0,
+                     b->stream, a);
   HIP_TRY(b, hipGetLastError());
   return Sync(b);
 }

@@ -10,11 +10,8 @@
 // wave takes (64 cell atoms, 64 neighbour atoms) items and queues their
 // in-cutoff pairs in its LDS, so the pair terms run once per 64 queued
 // pairs, not once per 64 tested.
-// RecipVirialKernel: blocks [0, kBlocks) one k-vector per thread (the
-// k-space term); the others one atom per thread over one chunk of LDS-staged
-// k data (the intramolecular term: q 2 pref (S_I cos - S_R sin) k_d times
-// the atom's offset from its molecule's centre).  Each block writes its partial sums;
-// the host adds them in block order.
+// RecipVirialKernel: the reciprocal part.  Each block writes its partial
+// sums; the host adds them in block order.
 #include <algorithm>
 #include <cmath>
 
@@ -169,19 +166,16 @@ __global__ void __launch_bounds__(kBlock, 4) PairVirialKernel(const PairVirArgs 
   }
 }
 
-// Segments of the k list (consecutive nz, at most kSeg vectors) staged in
-// LDS this many at a time by the intramolecular term.
-constexpr int kVirSegTile = 32;
-
+// The reciprocal part: blocks [0, kBlocks) one k-vector per thread (the
+// k-space term); the others one atom per thread (the intramolecular term:
+// minus the atom's k-space force, in parts from recip.hip's matrix product,
+// times its offset from its molecule's centre).
 struct RecipVirArgs {
   BoxGeom g;
   const double *x, *y, *z, *q;
   const int *mol;
   int natoms, K, kBlocks;
-  int segChunk, kChunks;  // segments per chunk, chunks per atom block
-  const int *kseg;        // segment starts [nseg + 1]
-  int nseg;
-  double kzStep;          // the nz step of every segment, 2 pi / L_z
+  RecipParts f;
   const double *kx, *ky, *kz, *pref, *sumR, *sumI;
   const double *cx, *cy, *cz;
   double constVal;  // 1 / (4 alpha^2)
@@ -190,9 +184,6 @@ struct RecipVirArgs {
 
 __global__ void __launch_bounds__(kBlock) RecipVirialKernel(const RecipVirArgs a) {
   __shared__ double red[kBlock / kWave];
-  __shared__ double2 sk[3][kVirSegTile * kSeg];  // (pref S_R k_d, pref S_I k_d) per k
-  __shared__ double sf[3][kVirSegTile];           // each segment's first k-vector
-  __shared__ int ss[kVirSegTile + 1];
   double w[3] = {0, 0, 0};
   if (int(blockIdx.x) < a.kBlocks) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -205,88 +196,22 @@ __global__ void __launch_bounds__(kBlock) RecipVirialKernel(const RecipVirArgs a
       w[2] = factor * (1.0 - 2.0 * (a.constVal + 1.0 / hsqr) * kz * kz);
     }
   } else {
-    const int p = (blockIdx.x - a.kBlocks) / a.kChunks * kBlock + threadIdx.x;
-    bool on = false;
-    double xp = 0, yp = 0, zp = 0, qp = 0, ddx = 0, ddy = 0, ddz = 0;
-    if (p < a.natoms) {
-      qp = a.q[p];
-      const int m = a.mol[p];
-      on = m >= 0 && !(fabs(qp) < 0.000000001);
-      if (on) {
-        xp = a.x[p];
-        yp = a.y[p];
-        zp = a.z[p];
-        const double cx = a.cx[m], cy = a.cy[m], cz = a.cz[m];
-        ddx = Unwrap(xp, cx, a.g.L[0], a.g.half[0]) - cx;
-        ddy = Unwrap(yp, cy, a.g.L[1], a.g.half[1]) - cy;
-        ddz = Unwrap(zp, cz, a.g.L[2], a.g.half[2]) - cz;
+    const int p = (blockIdx.x - a.kBlocks) * kBlock + threadIdx.x;
+    const int m = p < a.natoms ? a.mol[p] : -1;
+    if (m >= 0 && !(fabs(a.q[p]) < 0.000000001)) {
+      const double r[3] = {a.x[p], a.y[p], a.z[p]}, c[3] = {a.cx[m], a.cy[m], a.cz[m]};
+      double f[3] = {0, 0, 0};
+#pragma unroll 4
+      for (int ch = 0; ch < a.f.chunks; ++ch) {
+        const double *part = a.f.part + size_t(ch) * 3 * a.natoms + p;
+        f[0] += part[0];
+        f[1] += part[a.natoms];
+        f[2] += part[2 * size_t(a.natoms)];
       }
-    }
-    // this chunk's segments, kVirSegTile at a time: one sincos per run of
-    // consecutive nz, for its first phase (the nz step's phase is the
-    // atom's own), then one complex product and six FMAs per k-vector
-    // against pref S_R k and pref S_I k; 2 q times the offset at the end
-    const int chunk = (blockIdx.x - a.kBlocks) % a.kChunks;
-    const int s0 = min(a.nseg, chunk * a.segChunk), s1 = min(a.nseg, s0 + a.segChunk);
-    double sn = 0.0, cn = 1.0;  // the atom's phase step e^{i c_z z}, every segment's
-    if (on) sincos(a.kzStep * zp, &sn, &cn);
-    double W[3] = {0.0, 0.0, 0.0};
-    // a segment that continues the previous one's run (same nx, ny after a
-    // full segment) starts at the phase the previous one rotated to
-    double s = 0.0, c = 1.0, pkx = 0.0, pky = 0.0;
-    int plen = 0;
-    for (int t = s0; t < s1; t += kVirSegTile) {
-      const int tn = min(kVirSegTile, s1 - t);
-      const int kA = a.kseg[t], kn = a.kseg[t + tn] - kA;
-      __syncthreads();
-      for (int i = threadIdx.x; i <= tn; i += kBlock) {
-        const int k = a.kseg[t + i];
-        ss[i] = k - kA;
-        if (i < tn) {
-          sf[0][i] = a.kx[k];
-          sf[1][i] = a.ky[k];
-          sf[2][i] = a.kz[k];
-        }
-      }
-      for (int i = threadIdx.x; i < kn; i += kBlock) {
-        const int k = kA + i;
-        const double pr = a.pref[k] * a.sumR[k], pi = a.pref[k] * a.sumI[k];
-        sk[0][i] = make_double2(pr * a.kx[k], pi * a.kx[k]);
-        sk[1][i] = make_double2(pr * a.ky[k], pi * a.ky[k]);
-        sk[2][i] = make_double2(pr * a.kz[k], pi * a.kz[k]);
-      }
-      __syncthreads();
-      if (on)
-        for (int j = 0; j < tn; ++j) {
-          const int k0 = ss[j], len = ss[j + 1] - k0;
-          const double kx0 = sf[0][j], ky0 = sf[1][j];
-          if (!(plen == kSeg && kx0 == pkx && ky0 == pky))
-            sincos(xp * kx0 + yp * ky0 + zp * sf[2][j], &s, &c);
-          pkx = kx0;
-          pky = ky0;
-          plen = len;
 #pragma unroll
-          for (int i = 0; i < kSeg; ++i) {
-            if (i < len) {
-              const int k = k0 + i;
-              const double2 vx = sk[0][k], vy = sk[1][k], vz = sk[2][k];
-              W[0] = fma(c, vx.y, W[0]);
-              W[0] = fma(-s, vx.x, W[0]);
-              W[1] = fma(c, vy.y, W[1]);
-              W[1] = fma(-s, vy.x, W[1]);
-              W[2] = fma(c, vz.y, W[2]);
-              W[2] = fma(-s, vz.x, W[2]);
-            }
-            const double nc = fma(c, cn, -(s * sn));
-            s = fma(c, sn, s * cn);
-            c = nc;
-          }
-        }
+      for (int d = 0; d < 3; ++d)
+        w[d] = -f[d] * (Unwrap(r[d], c[d], a.g.L[d], a.g.half[d]) - c[d]);
     }
-    const double q2 = 2.0 * qp;
-    w[0] = q2 * (W[0] * ddx);
-    w[1] = q2 * (W[1] * ddy);
-    w[2] = q2 * (W[2] * ddz);
   }
   for (int c = 0; c < 3; ++c) {
     const double s = BlockSum(w[c], red);
@@ -307,17 +232,7 @@ extern "C" int gomc_box_virial(gomc_box *b, double out[9]) {
   const int pairBlocks = b->ncell * 27;
   const int kBlocks = b->ewald ? (b->K + kBlock - 1) / kBlock : 0;
   const int atomBlocks = b->ewald ? (b->natoms + kBlock - 1) / kBlock : 0;
-  // The intramolecular term splits the k list's segments into chunks as
-  // well as the atoms into blocks, so that a large box fills the chip (about
-  // 2048 workgroups).
-  int kChunks = 1, segChunk = std::max(b->nseg, 1);
-  if (atomBlocks > 0) {
-    if (b->nseg <= 0) return Fail(b, GOMC_ERR_STATE, "k-vector segments not built");
-    kChunks = std::min(b->nseg, std::max(1, (2048 + atomBlocks - 1) / atomBlocks));
-    segChunk = (b->nseg + kChunks - 1) / kChunks;
-    kChunks = (b->nseg + segChunk - 1) / segChunk;
-  }
-  const int nblocks = pairBlocks + kBlocks + atomBlocks * kChunks;
+  const int nblocks = pairBlocks + kBlocks + atomBlocks;
   const size_t need = size_t(kVirSlots) * std::max(nblocks, 1);
   if (need > b->virCap) {  // grows only with the box's block count
     if (b->virBuf) (void)hipFree(b->virBuf);
@@ -351,6 +266,8 @@ extern "C" int gomc_box_virial(gomc_box *b, double out[9]) {
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && b->ewald) {
     RecipVirArgs r;
+    rc = RecipForceParts(b, b->sumRref, b->sumIref, &r.f);
+    if (rc) return rc;
     r.g = b->geom;
     r.x = b->x;
     r.y = b->y;
@@ -360,11 +277,6 @@ extern "C" int gomc_box_virial(gomc_box *b, double out[9]) {
     r.natoms = b->natoms;
     r.K = b->K;
     r.kBlocks = kBlocks;
-    r.segChunk = segChunk;
-    r.kChunks = kChunks;
-    r.kseg = b->kseg;
-    r.nseg = b->nseg;
-    r.kzStep = (1.0 / b->geom.L[2]) * (2.0 * M_PI);  // KVectorsOrth's z spacing
     r.kx = b->kx;
     r.ky = b->ky;
     r.kz = b->kz;
@@ -376,7 +288,7 @@ extern "C" int gomc_box_virial(gomc_box *b, double out[9]) {
     r.cz = a.cz;
     r.constVal = 1.0 / (4.0 * (b->alpha * b->alpha));
     r.part = part + size_t(pairBlocks) * kVirSlots;
-    hipLaunchKernelGGL(RecipVirialKernel, dim3(kBlocks + atomBlocks * kChunks), dim3(kBlock), 0,
+    hipLaunchKernelGGL(RecipVirialKernel, dim3(kBlocks + atomBlocks), dim3(kBlock), 0,
                        b->stream, r);
     e = hipGetLastError();
   }
