@@ -342,68 +342,6 @@ __global__ void __launch_bounds__(kBlock) CellSortKernel(const CellArgs a) {
   }
 }
 
-// ------------------------------------------------------------- box inter --
-// One workgroup per (cell, neighbour slot); pairs i < j of different
-// molecules (CalculateEnergy.cpp:205-250).  The neighbour cell's atoms are
-// staged in LDS; threads stride over the (i, j) product.
-struct BoxInterArgs {
-  BoxGeom g;
-  const double *x, *y, *z, *q;
-  const int *type, *mol;
-  const double *sigSq, *epsCn, *nHalf;
-  int ntypes;
-  const int *cellStart, *cellVec, *nbr;
-  Partial4 *partials;
-  unsigned *counter;
-  double *result;
-};
-
-__global__ void __launch_bounds__(kBlock) BoxInterKernel(const BoxInterArgs a) {
-  __shared__ double sx[kBlock], sy[kBlock], sz[kBlock], sq[kBlock];
-  __shared__ int sidx[kBlock], stype[kBlock], smol[kBlock];
-  __shared__ double red[kBlock / kWave];
-  const int cell = blockIdx.x / 27, nb = a.nbr[blockIdx.x];
-  const int cs = a.cellStart[cell], ce = a.cellStart[cell + 1];
-  const int ns = a.cellStart[nb], ne = a.cellStart[nb + 1];
-  const int ni = ce - cs;
-  double lj = 0.0, real = 0.0;
-  for (int tile = ns; tile < ne; tile += kBlock) {
-    const int tn = min(kBlock, ne - tile);
-    if (threadIdx.x < tn) {
-      int j = a.cellVec[tile + threadIdx.x];
-      sidx[threadIdx.x] = j;
-      sx[threadIdx.x] = a.x[j];
-      sy[threadIdx.x] = a.y[j];
-      sz[threadIdx.x] = a.z[j];
-      sq[threadIdx.x] = a.q[j];
-      stype[threadIdx.x] = a.type[j];
-      smol[threadIdx.x] = a.mol[j];
-    }
-    __syncthreads();
-    for (int p = threadIdx.x; p < ni * tn; p += kBlock) {
-      const int i = a.cellVec[cs + p / tn], jj = p % tn, j = sidx[jj];
-      if (i < j && a.mol[i] != smol[jj]) {
-        double d2 = DistSq(a.g, a.x[i], a.y[i], a.z[i], sx[jj], sy[jj], sz[jj]);
-        if (a.g.rCutSq > d2) {
-          if (a.g.elect) {
-            double qiqj = a.q[i] * sq[jj] * kQQFact;
-            if (qiqj != 0.0 && !(a.g.rCutCoulSq < d2)) real += CoulombEnergy(a.g, d2, qiqj);
-          }
-          if (!(a.g.rCutLJSq < d2)) {
-            int idx = a.type[i] + stype[jj] * a.ntypes;
-            lj += LJEnergy(d2, a.sigSq[idx], a.epsCn[idx], a.nHalf[idx]);
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-  Partial4 part{0, 0, 0, 0};
-  part.lj = BlockSum(lj, red);
-  part.real = BlockSum(real, red);
-  FinishPartials(part, a.partials, a.counter, a.result);
-}
-
 // Insertion (+) or removal (-) of one molecule: SwapDestRecip /
 // SwapSourceRecip (Ewald.cpp:478-531, 657-710).
 struct SwapArgs {
@@ -872,45 +810,11 @@ int BuildCells(gomc_box *b) {
                             hipMemcpyDeviceToHost, b->stream));
   int rc = Sync(b);
   if (rc) return rc;
-  b->hCellCount = counts;
   int mx = *std::max_element(counts.begin(), counts.end());
   if (mx * sizeof(int) > 60 * 1024) return Fail(b, GOMC_ERR_ARG, "cell too full for device sort");
   hipLaunchKernelGGL(CellSortKernel, dim3(b->ncell), dim3(kBlock), std::max(mx, 1) * sizeof(int),
                      b->stream, a);
   HIP_TRY(b, hipGetLastError());
-  return GOMC_OK;
-}
-
-int BoxInter(gomc_box *b, double *lj, double *real) {
-  int rc = BuildCells(b);
-  if (rc) return rc;
-  BoxInterArgs a;
-  a.g = b->geom;
-  a.x = b->x;
-  a.y = b->y;
-  a.z = b->z;
-  a.q = b->q;
-  a.type = b->type;
-  a.mol = b->mol;
-  a.sigSq = b->tSigSq;
-  a.epsCn = b->tEpsCn;
-  a.nHalf = b->tNHalf;
-  a.ntypes = b->ntypes;
-  a.cellStart = b->cellStart;
-  a.cellVec = b->cellVec;
-  a.nbr = b->nbr;
-  const int nblocks = b->ncell * 27;
-  rc = EnsurePartials(b, nblocks);
-  if (rc) return rc;
-  a.partials = b->partials;
-  a.counter = b->counter;
-  a.result = b->devRes;
-  hipLaunchKernelGGL(BoxInterKernel, dim3(nblocks), dim3(kBlock), 0, b->stream, a);
-  HIP_TRY(b, hipGetLastError());
-  rc = Sync(b);
-  if (rc) return rc;
-  *lj = b->hostRes[0];
-  *real = b->hostRes[1];
   return GOMC_OK;
 }
 
@@ -973,6 +877,7 @@ static void FreeAll(gomc_box *b) {
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   FreeKPlan(b->kp);
+  FreeMolCells(b->mc);
   MPFree(b);
   DevFree(b);
   if (b->trialBuf) (void)hipFree(b->trialBuf);

@@ -41,6 +41,18 @@ struct KPlan {
   size_t coefCap = 0;
 };
 
+// Molecules in cells for the whole-box pair sums (pair.hip), rebuilt from the
+// coordinates for each sum; `count` is zero between builds.
+struct MolCells {
+  int *count = nullptr, *start = nullptr;  // [cap], [cap + 1]
+  int cap = 0;
+  int *cell = nullptr, *slot = nullptr, *tmp = nullptr, *sid = nullptr;  // [nmols]
+  void *where = nullptr, *pack = nullptr;  // [nmols] centre and radius
+  unsigned long long *radBits = nullptr;
+  double *vpart = nullptr;  // per-block virials
+  size_t vcap = 0;
+};
+
 // Per-atom k-space forces in parts [chunks][xyz][natoms], to be added.
 struct RecipParts {
   const double *part = nullptr;
@@ -129,12 +141,8 @@ struct MPState {
   double *mF[2][3] = {}, *mFR[2][3] = {}, *tq[2][3] = {};  // molecule terms
   double *tk[3] = {};                                   // t_k or r_k
   int *inRange = nullptr, *fail = nullptr, *molStart = nullptr;
-  int *chunks = nullptr;                                // force work list
-  int nchunks = 0, maxChunks = 0;
   double *wpart = nullptr;                              // per-block products
   unsigned *wcounter = nullptr;
-  double *spart = nullptr;  // per-slice pair forces [slice][xyz][natoms]
-  size_t spartCap = 0;
 };
 
 // MoveSettings state of the driver (src/MoveSettings.cpp:19-258).
@@ -201,12 +209,13 @@ struct gomc_box {
   gomc::Partial4 *partials = nullptr;
   int maxPartials = 0;
   unsigned *counter = nullptr;
-  double *hostRes = nullptr, *devRes = nullptr;  // 8 doubles, host-mapped
+  double *hostRes = nullptr, *devRes = nullptr;  // 16 doubles, host-mapped
   // a molecule whose accepted coordinates the next trial launch writes
   int pendingMol = -1;
   double pend[3][gomc::kMaxMolAtoms];
 
-  std::vector<int> hCellCount;  // atoms per cell at the last build
+  gomc::MolCells mc;
+  double molRadius = 0.0;  // largest molecule radius of the first coordinates
   // Trial cell table (plain trial path, boxes of more than 27 cells): per
   // cell up to tcCap atom slots of the live atoms, in no particular order.
   // The host copy (hTc*) is authoritative; the device copy trails it by the
@@ -287,6 +296,9 @@ void FreeKPlan(KPlan &p);
 int RecipSumsNoAlloc(gomc_box *b, double *erecip);
 int RecipForceParts(gomc_box *b, const double *sumR, const double *sumI, RecipParts *out);
 int BoxInter(gomc_box *b, double *lj, double *real);
+int PairForces(gomc_box *b, double *const f[3]);
+int PairVirials(gomc_box *b, double *const com[3], const double **vpart, int *nblocks);
+void FreeMolCells(MolCells &c);
 int EnsurePartials(gomc_box *b, int nblocks);
 int Sync(gomc_box *b);
 int BuildCells(gomc_box *b);

@@ -122,6 +122,12 @@ static void CalcCOM(gomc_box *b) {
     b->comx[m] = Wrap(cx * inv, L[0]);
     b->comy[m] = Wrap(cy * inv, L[1]);
     b->comz[m] = Wrap(cz * inv, L[2]);
+    for (int p = s; p < e; ++p) {
+      const double dx = Unwrap(b->hx[p], rx, L[0], H[0]) - cx * inv,
+                   dy = Unwrap(b->hy[p], ry, L[1], H[1]) - cy * inv,
+                   dz = Unwrap(b->hz[p], rz, L[2], H[2]) - cz * inv;
+      b->molRadius = std::max(b->molRadius, std::sqrt(dx * dx + dy * dy + dz * dz));
+    }
   }
 }
 
@@ -315,7 +321,7 @@ int gomc_box_create(const gomc_system_desc *d, int device, gomc_box **out) {
   ok &= hipMalloc(&b->atomCell, ni) == hipSuccess;
   ok &= hipMalloc(&b->nbr, sizeof(int) * b->ncell * 27) == hipSuccess;
   ok &= hipMalloc(&b->counter, sizeof(unsigned)) == hipSuccess;
-  ok &= hipHostMalloc(&b->hostRes, sizeof(double) * 8, hipHostMallocMapped) == hipSuccess;
+  ok &= hipHostMalloc(&b->hostRes, sizeof(double) * 16, hipHostMallocMapped) == hipSuccess;
   if (!ok) return fail(GOMC_ERR_HIP, "device allocation failed");
   if (hipHostGetDevicePointer((void **)&b->devRes, b->hostRes, 0) != hipSuccess)
     return fail(GOMC_ERR_HIP, "mapped result pointer");

@@ -17,7 +17,6 @@ using namespace gomc;
 
 namespace {
 
-constexpr int kChunk = 64;  // home atoms per force workgroup
 constexpr double kMinForce = 1E-12, kMaxForce = 30;  // MultiParticle.h:18-19
 constexpr double kLambda = 0.5;                      // MultiParticle.h:95
 
@@ -28,246 +27,6 @@ struct Vec3D {
 // r123::uneg11<double> for a 64-bit word (lib/Random123/uniform.hpp:196-214).
 __device__ __forceinline__ double Uneg11(uint64_t v) {
   return double(int64_t(v)) * 0x1p-63 + 0x1p-64;
-}
-
-// ------------------------------------------------------------ pair force --
-// CalculateEnergy::BoxForce (CalculateEnergy.cpp:268-406).  A chunk is a
-// cell's atoms 64 at a time (one per lane); its 27 neighbour cells, taken
-// 64 atoms at a time, make a list of tiles.  `slices` workgroups of G waves
-// share a chunk and its waves take the tiles round robin: wave w of slice s
-// takes tiles s G + w, s G + w + slices G, ...  A wave stages each tile
-// (position, charge, type, molecule of 64 neighbour atoms) in its LDS, one
-// coalesced load per tile instead of a chain of dependent loads per pair,
-// and marks each lane's in-cutoff partners of the tile in a bit mask.  It
-// then lists the tile's pairs in (home atom, tile entry) order and
-// evaluates them 64 at a time, so the pair math runs about (pairs / 64)
-// times per tile rather than as often as the busiest lane has partners;
-// the force contributions of a batch are summed per home atom by a
-// segmented scan and added to that atom's sum in the wave's LDS, an order
-// fixed by the positions alone.  A workgroup adds its waves' per-atom
-// forces in wave order through LDS; with one slice it writes the chunk's
-// forces, with several each slice writes its own and
-// PairForceSumKernel adds them in slice order.  Energies count each pair
-// once (i < j).  The host picks G and the slice count so that a box of any
-// size puts a few thousand waves on the device.
-constexpr int kPairChunksFor4 = 1024;  // from this many chunks: 4 waves per workgroup
-constexpr int kPairChunksFor8 = 256;   // from this many: 8; below: 8 and slices
-constexpr int kPairSmallWaves = 2048;  // waves a small box is split into, about
-constexpr int kPairMaxSlices = 8;
-
-struct PairForceArgs {
-  BoxGeom g;
-  const double *x, *y, *z, *q;
-  const int *type, *mol;
-  const double *sigSq, *epsCn, *nHalf, *epsCn6, *nOver6;
-  int ntypes;
-  const int *cellStart, *cellVec, *nbr;
-  const int *chunks;  // [3 * nchunks]: cell, first atom within the cell, count
-  int slices, natoms;
-  double *fx, *fy, *fz;
-  double *spart;  // slices > 1: [slice][xyz][natoms]
-  Partial4 *partials;
-  unsigned *counter;
-  double *result;
-};
-
-struct PairTile {
-  double x[kChunk], y[kChunk], z[kChunk], q[kChunk];
-  int type[kChunk], mol[kChunk], idx[kChunk];
-};
-
-// In-cutoff pairs of one tile listed per wave, evaluated 64 at a time.
-constexpr int kPairList = 512;  // list entries per wave and window
-
-// Sum of v over the lanes of each run of equal, non-decreasing keys, in a
-// fixed tree order (inclusive scan; the run's last lane holds the total).
-__device__ __forceinline__ double SegScan(double v, int key, int lane) {
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    const double u = __shfl_up(v, d);
-    const int ku = __shfl_up(key, d);
-    if (lane >= d && ku == key) v += u;
-  }
-  return v;
-}
-
-template <int kGroups>
-__global__ void __launch_bounds__(kGroups * kChunk) PairForceKernel(const PairForceArgs a) {
-  static_assert(kChunk == kWave, "one tile entry per lane");
-  __shared__ double sf[kGroups][3][kChunk];
-  __shared__ double red[kGroups * kChunk / kWave];
-  __shared__ PairTile tile[kGroups];
-  __shared__ PairTile home;
-  __shared__ uint16_t plist[kGroups][kPairList];
-  __shared__ double poly[kErfcxDeg + 1];
-  __shared__ int nbS[27], nbE[27], tileS[28];
-  const int chunkId = blockIdx.x / a.slices, slice = blockIdx.x - chunkId * a.slices;
-  const int cell = a.chunks[3 * chunkId], off = a.chunks[3 * chunkId + 1],
-            cnt = a.chunks[3 * chunkId + 2];
-  const int lane = threadIdx.x % kChunk, grp = threadIdx.x / kChunk;
-  const bool valid = lane < cnt;
-  const int i = valid ? a.cellVec[a.cellStart[cell] + off + lane] : 0;
-  if (threadIdx.x <= kErfcxDeg) poly[threadIdx.x] = kErfcxPoly[threadIdx.x];
-  if (threadIdx.x < 27) {
-    const int nb = a.nbr[cell * 27 + threadIdx.x];
-    nbS[threadIdx.x] = a.cellStart[nb];
-    nbE[threadIdx.x] = a.cellStart[nb + 1];
-  }
-  if (grp == 0) {
-    home.x[lane] = a.x[i];
-    home.y[lane] = a.y[i];
-    home.z[lane] = a.z[i];
-    home.q[lane] = a.q[i];
-    home.type[lane] = a.type[i];
-    home.idx[lane] = i;
-  }
-  sf[grp][0][lane] = 0.0;
-  sf[grp][1][lane] = 0.0;
-  sf[grp][2][lane] = 0.0;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int t = 0;
-    for (int c = 0; c < 27; ++c) {
-      tileS[c] = t;
-      t += (nbE[c] - nbS[c] + kChunk - 1) / kChunk;
-    }
-    tileS[27] = t;
-  }
-  __syncthreads();
-  const double xi = home.x[lane], yi = home.y[lane], zi = home.z[lane];
-  const int mi = valid ? a.mol[i] : -1;
-  double lj = 0.0, real = 0.0;
-  PairTile &t = tile[grp];
-  uint16_t *list = plist[grp];
-  const int ntiles = tileS[27], stride = a.slices * kGroups;
-  int c = 0;
-  for (int tt = slice * kGroups + grp; tt < ntiles; tt += stride) {
-    while (tileS[c + 1] <= tt) ++c;
-    const int base = nbS[c] + (tt - tileS[c]) * kChunk;
-    const int n = min(kChunk, nbE[c] - base);
-    if (lane < n) {
-      const int j = a.cellVec[base + lane];
-      t.idx[lane] = j;
-      t.x[lane] = a.x[j];
-      t.y[lane] = a.y[j];
-      t.z[lane] = a.z[j];
-      t.q[lane] = a.q[j];
-      t.type[lane] = a.type[j];
-      t.mol[lane] = a.mol[j];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    uint64_t near = 0;
-    if (valid)
-      for (int k = 0; k < n; ++k) {
-        const double dx = MinImage(xi - t.x[k], a.g.L[0], a.g.half[0]);
-        const double dy = MinImage(yi - t.y[k], a.g.L[1], a.g.half[1]);
-        const double dz = MinImage(zi - t.z[k], a.g.L[2], a.g.half[2]);
-        const double d2 = dx * dx + dy * dy + dz * dz;
-        if (t.mol[k] != mi && a.g.rCutSq > d2) near |= uint64_t(1) << k;
-      }
-    // the wave's pairs in (lane, k) order: lane's pairs start at `pos`
-    const int mine = __popcll(near);
-    int incl = mine;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-      const int u = __shfl_up(incl, d);
-      if (lane >= d) incl += u;
-    }
-    const int total = __shfl(incl, kWave - 1);
-    int pos = incl - mine;
-    for (int b = 0; b < total; b += kPairList) {
-      while (near && pos < b + kPairList) {
-        list[pos - b] = uint16_t((lane << 6) | __builtin_ctzll(near));
-        near &= near - 1;
-        ++pos;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const int nb = min(kPairList, total - b);
-      for (int r = 0; r < nb; r += kWave) {
-        const bool on = r + lane < nb;
-        const int e = on ? list[r + lane] : 0;
-        const int owner = on ? e >> 6 : kWave, k = e & 63;
-        double fx = 0.0, fy = 0.0, fz = 0.0;
-        if (on) {
-          const double dx = MinImage(home.x[owner] - t.x[k], a.g.L[0], a.g.half[0]);
-          const double dy = MinImage(home.y[owner] - t.y[k], a.g.L[1], a.g.half[1]);
-          const double dz = MinImage(home.z[owner] - t.z[k], a.g.L[2], a.g.half[2]);
-          const double d2 = dx * dx + dy * dy + dz * dz;
-          const int idx = home.type[owner] + t.type[k] * a.ntypes;
-          const PairTerms p = PairMath(a.g, poly, d2, home.q[owner] * t.q[k] * kQQFact,
-                                       a.sigSq[idx], a.epsCn[idx], a.nHalf[idx], a.epsCn6[idx],
-                                       a.nOver6[idx], home.idx[owner] < t.idx[k]);
-          real += p.eReal;
-          lj += p.eLJ;
-          fx = dx * p.vLJ + dx * p.vReal;
-          fy = dy * p.vLJ + dy * p.vReal;
-          fz = dz * p.vLJ + dz * p.vReal;
-        }
-        fx = SegScan(fx, owner, lane);
-        fy = SegScan(fy, owner, lane);
-        fz = SegScan(fz, owner, lane);
-        const int nextOwner = __shfl_down(owner, 1);
-        if (on && (lane == kWave - 1 || nextOwner != owner)) {
-          sf[grp][0][owner] += fx;
-          sf[grp][1][owner] += fy;
-          sf[grp][2][owner] += fz;
-        }
-      }
-      // the list is read before the next window overwrites it
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    // every lane is done with the tile before the next one overwrites it
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-  Partial4 part{0, 0, 0, 0};
-  part.lj = BlockSum(lj, red);  // synchronises the LDS writes above
-  part.real = BlockSum(real, red);
-  if (grp == 0 && valid) {
-    double sx = sf[0][0][lane], sy = sf[0][1][lane], sz = sf[0][2][lane];
-    for (int g = 1; g < kGroups; ++g) {
-      sx += sf[g][0][lane];
-      sy += sf[g][1][lane];
-      sz += sf[g][2][lane];
-    }
-    if (a.slices == 1) {
-      a.fx[i] = sx;
-      a.fy[i] = sy;
-      a.fz[i] = sz;
-    } else {
-      double *sp = a.spart + size_t(slice) * 3 * a.natoms;
-      sp[i] = sx;
-      sp[a.natoms + i] = sy;
-      sp[2 * size_t(a.natoms) + i] = sz;
-    }
-  }
-  FinishPartials(part, a.partials, a.counter, a.result);
-}
-
-// The slices' forces of every chunk atom, added in slice order.
-__global__ void __launch_bounds__(kChunk) PairForceSumKernel(const PairForceArgs a) {
-  const int cell = a.chunks[3 * blockIdx.x], off = a.chunks[3 * blockIdx.x + 1],
-            cnt = a.chunks[3 * blockIdx.x + 2];
-  if (int(threadIdx.x) >= cnt) return;
-  const int i = a.cellVec[a.cellStart[cell] + off + threadIdx.x];
-  const size_t n = a.natoms;
-  double sx = a.spart[i], sy = a.spart[n + i], sz = a.spart[2 * n + i];
-  for (int s = 1; s < a.slices; ++s) {
-    const double *sp = a.spart + size_t(s) * 3 * n;
-    sx += sp[i];
-    sy += sp[n + i];
-    sz += sp[2 * n + i];
-  }
-  a.fx[i] = sx;
-  a.fy[i] = sy;
-  a.fz[i] = sz;
 }
 
 // ------------------------------------------------------ reciprocal force --
@@ -542,8 +301,8 @@ namespace gomc {
 
 void MPFree(gomc_box *b) {
   MPState &mp = b->mp;
-  std::vector<void *> ptrs = {mp.xn, mp.yn, mp.zn, mp.inRange, mp.fail, mp.chunks, mp.wpart,
-                              mp.wcounter, mp.spart};
+  std::vector<void *> ptrs = {mp.xn, mp.yn, mp.zn, mp.inRange, mp.fail, mp.wpart,
+                              mp.wcounter};
   for (int s = 0; s < 2; ++s)
     for (int d = 0; d < 3; ++d) {
       ptrs.push_back(mp.com[s][d]);
@@ -605,89 +364,8 @@ int MPUploadCom(gomc_box *b) {
 
 // Pair forces of the current coordinates into force set `set`; energies out.
 int MPPairForce(gomc_box *b, int set, double *lj, double *real) {
-  MPState &mp = b->mp;
-  int rc = BuildCells(b);
-  if (rc) return rc;
-  std::vector<int> ch;
-  for (int c = 0; c < b->ncell; ++c)
-    for (int o = 0; o < b->hCellCount[c]; o += kChunk) {
-      ch.push_back(c);
-      ch.push_back(o);
-      ch.push_back(std::min(kChunk, b->hCellCount[c] - o));
-    }
-  const int n = int(ch.size() / 3);
-  if (n > mp.maxChunks) {
-    if (mp.chunks) (void)hipFree(mp.chunks);
-    mp.chunks = nullptr;
-    mp.maxChunks = 0;
-    HIP_TRY(b, hipMalloc(&mp.chunks, sizeof(int) * 3 * std::max(n, 1)));
-    mp.maxChunks = n;
-  }
-  mp.nchunks = n;
-  if (n == 0) {
-    *lj = *real = 0.0;
-    return GOMC_OK;
-  }
-  HIP_TRY(b, hipMemcpyAsync(mp.chunks, ch.data(), sizeof(int) * ch.size(), hipMemcpyHostToDevice,
-                            b->stream));
-  // waves per workgroup and slices per chunk: a large box fills the device
-  // with chunks alone, a small one splits each chunk's tiles over slices
-  int G = 8, slices = 1;
-  if (n >= kPairChunksFor4) {
-    G = 4;
-  } else if (n < kPairChunksFor8) {
-    slices = std::min(kPairMaxSlices, std::max(1, (kPairSmallWaves + 8 * n - 1) / (8 * n)));
-  }
-  if (slices > 1) {
-    const size_t need = size_t(slices) * 3 * size_t(b->natoms);
-    if (need > mp.spartCap) {
-      if (mp.spart) (void)hipFree(mp.spart);
-      mp.spart = nullptr;
-      mp.spartCap = 0;
-      HIP_TRY(b, hipMalloc(&mp.spart, sizeof(double) * need));
-      mp.spartCap = need;
-    }
-  }
-  rc = EnsurePartials(b, n * slices);
-  if (rc) return rc;
-  PairForceArgs a;
-  a.g = b->geom;
-  a.x = b->x;
-  a.y = b->y;
-  a.z = b->z;
-  a.q = b->q;
-  a.type = b->type;
-  a.mol = b->mol;
-  a.sigSq = b->tSigSq;
-  a.epsCn = b->tEpsCn;
-  a.nHalf = b->tNHalf;
-  a.epsCn6 = b->tEpsCn6;
-  a.nOver6 = b->tNOver6;
-  a.ntypes = b->ntypes;
-  a.cellStart = b->cellStart;
-  a.cellVec = b->cellVec;
-  a.nbr = b->nbr;
-  a.chunks = mp.chunks;
-  a.fx = mp.aF[set][0];
-  a.fy = mp.aF[set][1];
-  a.fz = mp.aF[set][2];
-  a.partials = b->partials;
-  a.counter = b->counter;
-  a.result = b->devRes;
-  a.slices = slices;
-  a.natoms = b->natoms;
-  a.spart = mp.spart;
-  const dim3 grid(n * slices);
-  if (G == 8)
-    hipLaunchKernelGGL(PairForceKernel<8>, grid, dim3(8 * kChunk), 0, b->stream, a);
-  else
-    hipLaunchKernelGGL(PairForceKernel<4>, grid, dim3(4 * kChunk), 0, b->stream, a);
-  HIP_TRY(b, hipGetLastError());
-  if (slices > 1) {
-    hipLaunchKernelGGL(PairForceSumKernel, dim3(n), dim3(kChunk), 0, b->stream, a);
-    HIP_TRY(b, hipGetLastError());
-  }
-  rc = Sync(b);
+  int rc = PairForces(b, b->mp.aF[set]);
+  if (!rc) rc = Sync(b);
   if (rc) return rc;
   *lj = b->hostRes[0];
   *real = b->hostRes[1];
