@@ -20,6 +20,11 @@
 // in registers until the end, so there are no atomics and the order of
 // every sum is fixed by the positions.  Energies and virials: the partner
 // must come later in the cell order, so each pair is met once.
+//
+// Bound by FP64 issue and, at four waves a SIMD, the tail of the last round.
+// 10,000 waters, rc 12 A: forces 336 us (with atom cells, tiles and sorted
+// hit lists 733), virial 170 us (606), energy 173 us (950); 1000 waters, rc
+// 10 A: forces 64 us (154).
 #include <algorithm>
 #include <cmath>
 
@@ -202,6 +207,15 @@ __device__ __forceinline__ Coefs Fresh(Coefs c) {
   return c;
 }
 
+// a b + c with c from scalar registers.  Written out because the compiler
+// otherwise takes the two-operand form and first moves every coefficient to
+// vector registers, two more instructions for each multiply-add.
+__device__ __forceinline__ double FmaS(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+
 // e^y for y in [-700, 0]: y = n ln 2 + r with |r| <= ln 2 / 2, the Taylor
 // series of e^r (truncation 4e-18), scaled by 2^n.
 __device__ __forceinline__ double ExpNeg(Coefs c, double y) {
@@ -210,12 +224,9 @@ __device__ __forceinline__ double ExpNeg(Coefs c, double y) {
   r = fma(-n, 0x1.abc9e3b39803fp-56, r);
   double p = c[0];
 #pragma unroll
-  for (int k = 1; k <= kExpDeg; ++k) p = fma(p, r, c[k]);
+  for (int k = 1; k <= kExpDeg; ++k) p = FmaS(p, r, c[k]);
   return ldexp(p, int(n));
 }
-
-__device__ __noinline__ double ErfcxFar(double x) { return ErfcxTail(x); }
-__device__ __noinline__ double MieFar(double x, double h) { return MiePow(x, h); }
 
 // Energies and virial factors F.r / r^2 of one pair inside the box cutoff
 // (FFParticle::CalcCoulomb / CalcCoulombVir, src/FFParticle.cpp:387-446,
@@ -223,7 +234,7 @@ __device__ __noinline__ double MieFar(double x, double h) { return MiePow(x, h);
 // estimate, then one correction each for r and 1 / r^2, to the last place)
 // stands for every root and division, and one exponential for erfc's and the
 // virial's Gaussian.
-template <bool E, bool F>
+template <bool E, bool F, bool MIE>  // MIE: some repulsion exponent is not 12
 __device__ __forceinline__ PairTerms PairEval(const BoxGeom &g, Coefs c, double d2, double qiqj,
                                               const PairType &t) {
   PairTerms p{0.0, 0.0, 0.0, 0.0};
@@ -242,9 +253,9 @@ __device__ __forceinline__ PairTerms PairEval(const BoxGeom &g, Coefs c, double 
         const double u = (x - kErfcxMid) * kErfcxInvHalf;
         ex = c[kExpDeg + 1];
 #pragma unroll
-        for (int k = 1; k <= kErfcxDeg; ++k) ex = fma(ex, u, c[kExpDeg + 1 + k]);
+        for (int k = 1; k <= kErfcxDeg; ++k) ex = FmaS(ex, u, c[kExpDeg + 1 + k]);
       } else {
-        ex = ErfcxFar(x);
+        ex = ErfcxTail(x);
       }
       const double ec = gauss * ex * ir;
       if (E) p.eReal = qiqj * ec;
@@ -257,7 +268,8 @@ __device__ __forceinline__ PairTerms PairEval(const BoxGeom &g, Coefs c, double 
   if (t.eps6 != 0.0 && !(g.rCutLJSq < d2)) {
     const double rRat2 = t.sig * ir2;
     const double att = rRat2 * rRat2 * rRat2;
-    const double rep = t.nh == 6.0 ? att * att : MieFar(rRat2, t.nh);
+    double rep = att * att;
+    if (MIE && t.nh != 6.0) rep = MiePow(rRat2, t.nh);
     if (E) p.eLJ = t.eps * (rep - att);
     if (F) p.vLJ = t.eps6 * (t.nov6 * rep - att) * ir2;
   }
@@ -274,13 +286,13 @@ struct HomeAtom {
   double x, y, z, q;
 };
 
-template <int MODE, int S>
-__global__ void __launch_bounds__(kPairThreads, 4) PairKernel(const PairArgs a) {
+template <int MODE, int S, bool MIE>
+__global__ void __launch_bounds__(kPairThreads, MIE ? 2 : 4) PairKernel(const PairArgs a) {
   constexpr bool kE = MODE != kVirial, kF = MODE != kEnergy;
   __shared__ int lists[kPairWaves][kAtomList];
   __shared__ HomeAtom homes[kPairWaves][kHomeAtoms];
   __shared__ int htype[kPairWaves][kHomeAtoms];
-  __shared__ PairType tab[kPairTypesLds * kPairTypesLds];
+  __shared__ double tab[5][kPairTypesLds * kPairTypesLds];
   __shared__ double red[kPairWaves][3 * kHomeAtoms];
   __shared__ double bred[kPairWaves];
   const int tid = threadIdx.x, lane = tid % kWave;
@@ -288,8 +300,13 @@ __global__ void __launch_bounds__(kPairThreads, 4) PairKernel(const PairArgs a) 
   const int nt2 = a.ntypes * a.ntypes;
   const bool inLds = a.ntypes <= kPairTypesLds;
   if (inLds)
-    for (int i = tid; i < nt2; i += kPairThreads)
-      tab[i] = PairType{a.sigSq[i], a.epsCn[i], a.nHalf[i], a.epsCn6[i], a.nOver6[i]};
+    for (int i = tid; i < nt2; i += kPairThreads) {
+      tab[0][i] = a.sigSq[i];
+      tab[1][i] = a.epsCn[i];
+      tab[2][i] = a.nHalf[i];
+      tab[3][i] = a.epsCn6[i];
+      tab[4][i] = a.nOver6[i];
+    }
   __syncthreads();
   const int u = blockIdx.x * (kPairWaves / S) + w / S;  // home's place in the cell order
   const int slice = w % S;
@@ -437,11 +454,12 @@ __global__ void __launch_bounds__(kPairThreads, 4) PairKernel(const PairArgs a) 
             PairType t{0.0, 0.0, 0.0, 0.0, 0.0};
             if (ht >> 30) {
               const int idx = (ht & ~(1 << 30)) + tj;
-              t = inLds ? tab[idx]
-                        : PairType{a.sigSq[idx], a.epsCn[idx], a.nHalf[idx], a.epsCn6[idx],
-                                   a.nOver6[idx]};
+              if (inLds)
+                t = PairType{tab[0][idx], tab[1][idx], tab[2][idx], tab[3][idx], tab[4][idx]};
+              else
+                t = PairType{a.sigSq[idx], a.epsCn[idx], a.nHalf[idx], a.epsCn6[idx], a.nOver6[idx]};
             }
-            const PairTerms e = PairEval<kE, kF>(a.g, Fresh(coefs), d2, h.q * qj, t);
+            const PairTerms e = PairEval<kE, kF, MIE>(a.g, Fresh(coefs), d2, h.q * qj, t);
             if (kE) {
               lj += e.eLJ;
               real += e.eReal;
@@ -636,12 +654,23 @@ static int BuildMolCells(gomc_box *b, PairArgs *out) {
 // with less than three waves each.
 constexpr int kPairOneWave = 3072;
 
-template <int MODE>
-static hipError_t LaunchPairs(const PairArgs &a, int blocks, bool split, hipStream_t s) {
+template <int MODE, bool MIE>
+static void LaunchPairsAs(const PairArgs &a, int blocks, bool split, hipStream_t s) {
   if (split)
-    hipLaunchKernelGGL((PairKernel<MODE, kPairWaves>), dim3(blocks), dim3(kPairThreads), 0, s, a);
+    hipLaunchKernelGGL((PairKernel<MODE, kPairWaves, MIE>), dim3(blocks), dim3(kPairThreads), 0, s, a);
   else
-    hipLaunchKernelGGL((PairKernel<MODE, 1>), dim3(blocks), dim3(kPairThreads), 0, s, a);
+    hipLaunchKernelGGL((PairKernel<MODE, 1, MIE>), dim3(blocks), dim3(kPairThreads), 0, s, a);
+}
+
+template <int MODE>
+static hipError_t LaunchPairs(const gomc_box *b, const PairArgs &a, int blocks, bool split) {
+  // any other exponent than 12 brings pow's registers into the kernel
+  bool mie = false;
+  for (double h : b->nHalf) mie = mie || h != 6.0;
+  if (mie)
+    LaunchPairsAs<MODE, true>(a, blocks, split, b->stream);
+  else
+    LaunchPairsAs<MODE, false>(a, blocks, split, b->stream);
   return hipGetLastError();
 }
 
@@ -660,7 +689,7 @@ int BoxInter(gomc_box *b, double *lj, double *real) {
   a.partials = b->partials;
   a.counter = b->counter;
   a.result = b->devRes;
-  HIP_TRY(b, LaunchPairs<kEnergy>(a, blocks, split, b->stream));
+  HIP_TRY(b, LaunchPairs<kEnergy>(b, a, blocks, split));
   rc = Sync(b);
   if (rc) return rc;
   *lj = b->hostRes[0];
@@ -683,7 +712,7 @@ int PairForces(gomc_box *b, double *const f[3]) {
   a.partials = b->partials;
   a.counter = b->counter;
   a.result = b->devRes;
-  HIP_TRY(b, LaunchPairs<kForce>(a, blocks, split, b->stream));
+  HIP_TRY(b, LaunchPairs<kForce>(b, a, blocks, split));
   return GOMC_OK;
 }
 
@@ -708,7 +737,7 @@ int PairVirials(gomc_box *b, double *const com[3], const double **vpart, int *nb
   a.cz = com[2];
   a.mol = b->mol;
   a.vpart = c.vpart;
-  HIP_TRY(b, LaunchPairs<kVirial>(a, blocks, split, b->stream));
+  HIP_TRY(b, LaunchPairs<kVirial>(b, a, blocks, split));
   *vpart = c.vpart;
   *nblocks = blocks;
   return GOMC_OK;
