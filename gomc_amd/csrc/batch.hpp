@@ -25,21 +25,21 @@ constexpr uint64_t kPhiloxTag = 0x474F4D43ull;  // key word 1 of every box strea
 // members exchange their partial energy sums.
 constexpr int kTeamMax = 8;
 // Exchange block per box (64-bit words): tagged partial sums
-// [2 parities][8 members][4].
-constexpr int kXchgWords = 2 * kTeamMax * 4;
+// [2 parities][8 members][kXchgVals].
+constexpr int kXchgVals = 16;
+constexpr int kXchgWords = 2 * kTeamMax * kXchgVals;
 // Polls of a member's counter before a team gives up and flags an error.
 constexpr int64_t kTeamSpinLimit = int64_t(1) << 22;
-// Molecules whose FP64 centres fit in the LDS left beside the static
-// tables, pair queues and near list (160 KiB per CU on gfx950, ~60 KiB
-// static): 4096 x 24 B.
+// Molecules whose FP32 centres are kept in LDS beside the static tables
+// (phase tables of two moves, pair queues, near lists; 78 of the 160 KiB of a
+// CU): 4096 x 12 B.
 constexpr int kBatchLdsMolCap = 4096;
-// Capacity of the per-move list of molecules near the moving one; boxes of
-// more molecules skip the centre cull.
+// Boxes of more molecules skip the centre cull.
 constexpr int kBatchNearCap = 4096;
-// Pair-phase waves per box and the near-list entries each wave may hold:
-// a wave tests at most ceil(4096 / (64 w)) chunks of 64 molecules.
+// Pair-phase waves per box, and the near molecules a wave lists per move:
+// less than a wave's worth left over, and 64 more.
 constexpr int kPairWavesMax = 12;
-constexpr int kNearListLen = 4608;  // 12 x 384, 8 x 576, 4 x 1152
+constexpr int kNearListLen = 128;
 
 // Read-only description of one box (host-filled, 8-byte aligned fields).
 struct BatchBox {
@@ -47,8 +47,7 @@ struct BatchBox {
   double rCutSq, rCutLJSq, rCutCoulSq, rCutLowSq;
   double alpha, beta, pDisp;
   double kc[3];                       // (1/L) * 2pi, the k-vector spacing
-  double nearCutSq;                   // (rc + 2 r_max + 1e-6)^2: centres farther apart
-                                      // than this hold no pair inside the cutoff
+  double twoInvL[3];                  // 2 / L: half-turns per A
   double sigSq[kBatchMaxAtoms * kBatchMaxAtoms];  // per (atom p, atom q) of the kind
   double epsCn[kBatchMaxAtoms * kBatchMaxAtoms];
   double nHalf[kBatchMaxAtoms * kBatchMaxAtoms];
@@ -57,13 +56,15 @@ struct BatchBox {
   int64_t atomOff, molOff, kOff;      // offsets into the flat arrays
   int64_t perAdjust;
   uint64_t seed;
-  uint64_t magicLen, magicLen2;       // ceil(2^32 / len), ceil(2^32 / len^2)
   int natoms, nmols, molLen;
   int K;       // k-vector slots of the box: kChunk * kSeg * kBatchThreads
   int kChunk;  // rounds: segments per thread
   int kSeg;    // S: k-vectors per segment (1, 2, 4 or 8)
   int nmax[3], ewald, elect;
   int cull;  // 1: cull far molecules by their centres before atom pairs
+  float nearCutSqF;  // (rc + 2 r_max + margin)^2: centres farther apart than this hold
+                     // no pair inside the cutoff; the margin covers FP32 centres
+  int wide;          // 1: half of every edge exceeds the cutoff and the molecule's radius
   int team;  // workgroups running the box (1, 2, 4, 8)
   int live;  // bit p * kBatchMaxAtoms + q: atoms p, q interact (charge or LJ)
   int pairWaves;  // waves 0 .. pairWaves-1 run the pair phase (4, 8 or 12)
@@ -79,7 +80,7 @@ struct BatchState {
   double scale[2];    // displacement, rotation
   int64_t step;       // moves made so far (the Philox counter)
   int64_t tries[2], accepted[2], tempTries[2], tempAccepted[2];
-  int64_t pad;
+  int64_t passes;     // passes made so far (the team exchange's sequence)
 };
 
 struct BatchTrace {
@@ -109,7 +110,8 @@ struct BatchArgs {
   const int32_t *kn;          // packed (nx, ny+128, nz+128) bytes, -1 unused slot
   const double *pref;
   double *sumR, *sumI;        // reference structure factors
-  double *dR, *dI;            // structure-factor change of the last trial
+  double *dR, *dI;            // structure-factor change of a pass's first move
+  double *dR2, *dI2;          // and of its second; null: one move per pass
   const int64_t *moves;       // [nboxes] moves to make in this launch
   int ldsMols;                // per-box centre capacity of dynamic LDS
   BatchTrace trace;
@@ -131,6 +133,7 @@ struct gomc_batch {
   double *x = nullptr, *y = nullptr, *z = nullptr, *cx = nullptr, *cy = nullptr, *cz = nullptr;
   int32_t *kn = nullptr;
   double *pref = nullptr, *sumR = nullptr, *sumI = nullptr, *dR = nullptr, *dI = nullptr;
+  double *dR2 = nullptr, *dI2 = nullptr;
   int64_t *moves = nullptr;
   // workgroup task lists (device) and their capacity; team exchange blocks
   gomc::BatchTask *tasks = nullptr;
@@ -183,8 +186,9 @@ struct PackedBox {
 // factors, centres) and packs it at the given offsets; errors go to bt->err.
 int PackBox(gomc_batch *bt, const gomc_system_desc &d, int64_t atomOff, int64_t molOff,
             int64_t kOff, PackedBox &out);
-// Device buffers for `nboxes` boxes and the given flat-array lengths.
-int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec);
+// Device buffers for `nboxes` boxes and the given flat-array lengths; pairs:
+// with the second change of S(k) that passes of two moves need.
+int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec, bool pairs);
 // Team size of a box of n molecules (a function of n alone, so a box's
 // results do not depend on the other boxes of its batch).
 int TeamSize(const gomc_batch *bt, int nmols);

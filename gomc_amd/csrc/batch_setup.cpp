@@ -26,7 +26,7 @@ int BFail(gomc_batch *bt, int code, const std::string &msg) {
 
 void FreeBatch(gomc_batch *bt) {
   void *ptrs[] = {bt->boxes, bt->state, bt->x,    bt->y,    bt->z,    bt->cx,         bt->cy,
-                  bt->cz,    bt->kn,    bt->pref, bt->sumR, bt->sumI, bt->dR, bt->dI, bt->moves,      bt->trace.acc,
+                  bt->cz,    bt->kn,    bt->pref, bt->sumR, bt->sumI, bt->dR, bt->dI, bt->dR2, bt->dI2, bt->moves,      bt->trace.acc,
                   bt->trace.dlj, bt->trace.dreal, bt->trace.drecip, bt->tasks, bt->wgTask,
                   bt->xchg, bt->errFlag, bt->boxTicks};
   for (void *p : ptrs)
@@ -77,26 +77,21 @@ int PackBox(gomc_batch *bt, const gomc_system_desc &d, int64_t atomOff, int64_t 
     P.L[a] = b->geom.L[a];
     P.half[a] = b->geom.half[a];
     P.kc[a] = (1.0 / b->geom.L[a]) * (2.0 * M_PI);
+    P.twoInvL[a] = 2.0 / b->geom.L[a];
     P.nmax[a] = int(b->recipRcut * b->geom.L[a] / (2.0 * M_PI)) + 1;
     if (P.nmax[a] > kBatchMaxN) return BFail(bt, GOMC_ERR_ARG, "box too large for the batched phase tables");
   }
-  // largest atom-to-centre distance of the kind (its first molecule), for
-  // the centre cull of the pair phase
-  double rmax = 0.0;
-  for (int p = 0; p < len; ++p) {
-    double d2 = 0.0;
-    const double *P3[3] = {b->hx.data(), b->hy.data(), b->hz.data()};
-    const double c3[3] = {b->comx[0], b->comy[0], b->comz[0]};
-    for (int a = 0; a < 3; ++a) {
-      double v = P3[a][p] - c3[a];
-      if (v > b->geom.half[a]) v -= b->geom.L[a];
-      else if (v < -b->geom.half[a]) v += b->geom.L[a];
-      d2 += v * v;
-    }
-    rmax = std::max(rmax, std::sqrt(d2));
-  }
-  const double nearCut = std::sqrt(b->geom.rCutSq) + 2.0 * rmax + 1e-6;
-  P.nearCutSq = nearCut * nearCut;
+  // largest atom-to-centre distance of its molecules, for the centre cull of
+  // the pair phase
+  const double rmax = b->molRadius;
+  // FP32 centres: rounding a coordinate, a difference and a box multiple each
+  // moves a distance by less than L 2^-23, all of them by less than 1e-6 L
+  const double lmax = std::max(P.L[0], std::max(P.L[1], P.L[2]));
+  const double nearCut = std::sqrt(b->geom.rCutSq) + 2.0 * rmax + 1e-6 + 2e-6 * lmax;
+  P.nearCutSqF = float(nearCut * nearCut * (1.0 + 1e-6));
+  P.wide = 1;
+  for (int a = 0; a < 3; ++a)
+    if (!(P.half[a] > std::sqrt(b->geom.rCutSq) + rmax + 1e-6)) P.wide = 0;
   // the cull pays when the near sphere is well inside the box
   P.cull = (b->nmols <= kBatchNearCap &&
             (4.0 / 3.0) * M_PI * nearCut * nearCut * nearCut < 0.5 * b->volume) ? 1 : 0;
@@ -139,9 +134,6 @@ int PackBox(gomc_batch *bt, const gomc_system_desc &d, int64_t atomOff, int64_t 
   P.natoms = b->natoms;
   P.nmols = b->nmols;
   P.molLen = len;
-  // exact floor division by len and len^2 for item indices < 2^32 / len^2
-  P.magicLen = ((uint64_t(1) << 32) + uint64_t(len) - 1) / uint64_t(len);
-  P.magicLen2 = ((uint64_t(1) << 32) + uint64_t(len * len) - 1) / uint64_t(len * len);
   if (uint64_t(b->nmols) * len * len >= (uint64_t(1) << 32) / uint64_t(len * len))
     return BFail(bt, GOMC_ERR_ARG, "box too large for the batched item indexing");
   P.ewald = b->ewald;
@@ -251,6 +243,8 @@ BatchArgs MakeArgs(const gomc_batch *bt) {
   a.sumI = bt->sumI;
   a.dR = bt->dR;
   a.dI = bt->dI;
+  a.dR2 = bt->dR2;
+  a.dI2 = bt->dI2;
   a.moves = bt->moves;
   a.tasks = bt->tasks;
   a.wgTask = bt->wgTask;
@@ -262,7 +256,8 @@ BatchArgs MakeArgs(const gomc_batch *bt) {
   return a;
 }
 
-int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec) {
+int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec,
+               bool pairs) {
   BHIP(bt, hipSetDevice(bt->device));
   auto alloc = [&](void **p, size_t bytes) { return hipMalloc(p, std::max<size_t>(bytes, 8)) == hipSuccess; };
   bool ok = hipStreamCreateWithFlags(&bt->stream, hipStreamNonBlocking) == hipSuccess;
@@ -283,6 +278,10 @@ int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t 
   ok &= alloc((void **)&bt->sumI, sizeof(double) * kvec);
   ok &= alloc((void **)&bt->dR, sizeof(double) * kvec);
   ok &= alloc((void **)&bt->dI, sizeof(double) * kvec);
+  if (pairs) {
+    ok &= alloc((void **)&bt->dR2, sizeof(double) * kvec);
+    ok &= alloc((void **)&bt->dI2, sizeof(double) * kvec);
+  }
   // one workgroup per compute unit: the kernel's 1024 threads at 128
   // registers fill a CU, and team members must all be resident at once
   int cus = 0;
@@ -301,6 +300,10 @@ int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t 
   if (kvec > 0) {
     BHIP(bt, hipMemsetAsync(bt->dR, 0, sizeof(double) * kvec, bt->stream));
     BHIP(bt, hipMemsetAsync(bt->dI, 0, sizeof(double) * kvec, bt->stream));
+    if (pairs) {
+      BHIP(bt, hipMemsetAsync(bt->dR2, 0, sizeof(double) * kvec, bt->stream));
+      BHIP(bt, hipMemsetAsync(bt->dI2, 0, sizeof(double) * kvec, bt->stream));
+    }
   }
   bt->totalAtoms = atoms;
   bt->totalMols = mols;
@@ -539,7 +542,7 @@ int gomc_batch_create_tuned(const gomc_system_desc *descs, int nboxes, int devic
     for (auto &pb : packed) teams = teams || pb.P.team > 1;
     if (teams && int64_t(perCU) * cus < gridCap) return fail(GOMC_ERR_STATE);
   }
-  int rc = AllocBatch(bt, nboxes, atoms, mols, kvec);
+  int rc = AllocBatch(bt, nboxes, atoms, mols, kvec, true);
   if (rc) return fail(rc);
   bt->hboxes.resize(nboxes);
   for (int i = 0; i < nboxes; ++i) {

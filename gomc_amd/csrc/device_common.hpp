@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "erfcx_poly.hpp"
 
 namespace gomc {
@@ -75,17 +77,6 @@ __device__ __forceinline__ double LJEnergy(double distSq, double sigmaSq, double
   return epsCn * (repulse - attract);
 }
 
-// FFParticle::CalcVir (src/FFParticle.cpp:327-359): F.r / r^2.
-__device__ __forceinline__ double LJVirial(double distSq, double sigmaSq, double epsCn6,
-                                           double nOver6, double nHalf) {
-  double rNeg2 = 1.0 / distSq;
-  double rRat2 = rNeg2 * sigmaSq;
-  double rRat4 = rRat2 * rRat2;
-  double attract = rRat4 * rRat2;
-  double repulse = (nHalf == 6.0) ? attract * attract : pow(rRat2, nHalf);
-  return epsCn6 * (nOver6 * repulse - attract) * rNeg2;
-}
-
 // FFParticle::CalcCoulomb (src/FFParticle.cpp:387-399).
 __device__ __forceinline__ double CoulombEnergy(const BoxGeom &g, double distSq,
                                                 double qiqj) {
@@ -118,19 +109,6 @@ __device__ __forceinline__ void SincosF32(double ang, double *s, double *c) {
   sincosf(red, &sf, &cf);
   *s = sf;
   *c = cf;
-}
-
-// FFParticle::CalcCoulombVir (src/FFParticle.cpp:432-446).
-__device__ __forceinline__ double CoulombVirial(const BoxGeom &g, double distSq,
-                                                double qiqj) {
-  double dist = sqrt(distSq);
-  if (g.ewald) {
-    double constValue = g.alpha * M_2_SQRTPI;
-    double expConst = exp(-1.0 * (g.alpha * g.alpha) * distSq);
-    double temp = 1.0 - erf(g.alpha * dist);
-    return qiqj * (temp / dist + constValue * expConst) / distSq;
-  }
-  return qiqj / (distSq * dist);
 }
 
 // ---------------------------------------------------------- Philox -------
@@ -186,17 +164,6 @@ __host__ __device__ __forceinline__ double U01(uint64_t v) {
   return double(v) * 0x1p-64 + 0x1p-65;
 }
 
-// erfc for 0 <= x <= 4 as exp(-x^2) erfcx(x), erfcx from the fitted
-// polynomial of erfcx_poly.hpp (relative error about 3e-15); libm beyond.
-__device__ __forceinline__ double ErfcPoly(double x) {
-  if (!(x <= kErfcxUse)) return erfc(x);
-  const double t = (x - kErfcxMid) * kErfcxInvHalf;
-  double p = kErfcxPoly[kErfcxDeg];
-#pragma unroll
-  for (int k = kErfcxDeg - 1; k >= 0; --k) p = fma(p, t, kErfcxPoly[k]);
-  return exp(-(x * x)) * p;
-}
-
 // erfcx(x) = exp(x^2) erfc(x) for x >= 4 from Laplace's continued fraction
 // erfc(x) = exp(-x^2) / sqrt(pi) / (x + (1/2) / (x + 1 / (x + (3/2) / ...))),
 // evaluated from the tail, 24 levels: relative error about 4e-16 for every
@@ -236,63 +203,75 @@ __device__ __forceinline__ double Rsqrt64(double d2) {
   return y;
 }
 
-// The energies (counted when `count`) and virial factors of one in-cutoff
-// pair: FFParticle::CalcCoulomb / CalcCoulombVir (src/FFParticle.cpp:
-// 387-399, 432-446) and CalcEn / CalcVir (295-359).  erfc(a r) is
-// exp(-(a r)^2) erfcx(a r) with erfcx from the fitted polynomial of
-// erfcx_poly.hpp (coefficients `poly`, in LDS), and the same exponential is the virial's Gaussian: one
-// exp and one polynomial per pair instead of libm's erfc, erf and exp, whose
-// range branches split a wave.  (1 - erf is erfc up to rounding: the
-// reference's form differs from this one by about 1e-16 absolute.)
-struct PairTerms {
-  double eLJ, eReal, vLJ, vReal;
+// Coefficients of the pair terms, highest power first: the Taylor series of
+// e^r to r^13 / 13!, then erfcx's fitted polynomial.  Read through the scalar
+// cache into scalar registers each time they are used (Coefs): they cost the
+// vector units nothing there, where LDS would feed four SIMDs one broadcast at
+// a time and 43 held values would not leave room for four waves a SIMD.
+constexpr int kExpDeg = 13;
+struct CoefTable {
+  double c[kExpDeg + 1 + kErfcxDeg + 1];
 };
-__device__ __forceinline__ PairTerms PairMath(const BoxGeom &g, const double *poly, double d2,
-                                              double qiqj, double sig, double eps, double nh,
-                                              double eps6, double nov6, bool count) {
-  PairTerms p{0.0, 0.0, 0.0, 0.0};
-  if (g.elect && qiqj != 0.0 && !(g.rCutCoulSq < d2)) {
-    const double dist = sqrt(d2);
-    if (g.ewald) {
-      const double x = g.alpha * dist;
-      double ec, gauss;
-      if (x <= kErfcxUse) {
-        const double t = (x - kErfcxMid) * kErfcxInvHalf;
-        double px = poly[kErfcxDeg];
-        // read from LDS each step, eight steps' reads issued together: fully
-        // unrolled, the coefficients would be held in 58 VGPRs across the
-        // pair loop
-#pragma unroll 8
-        for (int k = kErfcxDeg - 1; k >= 0; --k) px = fma(px, t, poly[k]);
-        gauss = exp(-(x * x));
-        ec = gauss * px;
-      } else {
-        gauss = exp(-(x * x));
-        ec = gauss * ErfcxTail(x);
-      }
-      if (count) p.eReal = qiqj * ec / dist;
-      p.vReal = qiqj * (ec / dist + g.alpha * M_2_SQRTPI * gauss) / d2;
-    } else {
-      if (count) p.eReal = qiqj / dist;
-      p.vReal = qiqj / (d2 * dist);
-    }
+constexpr CoefTable MakeCoefs() {
+  CoefTable t{};
+  double f = 1.0;
+  for (int k = 0; k <= kExpDeg; ++k) {
+    if (k > 0) f *= k;
+    t.c[kExpDeg - k] = 1.0 / f;
   }
-  if (!(g.rCutLJSq < d2)) {
-    // FFParticle::CalcEn and CalcVir in their operation orders, the
-    // repulsion by MiePow rather than libm's pow
-    if (count) {
-      const double rRat2 = sig / d2;
-      const double attract = rRat2 * rRat2 * rRat2;
-      const double repulse = nh == 6.0 ? attract * attract : MiePow(rRat2, nh);
-      p.eLJ = eps * (repulse - attract);
-    }
-    const double rNeg2 = 1.0 / d2;
-    const double rRat2 = rNeg2 * sig;
-    const double attract = rRat2 * rRat2 * rRat2;
-    const double repulse = nh == 6.0 ? attract * attract : MiePow(rRat2, nh);
-    p.vLJ = eps6 * (nov6 * repulse - attract) * rNeg2;
-  }
-  return p;
+  for (int k = 0; k <= kErfcxDeg; ++k) t.c[kExpDeg + 1 + k] = kErfcxPoly[kErfcxDeg - k];
+  return t;
+}
+static __constant__ CoefTable coefTable = MakeCoefs();
+typedef const double __attribute__((address_space(4))) *Coefs;
+__device__ __forceinline__ Coefs GetCoefs() { return (Coefs)coefTable.c; }
+// The same pointer, as far as the compiler knows another one: what is read
+// through it is not kept from one use to the next.
+__device__ __forceinline__ Coefs Fresh(Coefs c) {
+  asm volatile("" : "+s"(c));
+  return c;
+}
+
+// a b + c with c from scalar registers.  Written out because the compiler
+// otherwise takes the two-operand form and first moves every coefficient to
+// vector registers, two more instructions for each multiply-add.
+__device__ __forceinline__ double FmaS(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+
+// e^y for y in [-700, 0]: y = n ln 2 + r with |r| <= ln 2 / 2, the Taylor
+// series of e^r (truncation 4e-18), scaled by 2^n.
+__device__ __forceinline__ double ExpNeg(Coefs c, double y) {
+  const double n = rint(y * M_LOG2E);
+  double r = fma(-n, 0x1.62e42fefa39efp-1, y);  // ln 2 to 53 bits, and the rest
+  r = fma(-n, 0x1.abc9e3b39803fp-56, r);
+  double p = c[0];
+#pragma unroll
+  for (int k = 1; k <= kExpDeg; ++k) p = FmaS(p, r, c[k]);
+  return ldexp(p, int(n));
+}
+
+// Sum over the wave in a fixed tree, valid in lane 63: four steps within rows
+// of 16 lanes, then the rows.  Lane moves are VALU operations here, a shuffle
+// through LDS is several times their latency.
+__device__ __forceinline__ double WaveSumDpp(double v) {
+  auto step = [](double x, auto ctrl, auto rows) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0u, uint32_t(u), decltype(ctrl)::value,
+                                                    decltype(rows)::value, 0xf, false);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0u, uint32_t(u >> 32), decltype(ctrl)::value,
+                                                    decltype(rows)::value, 0xf, false);
+    return x + __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+  };
+  v = step(v, std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // row_shr:1
+  v = step(v, std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+  v = step(v, std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+  v = step(v, std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+  v = step(v, std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast:15
+  v = step(v, std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});  // row_bcast:31
+  return v;
 }
 
 // The pair terms and phases at precision P: 0 is FP64 throughout, 1 the

@@ -502,8 +502,9 @@ __attribute__((noinline)) __device__ double ErfcOutOfLine(double x) { return erf
 // read from there in the loop, they do not occupy registers.
 __shared__ double sErfcx[kErfcxDeg + 1];
 
-// ErfcPoly (device_common.hpp) with the coefficients from LDS and libm's
-// erfc out of line for x > 4.
+// erfc for 0 <= x <= 4 as exp(-x^2) erfcx(x), erfcx from the fitted polynomial
+// of erfcx_poly.hpp (relative error about 3e-15) with its coefficients in LDS;
+// libm's, out of line, beyond.
 __device__ __forceinline__ double ErfcLds(double x) {
   if (!(x <= kErfcxUse)) return ErfcOutOfLine(x);
   const double t = (x - kErfcxMid) * kErfcxInvHalf;

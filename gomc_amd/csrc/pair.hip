@@ -178,55 +178,9 @@ __device__ __forceinline__ CellRange Range(int at, int n, int reach) {
   return 2 * reach + 1 >= n ? CellRange{0, n} : CellRange{at - reach, 2 * reach + 1};
 }
 
-// Coefficients of the pair terms, highest power first: the Taylor series of
-// e^r to r^13 / 13!, then erfcx's fitted polynomial.  Read through the scalar
-// cache into scalar registers each time they are used (Coefs): they cost the
-// vector units nothing there, where LDS would feed four SIMDs one broadcast at
-// a time and 43 held values would not leave room for four waves a SIMD.
-constexpr int kExpDeg = 13;
-struct CoefTable {
-  double c[kExpDeg + 1 + kErfcxDeg + 1];
+struct PairTerms {
+  double eLJ, eReal, vLJ, vReal;
 };
-constexpr CoefTable MakeCoefs() {
-  CoefTable t{};
-  double f = 1.0;
-  for (int k = 0; k <= kExpDeg; ++k) {
-    if (k > 0) f *= k;
-    t.c[kExpDeg - k] = 1.0 / f;
-  }
-  for (int k = 0; k <= kErfcxDeg; ++k) t.c[kExpDeg + 1 + k] = kErfcxPoly[kErfcxDeg - k];
-  return t;
-}
-__constant__ CoefTable coefTable = MakeCoefs();
-typedef const double __attribute__((address_space(4))) *Coefs;
-__device__ __forceinline__ Coefs GetCoefs() { return (Coefs)coefTable.c; }
-// The same pointer, as far as the compiler knows another one: what is read
-// through it is not kept from one use to the next.
-__device__ __forceinline__ Coefs Fresh(Coefs c) {
-  asm volatile("" : "+s"(c));
-  return c;
-}
-
-// a b + c with c from scalar registers.  Written out because the compiler
-// otherwise takes the two-operand form and first moves every coefficient to
-// vector registers, two more instructions for each multiply-add.
-__device__ __forceinline__ double FmaS(double a, double b, double c) {
-  double d;
-  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
-  return d;
-}
-
-// e^y for y in [-700, 0]: y = n ln 2 + r with |r| <= ln 2 / 2, the Taylor
-// series of e^r (truncation 4e-18), scaled by 2^n.
-__device__ __forceinline__ double ExpNeg(Coefs c, double y) {
-  const double n = rint(y * M_LOG2E);
-  double r = fma(-n, 0x1.62e42fefa39efp-1, y);  // ln 2 to 53 bits, and the rest
-  r = fma(-n, 0x1.abc9e3b39803fp-56, r);
-  double p = c[0];
-#pragma unroll
-  for (int k = 1; k <= kExpDeg; ++k) p = FmaS(p, r, c[k]);
-  return ldexp(p, int(n));
-}
 
 // Energies and virial factors F.r / r^2 of one pair inside the box cutoff
 // (FFParticle::CalcCoulomb / CalcCoulombVir, src/FFParticle.cpp:387-446,

@@ -529,7 +529,10 @@ int gomc_server_create(int device, int precision, int slots, int64_t budget_byte
   bt->teams = false;  // a job's result must not depend on the jobs beside it
   bt->hboxes.assign(slots, BatchBox());
   std::memset(bt->hboxes.data(), 0, sizeof(BatchBox) * slots);
-  int rc = AllocBatch(bt, slots, sv->atomCap, sv->molCap, sv->kCap);
+  // passes of two moves keep 16 more bytes a k-vector slot: where the budget
+  // has room for them beside the arenas
+  const bool pairs = arena + 16.0 * double(sv->kCap) <= double(budget_bytes);
+  int rc = AllocBatch(bt, slots, sv->atomCap, sv->molCap, sv->kCap, pairs);
   if (!rc) {
     std::vector<BatchState> zs(slots);
     std::memset(zs.data(), 0, sizeof(BatchState) * slots);
