@@ -27,7 +27,7 @@ import time
 from . import systems
 from .api import TUNING_FILE, Batch
 
-PAIR12 = (0, 1024, 2048, 4096)
+PAIR12 = (0, 1024, 2048, 3072, 4096)
 TEAMS = ((1800, 2900, 3500), (1600, 2600, 3300), (2000, 2800, 3600), (1500, 2400, 3200),
          (2200, 3100, 3800))
 

@@ -57,7 +57,7 @@ struct BatchBox {
   int64_t perAdjust;
   uint64_t seed;
   int natoms, nmols, molLen;
-  int K;       // k-vector slots of the box: kChunk * kSeg * kBatchThreads
+  int K;       // k-vector slots of the box: kChunk * kSeg * kWidth
   int kChunk;  // rounds: segments per thread
   int kSeg;    // S: k-vectors per segment (1, 2, 4 or 8)
   int nmax[3], ewald, elect;
@@ -67,7 +67,7 @@ struct BatchBox {
   int wide;          // 1: half of every edge exceeds the cutoff and the molecule's radius
   int team;  // workgroups running the box (1, 2, 4, 8)
   int live;  // bit p * kBatchMaxAtoms + q: atoms p, q interact (charge or LJ)
-  int pairWaves;  // waves 0 .. pairWaves-1 run the pair phase (4, 8 or 12)
+  int pairWaves;  // waves 0 .. pairWaves-1 run the pair phase (8 or 12)
   int kWidth;     // W = 1024 - 64 pairWaves: threads of the reciprocal phase and
                   // columns of the k-vector layout
 };
@@ -143,7 +143,7 @@ struct gomc_batch {
   int grid = 0;        // workgroups per launch
   int gridCap = 0;     // workgroups that fit on the device at once
   bool teams = true;   // false: every box runs on one workgroup (serving)
-  gomc_batch_tuning tune{{1800, 2700, 3500}, 1024};
+  gomc_batch_tuning tune{{1800, 2700, 3500}, 3072};
   uint64_t *boxTicks = nullptr;
   std::vector<double> usPerMove;  // measured per-box cost of the last launch (0: none)
   std::vector<double> lastUs;     // per-box time of the last launch
