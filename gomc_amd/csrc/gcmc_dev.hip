@@ -20,9 +20,17 @@
 //                       each wave summing one pair over every atom;
 //   swap reciprocal     every k-vector's new structure factor.
 // Energies are summed in a fixed order, so a run does not depend on timing.
+//
+// One workgroup's move is bound by its CU: the pair and k-vector phases by
+// instruction issue and LDS reads, the rest by thread 0's chain of LDS and
+// global loads and by what the 64 KiB instruction cache cannot hold (the loop is
+// 70 KiB).  Microseconds a move in FP64 on MI355X: 1000 methane / CO2 molecules
+// in 40 A 42.8 -> 29 (pair terms without calls or divisions, the neighbour walk
+// without searches, two k-vectors a set of phases, trials picked by a wave).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <utility>
 
 #include "box.hpp"
 
@@ -59,7 +67,7 @@ struct DevBox {
   double pairEnCorr[kDevKinds * kDevKinds], fugacity[kDevKinds], selfKind[kDevKinds];
   double kindQ[kDevKinds][kDevKindAtoms];
   int kindT[kDevKinds][kDevKindAtoms], kindLen[kDevKinds];
-  double hedB[kDevKinds], hedP[kDevKinds], hedTh[kDevKinds];
+  double hedB[kDevKinds], hedP[kDevKinds], hedSin[kDevKinds], hedCos[kDevKinds];
   double moveW[13], movePerc[2];
   int nMoveTypes, lrc, nkinds, natoms, nmols, ntypes, K;
   int cbmcFirst, cbmcNth, cbmcAng;
@@ -70,9 +78,17 @@ struct DevBox {
   const int *type;
   int *mol;
   const double *sigSq, *epsCn, *nHalf;
-  const double *kx, *ky, *kz, *pref;
-  double *sumR, *sumI, *newR, *newI;
-  const int *kpack;  // k-vector index triples: ix | (iy + 128) << 8 | (iz + 128) << 16
+  const double *kpref;
+  double *sumR, *sumI;
+  // k-vectors two by two, (ix, iy, iz) and (ix, iy, -iz): the first's index
+  // triple ix | (iy + 128) << 8 | (iz + 128) << 16 and the two's places, equal
+  // where the box's half space holds only one of them (then bit 31 is set);
+  // kpref: the prefactor of both
+  const int *kcode, *kfirst, *ksecond;
+  // structure factors of the npairs pairs in their order, [4][npairs]: the
+  // firsts' R and I, then the seconds'; the current ones and a trial's
+  int npairs;
+  double *kCur, *kNew;
   int nmax[3];
   const int *molStart, *molKind;
   int *molBox;
@@ -88,7 +104,7 @@ struct DevBox {
   const int *nbr;
   int *cCount, *cSlots, *aCell, *aSlot;
   uint32_t *lookup;     // live, livePos and lookup are this member's own copies
-  // team: members, this member's rank, its k-vectors [k0, k1), the box's
+  // team: members, this member's rank, its k-vector pairs [k0, k1), the box's
   // exchange block (kDevXchgWords words, zero at the launch's start)
   int team, rank, k0, k1;
   uint64_t *xchg;
@@ -106,7 +122,6 @@ struct DevState {
   // block, once the workgroup has computed it (nextReady), is mt[mtCur ^ 1]
   uint32_t mt[2][kMtN];
   int mtIdx, mtCur, nextReady, status;
-  int recipSwapped;  // the launch ended with the two structure-factor arrays swapped
   double pot[7];  // inter, tc, real, recip, self, corr, total
   double scale[2][kDevKinds];
   uint64_t tries[2][kDevKinds], acc[2][kDevKinds], tTries[2][kDevKinds], tAcc[2][kDevKinds];
@@ -167,6 +182,44 @@ __device__ __forceinline__ GD *G(const double *p) { return (GD *)p; }
 __device__ __forceinline__ GI *G(const int *p) { return (GI *)p; }
 __device__ __forceinline__ GDW *GW(double *p) { return (GDW *)p; }
 
+// p[i] as a byte offset of 32 bits beside a scalar base (i is below 2^28: the
+// largest arrays are the per-cell slots and the atoms).
+template <typename T>
+__device__ __forceinline__ T At(const T __attribute__((address_space(1))) *p, uint32_t i) {
+  return *(const T __attribute__((address_space(1))) *)(
+      (const char __attribute__((address_space(1))) *)p + size_t(uint32_t(i * uint32_t(sizeof(T)))));
+}
+
+// A value every lane holds alike, moved to scalar registers: the box's
+// description comes from LDS, whose loads land in vector registers.
+template <typename T>
+__device__ __forceinline__ T Uni(T v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8);
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, v)));
+  } else {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(u)),
+                   hi = __builtin_amdgcn_readfirstlane(uint32_t(u >> 32));
+    return __builtin_bit_cast(T, (uint64_t(hi) << 32) | lo);
+  }
+}
+__device__ __forceinline__ BoxGeom UniGeom(const BoxGeom &b) {
+  BoxGeom g;
+  for (int d = 0; d < 3; ++d) {
+    g.L[d] = Uni(b.L[d]);
+    g.half[d] = Uni(b.half[d]);
+  }
+  g.rCutSq = Uni(b.rCutSq);
+  g.rCutLJSq = Uni(b.rCutLJSq);
+  g.rCutCoulSq = Uni(b.rCutCoulSq);
+  g.rCutLowSq = Uni(b.rCutLowSq);
+  g.alpha = Uni(b.alpha);
+  g.ewald = Uni(b.ewald);
+  g.elect = Uni(b.elect);
+  return g;
+}
+
 // ---------------------------------------------------------------- MT19937
 // The generator of host_rng.hpp over the state in LDS.  Thread 0 draws;
 // the workgroup computes the next block of state words ahead of need
@@ -196,7 +249,7 @@ NOINLINE __device__ void MtTwist(DevState &s) {
 // The in-place twist, as three data-parallel passes into the other block:
 // word i < 227 reads old words i, i+1, i+397; 227 <= i < 623 reads old i,
 // i+1 and new i-227; word 623 reads old 623, new 0 and new 396.
-__device__ void MtPrepareNext(DevState &s) {
+NOINLINE __device__ void MtPrepareNext(DevState &s) {
   const uint32_t *o = s.mt[s.mtCur];
   uint32_t *nw = s.mt[s.mtCur ^ 1];
   const int t = threadIdx.x;
@@ -279,7 +332,8 @@ __device__ void Apply(const DM3 &r, double x, double y, double z, double &ox, do
 NOINLINE __device__ DM3 AxisAngleD(double theta, double ax, double ay, double az) {
   const double av[3] = {ax, ay, az};
   const double cross[3][3] = {{0.0, -az, ay}, {az, 0.0, -ax}, {-ay, ax, 0.0}};
-  const double c = cos(theta), s = sin(theta);
+  double c, s;
+  sincospi(theta * M_1_PI, &s, &c);
   DM3 r;
   for (int i = 0; i < 3; ++i)
     for (int j = 0; j < 3; ++j) {
@@ -290,13 +344,13 @@ NOINLINE __device__ DM3 AxisAngleD(double theta, double ax, double ay, double az
 }
 // TransformMatrix::UniformRandom, as UniformRotation in host_rng.hpp.
 NOINLINE __device__ DM3 UniformRotationD(double u1, double u2, double u3) {
-  u1 *= 2.0 * M_PI;
-  u1 -= M_PI;
-  u2 *= 2.0 * M_PI;
+  // angles in half-turns: the reduction is exact and its code short
   u3 *= 2.0;
   const double r = sqrt(u3);
-  const double vx = sin(u2) * r, vy = cos(u2) * r, vz = sqrt(2.0 - u3);
-  const double sinTh = sin(u1), cosTh = cos(u1);
+  double s2, c2, sinTh, cosTh;
+  sincospi(2.0 * u2, &s2, &c2);
+  sincospi(2.0 * u1 - 1.0, &sinTh, &cosTh);
+  const double vx = s2 * r, vy = c2 * r, vz = sqrt(2.0 - u3);
   const double sx = vx * cosTh - vy * sinTh;
   const double sy = vx * sinTh + vy * cosTh;
   DM3 m;
@@ -316,39 +370,65 @@ __device__ uint32_t NumKindInBox(const DevBox &B, const DevState &s, int k, int 
   return s.bkStart[box * B.nkinds + k + 1] - s.bkStart[box * B.nkinds + k];
 }
 
-// PRNG::PickWeighted (src/PRNG.h:167-203).
-NOINLINE __device__ int PickWeightedD(DevState &s, const double *w, int n, double total) {
-  const double draw = MtClosed(s) * total;
-  double sum = 0.0;
-  for (int i = 0; i < n; ++i) {
-    sum += w[i];
-    if (sum >= draw) return i;
-  }
-  int lastZero = n;
-  for (int i = n - 1; i > 0 && w[i] == 0.0; --i) lastZero = i;
-  lastZero--;
-  if (fabs(draw - total) < 0.001) return lastZero;
-  return -1;
+// The k-th of n values a wave's lanes hold, in every lane.
+__device__ __forceinline__ double LaneValue(double v, int k) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(u), k),
+                 hi = __builtin_amdgcn_readlane(uint32_t(u >> 32), k);
+  return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
 }
 
-// Four sums over the workgroup, valid in c.res after the call.
+// The weights of a stage's n trials (lane i's w) summed in trial order; `upto`
+// is the sum to this lane's trial.
+__device__ __forceinline__ double WeightSum(double w, int n, double &upto) {
+  const int lane = threadIdx.x % kWave;
+  double sum = 0.0;
+  upto = 0.0;
+  for (int i = 0; i < n; ++i) {
+    sum += LaneValue(w, i);
+    if (lane == i) upto = sum;
+  }
+  return sum;
+}
+
+// PRNG::PickWeighted (src/PRNG.h:167-203) by a whole wave, from WeightSum's
+// results: the first trial whose running sum reaches the draw.
+__device__ __forceinline__ int PickWeightedD(DevState &s, double w, int n, double total,
+                                             double upto) {
+  const int lane = threadIdx.x % kWave;
+  double draw = 0.0;
+  if (lane == 0) draw = MtClosed(s) * total;
+  draw = LaneValue(draw, 0);
+  const uint64_t reach = __ballot(lane < n && upto >= draw);
+  if (reach) return __ffsll((unsigned long long)reach) - 1;
+  if (!(fabs(draw - total) < 0.001)) return -1;
+  int lastZero = n;  // the last trial of any weight
+  for (int i = n - 1; i > 0 && LaneValue(w, i) == 0.0; --i) lastZero = i;
+  return lastZero - 1;
+}
+
+// Four sums over the workgroup, valid in c.res after the call: each wave's by
+// lane moves, then one value a lane (wave l / 4, sum l % 4) in wave 0, added in
+// a fixed tree.
 __device__ void BlockSum4(Ctl &c, double a, double b, double d, double e) {
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  a = WaveSum(a);
-  b = WaveSum(b);
-  d = WaveSum(d);
-  e = WaveSum(e);
-  if (lane == 0) {
+  a = WaveSumDpp(a);
+  b = WaveSumDpp(b);
+  d = WaveSumDpp(d);
+  e = WaveSumDpp(e);
+  if (lane == kWave - 1) {
     c.red[wave][0] = a;
     c.red[wave][1] = b;
     c.red[wave][2] = d;
     c.red[wave][3] = e;
   }
   __syncthreads();
-  if (threadIdx.x < 4) {
-    double r = 0.0;
-    for (int w = 0; w < kDevWaves; ++w) r += c.red[w][threadIdx.x];
-    c.res[threadIdx.x] = r;
+  static_assert(kDevWaves * 4 == kWave, "one partial a lane");
+  if (wave == 0) {
+    double r = c.red[lane >> 2][lane & 3];
+#pragma unroll
+    for (int off = kWave / 2; off >= 4; off >>= 1) r += __shfl_down(r, off, kWave);
+    if (lane < 4) c.res[lane] = r;
   }
   __syncthreads();
 }
@@ -413,19 +493,24 @@ NOINLINE __device__ void TeamExchange(const DevBox &B, DevState &s, Ctl &c, int 
 // ---------------------------------------------------------- cell table --
 // The box's live atoms by cell, walked as CellList::EnumerateLocal walks the
 // 27 cells around a position (CalculateEnergy.cpp:595,745).  A wave takes
-// the 27 cells' counts in its lanes, their running sum gives each cell's
-// first index, and item idx of the neighbourhood is found by a binary
-// search of those starts.
+// the 27 cells' counts in its lanes, and their running sum gives each cell's
+// first index; a lane walks the neighbourhood's items in rising order and
+// moves its cell along with them.
 
 __device__ __forceinline__ bool UseCells(const DevBox &B, const Ctl &c) {
   return B.cells && !c.cellsOff;
 }
 
-// Wave-wide: the 27 cells around (px, py, pz) into cells[27] and their
-// first indices into start[28] (start[27] the total), in LDS; returns the
+// A neighbourhood: each cell's first slot less its first index (an item's slot
+// is this plus its index) and the index past its last item.
+struct WaveCellList {
+  int base[27], end[27];
+};
+
+// Wave-wide: the 27 cells around (px, py, pz) into `w`, in LDS; returns the
 // total.  Called by every lane of the wave.
 __device__ __forceinline__ int WaveCells(const DevBox &B, double px, double py, double pz, int lane,
-                                         int *cells, int *start) {
+                                         WaveCellList &w) {
   const int c0 = CellOf(px, py, pz, B.cs, B.edge);
   int cell = 0, n = 0;
   if (lane < 27) {
@@ -440,28 +525,20 @@ __device__ __forceinline__ int WaveCells(const DevBox &B, double px, double py, 
   }
   __builtin_amdgcn_wave_barrier();  // the wave's last reads of these arrays are done
   if (lane < 27) {
-    cells[lane] = cell;
-    start[lane + 1] = incl;
+    w.base[lane] = cell * B.ccap - (incl - n);
+    w.end[lane] = incl;
   }
-  if (lane == 0) start[0] = 0;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   return __shfl(incl, 26, kWave);
 }
 
-// Atom idx (0 <= idx < start[27]) of a neighbourhood from WaveCells.
-__device__ __forceinline__ int CellAtom(const DevBox &B, const int *cells, const int *start,
-                                        int idx) {
-  int lo = 0, hi = 27;  // the last cell whose first index is <= idx
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (start[mid] <= idx)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  return G(B.cSlots)[cells[lo] * B.ccap + (idx - start[lo])];
+// Slot of item idx (below the neighbourhood's total), `at` the cell of the
+// lane's last item of it.
+__device__ __forceinline__ int CellSlot(const WaveCellList &w, int idx, int &at) {
+  while (idx >= w.end[at]) ++at;
+  return w.base[at] + idx;
 }
 
 // Thread 0: CellList::RemoveMol / AddMol for one atom (CellList.h:28-29):
@@ -496,206 +573,408 @@ NOINLINE __device__ void CellPlace(const DevBox &B, Ctl &c, int a, double x, dou
 }
 
 // ------------------------------------------------- workgroup energy phases --
-__attribute__((noinline)) __device__ double ErfcOutOfLine(double x) { return erfc(x); }
-
-// The erfcx polynomial's coefficients, copied to LDS at the kernel's start:
-// read from there in the loop, they do not occupy registers.
-__shared__ double sErfcx[kErfcxDeg + 1];
-
-// erfc for 0 <= x <= 4 as exp(-x^2) erfcx(x), erfcx from the fitted polynomial
-// of erfcx_poly.hpp (relative error about 3e-15) with its coefficients in LDS;
-// libm's, out of line, beyond.
-__device__ __forceinline__ double ErfcLds(double x) {
-  if (!(x <= kErfcxUse)) return ErfcOutOfLine(x);
-  const double t = (x - kErfcxMid) * kErfcxInvHalf;
-  double p = sErfcx[kErfcxDeg];
+// Pair terms at precision P (FFParticle::CalcEn / CalcCoulomb,
+// src/FFParticle.cpp:295-399).  FP64: one reciprocal square root (a
+// Newton-refined estimate, then one correction each for r and 1 / r^2, to the
+// last place) stands for the root and the divisions, e^-x^2 and erfcx are
+// polynomials whose coefficients are scalar operands, and nothing is called:
+// a call would save and restore the registers of the pair loops.
+template <int P>
+__device__ __forceinline__ void PairTermsDev(const BoxGeom &g, Coefs cf, double d2, double qiqj,
+                                             double sigmaSq, double epsCn, double nHalf,
+                                             double sign, double &lj, double &real) {
+  const bool coul = g.elect && qiqj != 0.0 && !(g.rCutCoulSq < d2);
+  const bool inLJ = !(g.rCutLJSq < d2);
+  if (P) {
+    if (coul) real += sign * CoulombEnergyF32(g, d2, qiqj);
+    if (inLJ) lj += sign * LJEnergyF32(d2, sigmaSq, epsCn, nHalf);
+    return;
+  }
+  d2 = fmax(d2, 0x1p-1022);  // coincident atoms: huge, not 0 x inf
+  const double ir = Rsqrt64(d2);
+  double ir2 = ir * ir;
+  ir2 = fma(ir2, fma(-d2, ir2, 1.0), ir2);
+  if (coul) {
+    double e = qiqj * ir;
+    if (g.ewald) {
+      double dist = d2 * ir;
+      dist = fma(fma(-dist, dist, d2), 0.5 * ir, dist);
+      const double x = g.alpha * dist;
+      double ex;
+      if (x <= kErfcxUse) {
+        const double u = (x - kErfcxMid) * kErfcxInvHalf;
+        ex = cf[kExpDeg + 1];
 #pragma unroll
-  for (int k = kErfcxDeg - 1; k >= 0; --k) p = fma(p, t, sErfcx[k]);
-  return exp(-(x * x)) * p;
-}
-
-// erfc-Coulomb at precision P; FP64 through the erfcx polynomial.
-template <int P>
-__device__ __forceinline__ double CoulDev(const BoxGeom &g, double d2, double qiqj) {
-  if (P) return CoulombEnergyF32(g, d2, qiqj);
-  const double dist = sqrt(d2);
-  if (g.ewald) return qiqj * ErfcLds(g.alpha * dist) / dist;
-  return qiqj / dist;
-}
-
-// The Mie repulsion for exponents other than 12, out of line so that its
-// pow does not weigh on the registers of the pair loops.
-__attribute__((noinline)) __device__ double PowOutOfLine(double x, double y) { return pow(x, y); }
-
-// LJEnergy / LJEnergyF32 (device_common.hpp) with that out-of-line pow.
-template <int P>
-__device__ __forceinline__ double LJDev(double d2, double sigmaSq, double epsCn, double nHalf) {
-  if (P) return LJEnergyF32(d2, sigmaSq, epsCn, nHalf);
-  const double rRat2 = sigmaSq / d2;
-  const double rRat4 = rRat2 * rRat2;
-  const double attract = rRat4 * rRat2;
-  const double repulse = (nHalf == 6.0) ? attract * attract : PowOutOfLine(rRat2, nHalf);
-  return epsCn * (repulse - attract);
+        for (int k = 1; k <= kErfcxDeg; ++k) ex = FmaS(ex, u, cf[kExpDeg + 1 + k]);
+      } else {
+        ex = ErfcxTail(x);
+      }
+      e *= ExpNeg(cf, fmax(-(x * x), -700.0)) * ex;
+    }
+    real += sign * e;
+  }
+  if (inLJ) {
+    const double rRat2 = sigmaSq * ir2;
+    const double att = rRat2 * rRat2 * rRat2;
+    double rep = att * att;
+    if (nHalf != 6.0) rep = MiePow(rRat2, nHalf);
+    lj += sign * (epsCn * (rep - att));
+  }
 }
 
 // FP64 phases e^{i k.r} of a trial's positions as products of per-axis
-// tables e^{i (2 pi n / L_a) r_a}, |n| <= nmax_a: `np` positions given by
-// (px, py, pz) in LDS, tab[p][axis][n + kDevNMax] = (cos, sin).
-// With P = 1 the same LDS holds FP32 entries (float2, same indexing) and
-// the products are FP32 (the mixed mode's phases).
+// tables e^{i (2 pi n / L_a) r_a}, |n| <= nmax_a: position p of a trial is its
+// new one of atom p, or its old one of atom p - kDevKindAtoms,
+// tab[p][axis][n + kDevNMax] = (cos, sin).  With P = 1 the same LDS holds FP32
+// entries (float2, same indexing) and the products are FP32 (the mixed mode's
+// phases).
+//
+// Half a wave (a wave beyond nmax = 31) makes one axis of one position, n >= 0,
+// in half-turns, whose reduction is exact and short; n < 0 is the conjugate.
+// The last waves start: the first have the neighbour cells to find.
 typedef double2 PhaseTab[kDevPos][3][kTab];
-template <int P>
-__device__ void BuildPhases(const DevBox &B, const double *px, const double *py,
-                            const double *pz, int np, PhaseTab &tab) {
-  for (int e = threadIdx.x; e < np * 3 * kTab; e += kDevThreads) {
-    const int p = e / (3 * kTab), a = (e / kTab) % 3, n = e % kTab - kDevNMax;
-    if (n < -B.nmax[a] || n > B.nmax[a]) continue;
-    const double r = a == 0 ? px[p] : (a == 1 ? py[p] : pz[p]);
-    const double ca = (1.0 / B.g.L[a]) * (2.0 * M_PI);
+template <int P, bool OLD>
+__device__ __forceinline__ void BuildPhases(const DevBox &B, const Ctl &c, int len, PhaseTab &tab) {
+  const int nm = max(B.nmax[0], max(B.nmax[1], B.nmax[2]));
+  const int per = nm < 32 ? 32 : 64;
+  const int n = (kDevThreads - 1 - int(threadIdx.x)) & (per - 1);
+  const int rows = (OLD ? 2 : 1) * 3 * len;
+  for (int row = (kDevThreads - 1 - int(threadIdx.x)) / per; row < rows; row += kDevThreads / per) {
+    const int v = row / 3, a = row - 3 * v;  // v-th position: new ones, then old
+    if (n > B.nmax[a]) continue;
+    const bool old = OLD && v >= len;
+    const int i = old ? v - len : v, p = old ? kDevKindAtoms + i : i;
+    const double *pos = old ? (a == 0 ? c.ox : (a == 1 ? c.oy : c.oz))
+                            : (a == 0 ? c.nx : (a == 1 ? c.ny : c.nz));
     double sn, cs;
-    sincos((ca * n) * r, &sn, &cs);
-    if (P)
-      reinterpret_cast<float2 *>(&tab[0][0][0])[e] = make_float2(float(cs), float(sn));
-    else
-      tab[p][a][n + kDevNMax] = make_double2(cs, sn);
+    sincospi(double(n) * (2.0 * (pos[i] / B.g.L[a])), &sn, &cs);
+    if (P) {
+      float2 *t = reinterpret_cast<float2 *>(&tab[0][0][0]) + (p * 3 + a) * kTab + kDevNMax;
+      t[n] = make_float2(float(cs), float(sn));
+      t[-n] = make_float2(float(cs), n ? -float(sn) : float(sn));
+    } else {
+      tab[p][a][kDevNMax + n] = make_double2(cs, sn);
+      tab[p][a][kDevNMax - n] = make_double2(cs, n ? -sn : sn);
+    }
   }
-  __syncthreads();
 }
 
 __device__ __forceinline__ double2 CMulD(double2 a, double2 b) {
-  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+  return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 __device__ __forceinline__ float2 CMulF(float2 a, float2 b) {
   return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// e^{i k.r} of table position p for the k-vector with index triple (ix, iy, iz).
-template <int P>
-__device__ __forceinline__ double2 Phase(const PhaseTab &tab, int p, int ix, int iy, int iz) {
-  if (P) {
-    const float2 *t = reinterpret_cast<const float2 *>(&tab[0][0][0]) + p * 3 * kTab;
-    const float2 e = CMulF(CMulF(t[ix + kDevNMax], t[kTab + iy + kDevNMax]),
-                           t[2 * kTab + iz + kDevNMax]);
-    return make_double2(e.x, e.y);
-  }
-  return CMulD(CMulD(tab[p][0][ix + kDevNMax], tab[p][1][iy + kDevNMax]),
-               tab[p][2][iz + kDevNMax]);
+// e^{i k.r} of a table position (its row's three axes) for the k-vectors
+// (ix, iy, iz) and (ix, iy, -iz): one product of the x and y entries and four
+// real products of that with the z entry serve both.
+template <typename T2>
+struct TwoPhases {
+  T2 a, b;
+};
+__device__ __forceinline__ TwoPhases<double2> PhasesOf(const double2 *t, int ix, int iy, int iz) {
+  const double2 e = CMulD(t[ix], t[iy]), z = t[iz];
+  const double cc = e.x * z.x, sc = e.y * z.x;
+  return {make_double2(fma(-e.y, z.y, cc), fma(e.x, z.y, sc)),
+          make_double2(fma(e.y, z.y, cc), fma(-e.x, z.y, sc))};
 }
+__device__ __forceinline__ TwoPhases<float2> PhasesOf(const float2 *t, int ix, int iy, int iz) {
+  const float2 e = CMulF(t[ix], t[iy]), z = t[iz];
+  const float cc = e.x * z.x, ss = e.y * z.y, sc = e.y * z.x, cs = e.x * z.y;
+  return {make_float2(cc - ss, cs + sc), make_float2(cc + ss, sc - cs)};
+}
+
+// The new structure factor of every k-vector of the member and its energy
+// terms, by threads r0 .. r0 + rn - 1: the phases of table rows 0 .. len - 1
+// come with weight `sign`, those of rows kDevKindAtoms .. (OLD) leave.  The
+// next pair's values are loaded before this one is worked on.  Bound by LDS
+// reads (three entries a position) and by the structure factors' way through
+// the cache: two k-vectors share a set of reads, and a launch keeps them in the
+// pairs' order, where a wave's accesses are consecutive (in the box's order the
+// mirrors come in short descending runs, and the cache lines cost what the
+// reads save).  A transfer's 6600 k-vectors in 40 A took 6.0 us one by one,
+// 5.7 in the box's order, 5.0 so.
+template <int P, bool OLD>
+__device__ __forceinline__ double RecipTerms(const DevBox &B, const Ctl &c, const PhaseTab &tab,
+                                             int r0, int rn, double sign) {
+  const int len = Uni(c.len), k1 = Uni(B.k1);
+  const uint32_t np = Uni(B.npairs);
+  const GD *pref = Uni(G(B.kpref)), *cur = Uni(G(B.kCur));
+  const GI *kcode = Uni(G(B.kcode));
+  GDW *out = Uni(GW(B.kNew));
+  using T2 = std::conditional_t<P != 0, float2, double2>;
+  double q[kDevKindAtoms];
+#pragma unroll
+  for (int p = 0; p < kDevKindAtoms; ++p) {
+    const double qp = p < len ? c.mq[p] : 0.0;
+    q[p] = Uni(fabs(qp) < 0.000000001 ? 0.0 : qp * sign);
+  }
+  struct Item {
+    int code;
+    double Ra, Ia, Rb, Ib, pf;
+  };
+  auto load = [&](int k, Item &it) {
+    it.code = At(kcode, k);  // bit 31: the first k-vector alone
+    it.pf = At(pref, k);
+    it.Ra = At(cur, k);
+    it.Ia = At(cur + np, k);
+    it.Rb = At(cur + 2 * np, k);
+    it.Ib = At(cur + 3 * np, k);
+  };
+  int k = Uni(B.k0) + int(threadIdx.x) - r0;
+  if (k >= k1) return 0.0;
+  double e = 0.0;
+  Item now, next;
+  load(k, now);
+  while (true) {
+    load(min(k + rn, k1 - 1), next);
+    const int ix = kDevNMax + (now.code & 0xff),
+              iy = kTab + kDevNMax + ((now.code >> 8) & 0xff) - 128,
+              iz = 2 * kTab + kDevNMax + ((now.code >> 16) & 0xff) - 128;
+    double aR = 0.0, aI = 0.0, bR = 0.0, bI = 0.0;
+#pragma unroll
+    for (int p = 0; p < kDevKindAtoms; ++p) {
+      if (q[p] == 0.0) continue;
+      auto add = [&](int row, double w) {
+        const auto f = PhasesOf(reinterpret_cast<const T2 *>(&tab[0][0][0]) + row * 3 * kTab,
+                                ix, iy, iz);
+        aR = fma(w, double(f.a.x), aR);
+        aI = fma(w, double(f.a.y), aI);
+        bR = fma(w, double(f.b.x), bR);
+        bI = fma(w, double(f.b.y), bI);
+      };
+      add(p, q[p]);
+      if (OLD) add(kDevKindAtoms + p, -q[p]);
+    }
+    const double Ra = now.Ra + aR, Ia = now.Ia + aI, Rb = now.Rb + bR, Ib = now.Ib + bI;
+    out[k] = Ra;
+    out[np + k] = Ia;
+    out[2 * np + k] = Rb;
+    out[3 * np + k] = Ib;
+    const double ta = Ra * Ra + Ia * Ia, tb = now.code < 0 ? 0.0 : Rb * Rb + Ib * Ib;
+    e += (ta + tb) * now.pf;
+    k += rn;
+    if (k >= k1) break;
+    now = next;
+  }
+  return e;
+}
+
+// The member's structure factors into its pairs' order, at a launch's start,
+// and back at its end.
+__device__ void GatherRecip(const DevBox &B) {
+  const size_t np = B.npairs;
+  for (int k = B.k0 + int(threadIdx.x); k < B.k1; k += kDevThreads) {
+    const int a = B.kfirst[k], b = B.ksecond[k];
+    B.kCur[k] = B.sumR[a];
+    B.kCur[np + k] = B.sumI[a];
+    B.kCur[2 * np + k] = B.sumR[b];
+    B.kCur[3 * np + k] = B.sumI[b];
+  }
+}
+__device__ void ScatterRecip(const DevBox &B) {
+  const size_t np = B.npairs;
+  for (int k = B.k0 + int(threadIdx.x); k < B.k1; k += kDevThreads) {
+    const int a = B.kfirst[k], b = B.ksecond[k];
+    B.sumR[a] = B.kCur[k];
+    B.sumI[a] = B.kCur[np + k];
+    if (a == b) continue;
+    B.sumR[b] = B.kCur[2 * np + k];
+    B.sumI[b] = B.kCur[3 * np + k];
+  }
+}
+
 // In-cutoff pairs found by a wave wait in its queue in LDS until 64 are
 // there; the wave then evaluates 64 pair terms at once, one per lane, so
 // the erfc path runs with full waves however sparse the cutoff sphere is.
 constexpr int kQCap = 2 * kWave;
 struct WaveQ {
-  double d2[kQCap], qq[kQCap];
-  int code[kQCap];  // LJ table index * 2 + (1 if the term is added, 0 if subtracted)
+  double d2[kQCap];
+  int code[kQCap];  // atom * 8 + position
 };
 __shared__ WaveQ sQ[kDevWaves];
 
-template <int P>
-__device__ __forceinline__ void DrainQ(const BoxGeom &g, WaveQ &q, int n, int lane,
-                                       const GD *sigSq, const GD *epsCn, const GD *nHalf,
-                                       double &lj, double &real) {
-  if (lane < n) {
-    const double d2 = q.d2[lane], qq = q.qq[lane];
-    const int code = q.code[lane], idx = code >> 1;
-    const double sign = (code & 1) ? 1.0 : -1.0;
-    if (g.elect && qq != 0.0 && !(g.rCutCoulSq < d2)) real += sign * CoulDev<P>(g, d2, qq);
-    if (!(g.rCutLJSq < d2)) lj += sign * LJDev<P>(d2, sigSq[idx], epsCn[idx], nHalf[idx]);
-  }
-}
-
-// Appends this lane's pair (when `in`) to the wave's queue; drains 64 when
-// the queue holds that many.  Called by every lane of the wave.
-template <int P>
-__device__ __forceinline__ void PushQ(const BoxGeom &g, WaveQ &q, int &cnt, int lane, bool in,
-                                      double d2, double qq, int code, const GD *sigSq,
-                                      const GD *epsCn, const GD *nHalf, double &lj,
-                                      double &real) {
-  const uint64_t m = __ballot(in);
-  if (in) {
-    const int pos = cnt + __popcll(m & ((uint64_t(1) << lane) - 1));
-    q.d2[pos] = d2;
-    q.qq[pos] = qq;
-    q.code[pos] = code;
-  }
-  cnt += __popcll(m);
-  __builtin_amdgcn_wave_barrier();
-  if (cnt >= kWave) {
-    DrainQ<P>(g, q, kWave, lane, sigSq, epsCn, nHalf, lj, real);
-    __builtin_amdgcn_wave_barrier();
-    if (lane < cnt - kWave) {
-      q.d2[lane] = q.d2[kWave + lane];
-      q.qq[lane] = q.qq[kWave + lane];
-      q.code[lane] = q.code[kWave + lane];
-    }
-    cnt -= kWave;
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
 // Each wave's neighbourhood from WaveCells.
-__shared__ int sWCell[kDevWaves][27], sWStart[kDevWaves][28];
+__shared__ WaveCellList sWCell[kDevWaves];
+
+// Minimum image by the nearest multiple of the edge: for coordinates inside the
+// box the same single addition or subtraction as MinImage, in three
+// instructions for nine.
+__device__ __forceinline__ double Nearest(double d, double L, double inv) {
+  return fma(-rint(d * inv), L, d);
+}
+
+// The lane's sums of a wave's pairs.
+struct PairSums {
+  double lj, real, ov;
+};
+// The pairs of positions p0 .. p0 + npos - 1 of the control block's list with
+// the atoms of their neighbourhoods, sWCell[cell0] on (or, with the cell walk
+// off, with every live atom), by nw waves of which this is wave w0: the items
+// of all positions in one sequence, 64 a turn.  Bit v of newMask: position v's
+// terms are added, and its pairs tested for overlap; else subtracted.  Atoms
+// [skipSt, skipEnd) are left out.  Bound by instruction issue (a CU's four SIMDs
+// take four cycles for each of a wave's instructions): the test holds what it
+// must and all else, charges and types included, waits for the pairs inside the
+// cutoff; one copy for every caller, since the whole move loop should stay in
+// the 64 KiB instruction cache.  A CBMC stage of 16 positions, 840 neighbour
+// atoms each (1000 methane / CO2 molecules in 40 A): 12.3 us with 105
+// instructions a test and 170 a pair term, 7.9 us with about 62 and 105.
+template <int P>
+NOINLINE __device__ PairSums PairItems(const DevBox &B, const Ctl &c, int p0_, int npos_, int w0_,
+                                       int nw_, int cell0_, int skipSt_, int skipEnd_,
+                                       int newMask_) {
+  const int p0 = Uni(p0_), npos = Uni(npos_), w0 = Uni(w0_), nw = Uni(nw_), cell0 = Uni(cell0_),
+            skipSt = Uni(skipSt_), skipEnd = Uni(skipEnd_), newMask = Uni(newMask_);
+  const BoxGeom g = UniGeom(B.g);
+  const bool walk = Uni(int(UseCells(B, c))) != 0;
+  const int ntypes = Uni(B.ntypes), nLive = Uni(c.nLive);
+  const GD *q = Uni(G(B.q));
+  const GI *type = Uni(G(B.type));
+  const GD *sigSq = Uni(G(B.sigSq)), *epsCn = Uni(G(B.epsCn)), *nHalf = Uni(G(B.nHalf));
+  const Coefs coefs = GetCoefs();
+  PairSums sum{0.0, 0.0, 0.0};
+  // the index past position v's last item
+  int ends[kDevPos], items = 0;
+#pragma unroll
+  for (int v = 0; v < kDevPos; ++v) {
+    if (v < npos) items += walk ? Uni(sWCell[cell0 + v].end[26]) : nLive;
+    ends[v] = items;
+  }
+  // a wave's items are consecutive, so its lanes pass few cells a turn
+  const int chunk = Uni((items + nw * kWave - 1) / (nw * kWave) * kWave);
+  const int begin = w0 * chunk, total = min(items, begin + chunk);
+  if (begin >= total) return sum;
+  auto end = [&](int v) {
+    int r = ends[0];
+#pragma unroll
+    for (int k = 1; k < kDevPos; ++k) r = v >= k ? ends[k] : r;
+    return r;
+  };
+  const int lane = threadIdx.x % kWave;
+  const GD *x = Uni(G(B.x)), *y = Uni(G(B.y)), *z = Uni(G(B.z));
+  const GI *slots = Uni(walk ? G(B.cSlots) : G(B.live));
+  const double ix = Uni(1.0 / g.L[0]), iy = Uni(1.0 / g.L[1]), iz = Uni(1.0 / g.L[2]);
+  WaveQ &wq = sQ[threadIdx.x / kWave];
+  constexpr int step = kWave;
+  int vA = 0, first = 0, last = ends[0], at = 0, cnt = 0;
+  while (begin >= last) {
+    first = last;
+    last = end(++vA);
+  }
+  if (walk)  // the first item's cell
+    at = __popcll(__ballot(lane < 27 && sWCell[cell0 + vA].end[min(lane, 26)] <= begin - first));
+  int v = vA;
+  // the atom and position of item `it`, items in rising order
+  auto item = [&](int it, uint32_t &j, int &w) {
+    it = min(it, total - 1);
+    if (it >= last) {
+      do {
+        first = last;
+        last = end(++vA);
+      } while (it >= last);
+      at = 0;
+    }
+    w = vA;
+    const int idx = it - first;
+    j = At(slots, walk ? CellSlot(sWCell[cell0 + vA], idx, at) : idx);
+  };
+  double px = c.cx[p0 + v], py = c.cy[p0 + v], pz = c.cz[p0 + v];
+  // a turn's atoms are found two turns ahead and their coordinates read one
+  // turn ahead: the two loads hang on each other
+  uint32_t j0, j1;
+  int v0, v1;
+  item(begin + lane, j0, v0);
+  double x0 = At(x, j0), y0 = At(y, j0), z0 = At(z, j0);
+  item(begin + lane + step, j1, v1);
+  for (int base = begin;; base += step) {
+    const double x1 = At(x, j1), y1 = At(y, j1), z1 = At(z, j1);
+    uint32_t j2;
+    int v2;
+    item(base + lane + 2 * step, j2, v2);
+    if (v0 != v) {
+      v = v0;
+      px = c.cx[p0 + v];
+      py = c.cy[p0 + v];
+      pz = c.cz[p0 + v];
+    }
+    const double dx = Nearest(px - x0, g.L[0], ix), dy = Nearest(py - y0, g.L[1], iy),
+                 dz = Nearest(pz - z0, g.L[2], iz);
+    const double d2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const bool in = base + lane < total && g.rCutSq > d2 &&
+                    !(int(j0) >= skipSt && int(j0) < skipEnd);
+    if (in && d2 < g.rCutLowSq && ((newMask >> v) & 1)) sum.ov = 1.0;
+    const int code = int(j0) * 8 + v;
+    j0 = j1;
+    v0 = v1;
+    x0 = x1;
+    y0 = y1;
+    z0 = z1;
+    j1 = j2;
+    v1 = v2;
+    const uint64_t m = __ballot(in);
+    if (in) {
+      const int at_ = cnt + __popcll(m & ((uint64_t(1) << lane) - 1));
+      wq.d2[at_] = d2;
+      wq.code[at_] = code;
+    }
+    cnt += __popcll(m);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const bool done = base + step >= total;
+    while (cnt >= kWave || (done && cnt > 0)) {  // the queue's last 64, or what is left
+      const int n = min(cnt, kWave);
+      cnt -= n;
+      if (lane < n) {
+        const int code = wq.code[cnt + lane], j = code >> 3, w = code & 7;
+        const double qj = At(q, j);
+        const int idx = c.ct[p0 + w] + At(type, j) * ntypes;
+        PairTermsDev<P>(g, Fresh(coefs), wq.d2[cnt + lane], qj * c.cq[p0 + w] * kQQFact,
+                        At(sigSq, idx), At(epsCn, idx), At(nHalf, idx),
+                        ((newMask >> w) & 1) ? 1.0 : -1.0, sum.lj, sum.real);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    if (done) break;
+  }
+  return sum;
+}
 
 // ParticleInter (src/CalculateEnergy.cpp:727-785) for the stage's nc
 // (position, atom) combinations: one wave per combination, the lanes over
 // the atoms of the 27 cells around the position (or, with the cell walk
 // off, over the live list), then the wave's sum.
 template <int P>
-NOINLINE __device__ void ComboEnergies(const DevBox &B, Ctl &c) {
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+__device__ __forceinline__ void ComboEnergies(const DevBox &B, Ctl &c) {
+  const int lane = threadIdx.x % kWave, wave = Uni(int(threadIdx.x / kWave));
   // live atoms only; the atoms of molecule `skip` (c.st, c.len) are left out
-  const int nc = c.nc, nLive = c.nLive, ntypes = B.ntypes;
+  const int nc = Uni(c.nc);
   const int skipSt = c.skip >= 0 ? c.st : 0, skipEnd = c.skip >= 0 ? c.st + c.len : 0;
-  const GI *live = G(B.live);
-  const BoxGeom g = B.g;
-  const GD *x = G(B.x), *y = G(B.y), *z = G(B.z), *q = G(B.q);
-  const GI *type = G(B.type);
-  const GD *sigSq = G(B.sigSq), *epsCn = G(B.epsCn), *nHalf = G(B.nHalf);
   for (int ci = wave; ci < nc; ci += kDevWaves) {
-    const double px = c.cx[ci], py = c.cy[ci], pz = c.cz[ci], charge = c.cq[ci];
-    const int atype = c.ct[ci];
-    double lj = 0.0, real = 0.0, ov = 0.0;
-    WaveQ &wq = sQ[wave];
-    int cnt = 0;
-    const bool walk = UseCells(B, c);
-    const int total = walk ? WaveCells(B, px, py, pz, lane, sWCell[wave], sWStart[wave]) : nLive;
-    for (int base = 0; base < total; base += kWave) {
-      const int li = base + lane;
-      bool in = false;
-      double d2 = 0.0, qiqj = 0.0;
-      int code = 0;
-      if (li < total) {
-        const int j = walk ? CellAtom(B, sWCell[wave], sWStart[wave], li) : live[li];
-        if (!(j >= skipSt && j < skipEnd)) {
-          d2 = DistSq(g, px, py, pz, x[j], y[j], z[j]);
-          in = g.rCutSq > d2;
-          if (in && d2 < g.rCutLowSq) ov = 1.0;
-          qiqj = q[j] * charge * kQQFact;
-          code = (atype + type[j] * ntypes) * 2 + 1;
-        }
-      }
-      PushQ<P>(g, wq, cnt, lane, in, d2, qiqj, code, sigSq, epsCn, nHalf, lj, real);
-    }
-    DrainQ<P>(g, wq, cnt, lane, sigSq, epsCn, nHalf, lj, real);
-    __builtin_amdgcn_wave_barrier();
-    lj = WaveSum(lj);
-    real = WaveSum(real);
-    ov = WaveSum(ov);
-    if (lane == 0) {
-      c.cE[ci] = lj;
-      c.cR[ci] = real;
-      c.cO[ci] = ov;
+    if (UseCells(B, c)) WaveCells(B, c.cx[ci], c.cy[ci], c.cz[ci], lane, sWCell[wave]);
+    PairSums t = PairItems<P>(B, c, ci, 1, 0, 1, wave, skipSt, skipEnd, 1);
+    t.lj = WaveSumDpp(t.lj);
+    t.real = WaveSumDpp(t.real);
+    const bool any = __any(t.ov > 0.0);
+    if (lane == kWave - 1) {
+      c.cE[ci] = t.lj;
+      c.cR[ci] = t.real;
+      c.cO[ci] = any ? 1.0 : 0.0;
     }
   }
   __syncthreads();
 }
 
 // Waves of a translate/rotate trial that take the pair terms while the rest
-// take the k-vectors, in proportion to 2 N_live distance tests per atom
-// against kRecipWeight K phase products per atom (at least two waves each).
-constexpr double kRecipWeight = 1.0;
-__device__ __forceinline__ int PairWaves(int nLive, int K) {
-  const double wp = 2.0 * double(nLive), wr = kRecipWeight * double(K);
+// take the k-vectors, in proportion to the distance tests per atom of the
+// molecule against kRecipWeight K phase products (at least two waves each).
+// Measured with 0.5, 0.7, 1, 1.5 (40 A, 1000 molecules, microseconds a move in
+// FP64): 29.1, 28.7, 29.5, 29.8.
+constexpr double kRecipWeight = 0.7;
+__device__ __forceinline__ int PairWaves(int items, int len, int K) {
+  const double wp = 2.0 * double((items + len - 1) / len), wr = kRecipWeight * double(K);
   const int pw = int(double(kDevWaves) * wp / (wp + wr) + 0.5);
   return pw < 2 ? 2 : (pw > kDevWaves - 2 ? kDevWaves - 2 : pw);
 }
@@ -706,193 +985,69 @@ __device__ __forceinline__ int PairWaves(int nLive, int K) {
 // pair waves and the k-vector waves running side by side.
 template <int P>
 NOINLINE __device__ void MolTrialEnergies(const DevBox &B, DevState &s, Ctl &c, PhaseTab &tab) {
-  double lj = 0.0, real = 0.0, ov = 0.0, e = 0.0;
-  const int st = c.st, len = c.len, ntypes = B.ntypes;
-  const BoxGeom g = B.g;
-  const bool doRecip = c.doRecip;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  // cell walk: wave sp takes position sp (atom sp >> 1; old when even, new
-  // when odd) and finds the atoms of the 27 cells around it
-  __shared__ int sPosTot[kDevPos];
-  const bool walk = UseCells(B, c);
-  if (walk && wave < 2 * len) {
+  double e = 0.0;
+  PairSums t{0.0, 0.0, 0.0};
+  const int st = Uni(c.st), len = Uni(c.len);
+  const bool doRecip = Uni(c.doRecip);
+  const int lane = threadIdx.x % kWave, wave = Uni(int(threadIdx.x / kWave));
+  // position v of the pair terms' list is atom v >> 1, old when even and new
+  // when odd; with the cell walk wave v finds the atoms of the 27 cells around
+  // it, while the last waves make the phases
+  const bool walk = Uni(int(UseCells(B, c))) != 0;
+  if (wave < 2 * len) {
     const int p = wave >> 1;
     const bool isNew = wave & 1;
-    const int tot = WaveCells(B, isNew ? c.nx[p] : c.ox[p], isNew ? c.ny[p] : c.oy[p],
-                              isNew ? c.nz[p] : c.oz[p], lane, sWCell[wave], sWStart[wave]);
-    if (lane == 0) sPosTot[wave] = tot;
-  }
-  if (doRecip) {  // new positions are table rows [0, len), old ones [kDevKindAtoms, +len)
-    __shared__ double tpx[kDevPos], tpy[kDevPos], tpz[kDevPos];
-    if (threadIdx.x < kDevKindAtoms) {
-      const int p = threadIdx.x;
-      tpx[p] = c.nx[p];
-      tpy[p] = c.ny[p];
-      tpz[p] = c.nz[p];
-      tpx[kDevKindAtoms + p] = c.ox[p];
-      tpy[kDevKindAtoms + p] = c.oy[p];
-      tpz[kDevKindAtoms + p] = c.oz[p];
+    const double px = isNew ? c.nx[p] : c.ox[p], py = isNew ? c.ny[p] : c.oy[p],
+                 pz = isNew ? c.nz[p] : c.oz[p];
+    if (lane == 0) {
+      c.cx[wave] = px;
+      c.cy[wave] = py;
+      c.cz[wave] = pz;
+      c.cq[wave] = c.mq[p];
+      c.ct[wave] = c.mt_[p];
     }
-    __syncthreads();
-    BuildPhases<P>(B, tpx, tpy, tpz, kDevPos, tab);  // ends with a barrier
-  } else if (walk) {
-    __syncthreads();
+    if (walk) WaveCells(B, px, py, pz, lane, sWCell[wave]);
   }
-  // (position, neighbour atom) items of the cell walk: one distance test
-  // each, weighted twice a live-list test in the wave split
-  int items = 0;
-  if (walk)
-    for (int sp = 0; sp < 2 * len; ++sp) items += sPosTot[sp];
+  if (doRecip)  // new positions are table rows [0, len), old ones [kDevKindAtoms, +len)
+    BuildPhases<P, true>(B, c, len, tab);
+  __syncthreads();
+  // (position, neighbour atom) items, one distance test each
+  int items = 2 * len * c.nLive;
+  if (walk) {
+    items = 0;
+    for (int v = 0; v < 2 * len; ++v) items += sWCell[v].end[26];
+  }
   // the same split in every member of a team (its pair sums, computed by
   // each member in full, must agree to the last bit)
-  const int nPair = walk ? (items + len - 1) / len : c.nLive;
-  const int pw = doRecip ? PairWaves(nPair, (B.K + B.team - 1) / B.team) : kDevWaves;
-  if (wave < pw && walk) {
-    const GD *x = G(B.x), *y = G(B.y), *z = G(B.z), *q = G(B.q);
-    const GI *type = G(B.type);
-    const GD *sigSq = G(B.sigSq), *epsCn = G(B.epsCn), *nHalf = G(B.nHalf);
-    WaveQ &wq = sQ[wave];
-    int cnt = 0;
-    for (int base = wave * kWave; base < items; base += pw * kWave) {
-      const int it = base + lane;
-      bool in = false;
-      double d2 = 0.0, qq = 0.0;
-      int code = 0;
-      if (it < items) {
-        int sp = 0, first = 0;
-        while (it >= first + sPosTot[sp]) first += sPosTot[sp++];
-        const int j = CellAtom(B, sWCell[sp], sWStart[sp], it - first);
-        if (!(j >= st && j < st + len)) {
-          const int p = sp >> 1;
-          const bool isNew = sp & 1;
-          const double xj = x[j], yj = y[j], zj = z[j];
-          d2 = isNew ? DistSq(g, c.nx[p], c.ny[p], c.nz[p], xj, yj, zj)
-                     : DistSq(g, c.ox[p], c.oy[p], c.oz[p], xj, yj, zj);
-          in = g.rCutSq > d2;
-          if (isNew && in && d2 < g.rCutLowSq) ov = 1.0;
-          qq = c.mq[p] * q[j] * kQQFact;
-          code = (c.mt_[p] + type[j] * ntypes) * 2 + (isNew ? 1 : 0);
-        }
-      }
-      PushQ<P>(g, wq, cnt, lane, in, d2, qq, code, sigSq, epsCn, nHalf, lj, real);
-    }
-    DrainQ<P>(g, wq, cnt, lane, sigSq, epsCn, nHalf, lj, real);
-    __builtin_amdgcn_wave_barrier();
-  } else if (wave < pw) {
-    // (atom p, old) then (atom p, new) for each p, the molecule's data read
-    // from LDS; in-cutoff pairs go through the wave's queue
-    const GD *x = G(B.x), *y = G(B.y), *z = G(B.z), *q = G(B.q);
-    const GI *type = G(B.type);
-    const GD *sigSq = G(B.sigSq), *epsCn = G(B.epsCn), *nHalf = G(B.nHalf);
-    WaveQ &wq = sQ[wave];
-    int cnt = 0;
-    const int nLive = c.nLive;
-    const GI *live = G(B.live);
-    for (int base = wave * kWave; base < nLive; base += pw * kWave) {
-      const int li = base + lane;
-      const int j = li < nLive ? live[li] : 0;
-      const bool valid = li < nLive && !(j >= st && j < st + len);
-      double xj = 0.0, yj = 0.0, zj = 0.0, qj = 0.0;
-      int tj = 0;
-      if (valid) {
-        xj = x[j];
-        yj = y[j];
-        zj = z[j];
-        qj = q[j];
-        tj = type[j];
-      }
-      for (int sp = 0; sp < 2 * len; ++sp) {
-        const int p = sp >> 1;
-        const bool isNew = sp & 1;
-        double d2 = 0.0;
-        bool in = false;
-        if (valid) {
-          d2 = isNew ? DistSq(g, c.nx[p], c.ny[p], c.nz[p], xj, yj, zj)
-                     : DistSq(g, c.ox[p], c.oy[p], c.oz[p], xj, yj, zj);
-          in = g.rCutSq > d2;
-          if (isNew && in && d2 < g.rCutLowSq) ov = 1.0;
-        }
-        PushQ<P>(g, wq, cnt, lane, in, d2, c.mq[p] * qj * kQQFact,
-                 (c.mt_[p] + tj * ntypes) * 2 + (isNew ? 1 : 0), sigSq, epsCn, nHalf, lj, real);
-      }
-    }
-    DrainQ<P>(g, wq, cnt, lane, sigSq, epsCn, nHalf, lj, real);
-    __builtin_amdgcn_wave_barrier();
+  const int pw = doRecip ? PairWaves(Uni(items), len, (B.K + B.team - 1) / B.team) : kDevWaves;
+  if (wave < pw) {
+    t = PairItems<P>(B, c, 0, 2 * len, wave, pw, 0, st, st + len, 0x2a);
   } else {
     // every k-vector's new structure factor and energy term, beside the pairs
-    const GD *pref = G(B.pref);
-    const GD *sumR = G(B.sumR), *sumI = G(B.sumI);
-    const GI *kpack = G(B.kpack);
-    GDW *newR = GW(B.newR), *newI = GW(B.newI);
-    const int r0 = pw * kWave, rn = kDevThreads - r0;
-    for (int k = B.k0 + int(threadIdx.x) - r0; k < B.k1; k += rn) {
-      double sRN = 0.0, sIN = 0.0, sRO = 0.0, sIO = 0.0;
-      const int code = kpack[k];
-      const int ix = code & 0xff, iy = ((code >> 8) & 0xff) - 128, iz = ((code >> 16) & 0xff) - 128;
-#pragma unroll 1
-      for (int p = 0; p < len; ++p) {
-        const double qp = c.mq[p];
-        if (fabs(qp) < 0.000000001) continue;
-        const double2 en = Phase<P>(tab, p, ix, iy, iz);
-        const double2 eo = Phase<P>(tab, kDevKindAtoms + p, ix, iy, iz);
-        sRN += qp * en.x;
-        sIN += qp * en.y;
-        sRO += qp * eo.x;
-        sIO += qp * eo.y;
-      }
-      const double R = sumR[k] + (sRN - sRO);
-      const double I = sumI[k] + (sIN - sIO);
-      newR[k] = R;
-      newI[k] = I;
-      e += (R * R + I * I) * pref[k];
-    }
+    e = RecipTerms<P, true>(B, c, tab, pw * kWave, kDevThreads - pw * kWave, 1.0);
   }
-  BlockSum4(c, lj, real, e, ov);
+  BlockSum4(c, t.lj, t.real, e, t.ov);
   TeamExchange(B, s, c, 2);  // the members' k-vector ranges
 }
 
 // Ewald::SwapDestRecip / SwapSourceRecip (Ewald.cpp:478-531,657-710).
 template <int P>
 NOINLINE __device__ void SwapRecipEnergy(const DevBox &B, DevState &s, Ctl &c, PhaseTab &tab) {
-  double e = 0.0;
-  const int len = c.len, sign = c.sign;
-  const GD *pref = G(B.pref);
-  const GD *sumR = G(B.sumR), *sumI = G(B.sumI);
-  const GI *kpack = G(B.kpack);
-  GDW *newR = GW(B.newR), *newI = GW(B.newI);
-  BuildPhases<P>(B, c.nx, c.ny, c.nz, kDevKindAtoms, tab);
-  for (int k = B.k0 + int(threadIdx.x); k < B.k1; k += kDevThreads) {
-    double sR = 0.0, sI = 0.0;
-    const int code = kpack[k];
-    const int ix = code & 0xff, iy = ((code >> 8) & 0xff) - 128, iz = ((code >> 16) & 0xff) - 128;
-#pragma unroll 1
-    for (int p = 0; p < len; ++p) {
-      const double qp = c.mq[p];
-      if (fabs(qp) < 0.000000001) continue;
-      const double2 e1 = Phase<P>(tab, p, ix, iy, iz);
-      sR += qp * e1.x;
-      sI += qp * e1.y;
-    }
-    const double R = (sign > 0) ? sumR[k] + sR : sumR[k] - sR;
-    const double I = (sign > 0) ? sumI[k] + sI : sumI[k] - sI;
-    newR[k] = R;
-    newI[k] = I;
-    e += (R * R + I * I) * pref[k];
-  }
+  BuildPhases<P, false>(B, c, c.len, tab);
+  __syncthreads();
+  const double e =
+      RecipTerms<P, false>(B, c, tab, 0, kDevThreads, Uni(c.sign) > 0 ? 1.0 : -1.0);
   BlockSum4(c, e, 0.0, 0.0, 0.0);
   TeamExchange(B, s, c, 0);
 }
 
 // An accepted trial's structure factors become the box's (thread 0): the
-// trial phases wrote every k of newR/newI, so the two arrays trade places
+// trial phases wrote every pair of kNew, so the two arrays trade places
 // instead of K values being copied.
 __device__ void SwapRecip(DevBox &B) {
-  double *t = B.sumR;
-  B.sumR = B.newR;
-  B.newR = t;
-  t = B.sumI;
-  B.sumI = B.newI;
-  B.newI = t;
+  double *t = B.kCur;
+  B.kCur = B.kNew;
+  B.kNew = t;
 }
 
 // ------------------------------------------------- thread-0 serial pieces --
@@ -1015,27 +1170,30 @@ NOINLINE __device__ void StageWeights(const DevBox &B, Ctl &c, int n, bool hedro
   __syncthreads();
 }
 
+// By wave 0: the winner and the stage's weight.
 NOINLINE __device__ void SingleFinish(const DevBox &B, DevState &s, Ctl &c, DTrial &t, int atom,
                                       bool isNew) {
-  const int n = B.cbmcFirst;
-  double stepWeight = 0.0;
-  for (int i = 0; i < n; ++i) stepWeight += c.w[i];
-  int win = 0;
-  if (isNew) {
-    win = PickWeightedD(s, c.w, n, stepWeight);
+  const int n = Uni(B.cbmcFirst), lane = threadIdx.x;
+  const double w = lane < n ? c.w[lane] : 0.0;
+  double upto;
+  const double stepWeight = WeightSum(w, n, upto);
+  int win = isNew ? PickWeightedD(s, w, n, stepWeight, upto) : 0;
+  if (lane == 0) {
     if (win < 0) {
       s.status = kStWeights;
       c.abort = 1;
       win = 0;
     }
-    t.px[atom] = c.cx[win];
-    t.py[atom] = c.cy[win];
-    t.pz[atom] = c.cz[win];
+    if (isNew) {
+      t.px[atom] = c.cx[win];
+      t.py[atom] = c.cy[win];
+      t.pz[atom] = c.cz[win];
+    }
+    t.overlap = t.overlap || (c.cO[win] > 0.0);
+    t.weight *= stepWeight / n;
+    t.inter += 0.0 + c.cE[win];
+    t.real += 0.0 + c.cR[win];
   }
-  t.overlap = t.overlap || (c.cO[win] > 0.0);
-  t.weight *= stepWeight / n;
-  t.inter += 0.0 + c.cE[win];
-  t.real += 0.0 + c.cR[win];
 }
 
 // SinglePrep with the trial positions computed one per thread from words
@@ -1064,7 +1222,7 @@ NOINLINE __device__ void SinglePrepParallel(const DevBox &B, DevState &s, Ctl &c
 }
 
 template <int P>
-__device__ void SingleStage(const DevBox &B, DevState &s, Ctl &c, DTrial &t, int atom,
+NOINLINE __device__ void SingleStage(const DevBox &B, DevState &s, Ctl &c, DTrial &t, int atom,
                             bool isNew) {
   if (MtAvail(s) >= 3 * B.cbmcFirst)
     SinglePrepParallel(B, s, c, t, atom, isNew);
@@ -1073,7 +1231,7 @@ __device__ void SingleStage(const DevBox &B, DevState &s, Ctl &c, DTrial &t, int
   __syncthreads();
   ComboEnergies<P>(B, c);
   StageWeights(B, c, B.cbmcFirst, false);
-  if (threadIdx.x == 0) SingleFinish(B, s, c, t, atom, isNew);
+  if (threadIdx.x < kWave) SingleFinish(B, s, c, t, atom, isNew);
   __syncthreads();
 }
 
@@ -1081,10 +1239,8 @@ __device__ void SingleStage(const DevBox &B, DevState &s, Ctl &c, DTrial &t, int
 // from atom 0: the fixed angle's trials (all of weight 1, the winner still
 // drawn when growing), the seed atom, then cbmcNth spins of the rigid frame.
 NOINLINE __device__ void HedronTheta(const DevBox &B, DevState &s, Ctl &c, bool isNew) {
-  double tw = 0.0;
   const int n = isNew ? B.cbmcAng : B.cbmcAng - 1;
-  for (int i = 0; i < n; ++i) tw += 1.0;
-  c.thetaW = tw;
+  c.thetaW = n > 0 ? double(n) : 0.0;
   if (isNew) (void)MtClosed(s);  // DCHedron::FreeAnglesNew's PickWeighted, equal weights
 }
 
@@ -1098,22 +1254,12 @@ NOINLINE __device__ void HedronDraw(const DevBox &B, DevState &s, Ctl &c, const 
   c.hc[1] = cy;
   c.hc[2] = cz;
   if (isNew) {
-    const double th = B.hedTh[kind];
-    const double sinTh = sin(th);
-    double pbx = B.hedB[kind], pby = B.hedB[kind], pbz = B.hedB[kind];
-    pbx *= sinTh * cos(0.0);
-    pby *= sinTh * sin(0.0);
-    pbz *= cos(th);
-    double ppx = B.hedP[kind], ppy = B.hedP[kind], ppz = B.hedP[kind];
-    ppx *= sin(0.0) * cos(0.0);
-    ppy *= sin(0.0) * sin(0.0);
-    ppz *= cos(0.0);
-    c.hb[0] = pbx;
-    c.hb[1] = pby;
-    c.hb[2] = pbz;
-    c.hp[0] = ppx;
-    c.hp[1] = ppy;
-    c.hp[2] = ppz;
+    // sin and cos of the polar angles 0 and theta, and of the azimuth 0
+    c.hb[0] = B.hedB[kind] * B.hedSin[kind];
+    c.hb[1] = 0.0;
+    c.hb[2] = B.hedB[kind] * B.hedCos[kind];
+    c.hp[0] = c.hp[1] = 0.0;
+    c.hp[2] = B.hedP[kind];
   } else {
     c.thetaW += exp(-1 * B.beta * (0.0 + 0.0));  // DCHedron::IncorporateOld
     c.hb[0] = Unwrap(t.px[2], cx, B.g.L[0], B.g.half[0]) + (-cx);
@@ -1176,31 +1322,34 @@ NOINLINE __device__ void HedronSpin(const DevBox &B, DevState &s, Ctl &c, bool i
   if (i == 0 && c.uPeek) MtSkip(s, 3 * (isNew ? n : n - 1));
 }
 
+// By wave 0, as SingleFinish.
 NOINLINE __device__ void HedronFinish(const DevBox &B, DevState &s, Ctl &c, DTrial &t,
                                       bool isNew) {
-  const int n = B.cbmcNth;
-  double stepWeight = 0.0;
-  for (int i = 0; i < n; ++i) stepWeight += c.w[i];
-  int win = 0;
-  if (isNew) {
-    win = PickWeightedD(s, c.w, n, stepWeight);
+  const int n = Uni(B.cbmcNth), lane = threadIdx.x;
+  const double w = lane < n ? c.w[lane] : 0.0;
+  double upto;
+  const double stepWeight = WeightSum(w, n, upto);
+  int win = isNew ? PickWeightedD(s, w, n, stepWeight, upto) : 0;
+  if (lane == 0) {
     if (win < 0) {
       s.status = kStWeights;
       c.abort = 1;
       win = 0;
     }
-    t.px[2] = c.cx[win];
-    t.py[2] = c.cy[win];
-    t.pz[2] = c.cz[win];
-    t.px[1] = c.cx[n + win];
-    t.py[1] = c.cy[n + win];
-    t.pz[1] = c.cz[n + win];
+    if (isNew) {
+      t.px[2] = c.cx[win];
+      t.py[2] = c.cy[win];
+      t.pz[2] = c.cz[win];
+      t.px[1] = c.cx[n + win];
+      t.py[1] = c.cy[n + win];
+      t.pz[1] = c.cz[n + win];
+    }
+    t.overlap = t.overlap || (c.cO[win] > 0.0 || c.cO[n + win] > 0.0);
+    t.inter += c.sI[win];
+    t.real += c.sR[win];
+    t.weight *= c.thetaW * 1.0;
+    t.weight *= stepWeight / n;
   }
-  t.overlap = t.overlap || (c.cO[win] > 0.0 || c.cO[n + win] > 0.0);
-  t.inter += c.sI[win];
-  t.real += c.sR[win];
-  t.weight *= c.thetaW * 1.0;
-  t.weight *= stepWeight / n;
 }
 
 template <int P>
@@ -1214,7 +1363,7 @@ __device__ void HedronStage(const DevBox &B, DevState &s, Ctl &c, DTrial &t, boo
   HedronSpin(B, s, c, isNew);
   ComboEnergies<P>(B, c);
   StageWeights(B, c, B.cbmcNth, true);
-  if (threadIdx.x == 0) HedronFinish(B, s, c, t, isNew);
+  if (threadIdx.x < kWave) HedronFinish(B, s, c, t, isNew);
   __syncthreads();
 }
 
@@ -1288,11 +1437,25 @@ NOINLINE __device__ void TransferPick(const DevBox &B, DevState &s, Ctl &c, int6
   c.nm.weight = c.om.weight = 1.0;
   c.nm.overlap = c.om.overlap = 0;
   c.nm.inter = c.nm.real = c.om.inter = c.om.real = 0.0;
-  for (int p = 0; p < kDevKindAtoms; ++p) {
-    c.nm.px[p] = c.nm.py[p] = c.nm.pz[p] = 0.0;
-    c.om.px[p] = p < c.len ? B.x[c.st + p] : 0.0;
-    c.om.py[p] = p < c.len ? B.y[c.st + p] : 0.0;
-    c.om.pz[p] = p < c.len ? B.z[c.st + p] : 0.0;
+  {  // all loads at once: they cost one latency
+    const GD *x = G(B.x), *y = G(B.y), *z = G(B.z);
+    const int st = c.st, len = c.len;
+    double v[kDevKindAtoms][3];
+#pragma unroll
+    for (int p = 0; p < kDevKindAtoms; ++p) {
+      const int a = st + (p < len ? p : 0);
+      v[p][0] = x[a];
+      v[p][1] = y[a];
+      v[p][2] = z[a];
+    }
+#pragma unroll
+    for (int p = 0; p < kDevKindAtoms; ++p) {
+      const bool in = p < len;
+      c.nm.px[p] = c.nm.py[p] = c.nm.pz[p] = 0.0;
+      c.om.px[p] = in ? v[p][0] : 0.0;
+      c.om.py[p] = in ? v[p][1] : 0.0;
+      c.om.pz[p] = in ? v[p][2] : 0.0;
+    }
   }
   if (c.len == 1)
     (void)MtBelow(s, 1);  // DCLinear::Build: forward or backward
@@ -1546,17 +1709,35 @@ NOINLINE __device__ void MolPick(const DevBox &B, DevState &s, Ctl &c, int64_t i
   c.st = B.molStart[m];
   c.len = B.molStart[m + 1] - c.st;
   const double *L = B.g.L, *H = B.g.half;
-  c.ncom[0] = B.com[m];
-  c.ncom[1] = B.com[B.nmols + m];
-  c.ncom[2] = B.com[2 * B.nmols + m];
-  for (int p = 0; p < kDevKindAtoms; ++p) {
-    const bool in = p < c.len;
-    c.ox[p] = in ? B.x[c.st + p] : 0.0;
-    c.oy[p] = in ? B.y[c.st + p] : 0.0;
-    c.oz[p] = in ? B.z[c.st + p] : 0.0;
-    c.mq[p] = in ? B.q[c.st + p] : 0.0;
-    c.mt_[p] = in ? B.type[c.st + p] : 0;
-    c.nx[p] = c.ny[p] = c.nz[p] = 0.0;
+  {  // all loads at once: they cost one latency
+    const GD *x = G(B.x), *y = G(B.y), *z = G(B.z), *q = G(B.q), *com = G(B.com);
+    const GI *type = G(B.type);
+    const int st = c.st, len = c.len, nm = B.nmols;
+    double v[kDevKindAtoms][4], w[3];
+    int t[kDevKindAtoms];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) w[d] = com[size_t(d) * nm + m];
+#pragma unroll
+    for (int p = 0; p < kDevKindAtoms; ++p) {
+      const int a = st + (p < len ? p : 0);
+      v[p][0] = x[a];
+      v[p][1] = y[a];
+      v[p][2] = z[a];
+      v[p][3] = q[a];
+      t[p] = type[a];
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) c.ncom[d] = w[d];
+#pragma unroll
+    for (int p = 0; p < kDevKindAtoms; ++p) {
+      const bool in = p < len;
+      c.ox[p] = in ? v[p][0] : 0.0;
+      c.oy[p] = in ? v[p][1] : 0.0;
+      c.oz[p] = in ? v[p][2] : 0.0;
+      c.mq[p] = in ? v[p][3] : 0.0;
+      c.mt_[p] = in ? t[p] : 0;
+      c.nx[p] = c.ny[p] = c.nz[p] = 0.0;
+    }
   }
   if (mv == kDisplace) {
     const double bb = s.scale[kDisplace][mk], b2 = 2.0 * bb;
@@ -1575,9 +1756,11 @@ NOINLINE __device__ void MolPick(const DevBox &B, DevState &s, Ctl &c, int64_t i
     const double bb = s.scale[kRotate][mk];
     const double theta = MtClosed(s) * (2.0 * bb) - bb;
     const double u = MtClosed(s) * (2.0 * 1.0) - 1.0;
-    const double phi = MtHalfOpen(s) * (2.0 * M_PI);
+    const double turns = MtHalfOpen(s);  // phi = 2 pi turns
     const double rr = sqrt(1.0 - u * u);
-    const DM3 R = AxisAngleD(theta, rr * cos(phi), rr * sin(phi), u);
+    double sphi, cphi;
+    sincospi(2.0 * turns, &sphi, &cphi);
+    const DM3 R = AxisAngleD(theta, rr * cphi, rr * sphi, u);
     const double cx = c.ncom[0], cy = c.ncom[1], cz = c.ncom[2];
     for (int p = 0; p < c.len; ++p) {
       const double vx = Unwrap(c.ox[p], cx, L[0], H[0]) + (-cx);
@@ -1672,7 +1855,6 @@ __global__ void __launch_bounds__(kDevThreads) DeviceMovesKernel(const DevBox *b
     uint32_t *dst = reinterpret_cast<uint32_t *>(&S);
     for (int w = threadIdx.x; w < int(sizeof(DevState) / 4); w += kDevThreads) dst[w] = src[w];
   }
-  if (threadIdx.x <= kErfcxDeg) sErfcx[threadIdx.x] = kErfcxPoly[threadIdx.x];
   if (threadIdx.x == 0) {
     c.nLive = B.nLive0;
     c.cellsOff = 0;
@@ -1683,6 +1865,7 @@ __global__ void __launch_bounds__(kDevThreads) DeviceMovesKernel(const DevBox *b
     c.xseq = 1;
   }
   __syncthreads();
+  GatherRecip(B);  // the first move's barriers order this and its reads
   while (true) {
     // keep the next block of the MT19937 stream ready (a move draws < 400 words)
     if (!S.nextReady && kMtN - S.mtIdx < 400) MtPrepareNext(S);
@@ -1707,7 +1890,7 @@ __global__ void __launch_bounds__(kDevThreads) DeviceMovesKernel(const DevBox *b
     S.sumN[1] += B.nkinds > 1 ? double(NumKindInBox(B, S, 1, 0)) : 0.0;
     S.samples++;
   }
-  if (threadIdx.x == 0) S.recipSwapped = B.sumR != boxes[blockIdx.x].sumR;
+  ScatterRecip(B);
   __syncthreads();
   if (B.rank == 0) {  // the members of a team hold the same state
     const uint32_t *src = reinterpret_cast<const uint32_t *>(&S);
@@ -1727,7 +1910,9 @@ struct DevDriver {
   int *molKind = nullptr, *molBox = nullptr, *live = nullptr, *livePos = nullptr;
   uint32_t *lookup = nullptr;
   double *com = nullptr;
-  int32_t *kpack = nullptr;     // k-vector index triples
+  int32_t *kcode = nullptr, *kfirst = nullptr, *ksecond = nullptr;  // k-vectors two by two
+  int npairs = 0;
+  double *kpref = nullptr, *kbuf = nullptr;  // their prefactors; a launch's structure factors
   int nmax[3] = {0, 0, 0};
   int32_t *trace = nullptr;     // [4][cap] ints then [3][cap] doubles
   int64_t traceCap = 0;
@@ -1746,7 +1931,7 @@ struct DevDriver {
 void DevFree(gomc_box *b) {
   DevDriver *d = b->dev;
   if (!d) return;
-  for (void *p : {(void *)d->state, (void *)d->kpack, (void *)d->molKind, (void *)d->molBox,
+  for (void *p : {(void *)d->state, (void *)d->kcode, (void *)d->kfirst, (void *)d->ksecond, (void *)d->kpref, (void *)d->kbuf, (void *)d->molKind, (void *)d->molBox,
                   (void *)d->live, (void *)d->livePos,
                   (void *)d->lookup, (void *)d->com, (void *)d->trace, (void *)d->list,
                   (void *)d->xchg, (void *)d->cCount, (void *)d->cSlots, (void *)d->aCell,
@@ -1807,10 +1992,39 @@ int DevEnsure(gomc_box *b, int64_t traceMoves) {
     }
     if (d->nmax[0] > kDevNMax || d->nmax[1] > kDevNMax || d->nmax[2] > kDevNMax)
       return Fail(b, GOMC_ERR_ARG, "device move loop: more than 40 k-vectors per axis");
-    HIP_TRY(b, hipMalloc(&d->kpack, sizeof(int32_t) * std::max<size_t>(1, packed.size())));
-    if (!packed.empty())
-      HIP_TRY(b, hipMemcpy(d->kpack, packed.data(), sizeof(int32_t) * packed.size(),
-                           hipMemcpyHostToDevice));
+    // each with its mirror in z, where the half space holds that too
+    std::vector<int32_t> code, first, second;
+    std::vector<double> kpref;
+    code.reserve(packed.size());
+    first.reserve(packed.size());
+    second.reserve(packed.size());
+    kpref.reserve(packed.size());
+    for (size_t k = 0; k < packed.size(); ++k) {
+      const int nz = ((packed[k] >> 16) & 0xff) - 128;
+      // the k-vectors of one (nx, ny) stand in rising nz
+      const int64_t m = int64_t(k) - 2 * nz;
+      const int other = m >= 0 && m < int64_t(packed.size()) &&
+                                packed[m] == ((packed[k] & 0xffff) | ((128 - nz) << 16))
+                            ? int(m)
+                            : int(k);
+      if (nz < 0 && other != int(k)) continue;  // listed with its mirror
+      code.push_back(packed[k] | (other == int(k) ? INT32_MIN : 0));
+      kpref.push_back(pref[k]);
+      first.push_back(int(k));
+      second.push_back(other);
+    }
+    d->npairs = int(code.size());
+    HIP_TRY(b, hipMalloc(&d->kbuf, sizeof(double) * std::max<size_t>(1, 8 * code.size())));
+    HIP_TRY(b, hipMalloc(&d->kpref, sizeof(double) * std::max<size_t>(1, kpref.size())));
+    if (!kpref.empty())
+      HIP_TRY(b, hipMemcpy(d->kpref, kpref.data(), sizeof(double) * kpref.size(), hipMemcpyHostToDevice));
+    for (auto [dst, src] : {std::pair<int32_t **, std::vector<int32_t> *>{&d->kcode, &code},
+                            {&d->kfirst, &first},
+                            {&d->ksecond, &second}}) {
+      HIP_TRY(b, hipMalloc(dst, sizeof(int32_t) * std::max<size_t>(1, src->size())));
+      if (!src->empty())
+        HIP_TRY(b, hipMemcpy(*dst, src->data(), sizeof(int32_t) * src->size(), hipMemcpyHostToDevice));
+    }
   }
   DevDriver *d = b->dev;
   const int team = DevTeamSize(b);
@@ -1859,7 +2073,8 @@ int DevUpload(gomc_box *b, int64_t step0, int64_t nsteps, int cycles, bool trace
     if (!b->hedron.empty()) {
       h.hedB[k] = b->hedron[k].bBonded;
       h.hedP[k] = b->hedron[k].bPrev;
-      h.hedTh[k] = b->hedron[k].theta;
+      h.hedSin[k] = std::sin(b->hedron[k].theta);
+      h.hedCos[k] = std::cos(b->hedron[k].theta);
     }
   }
   for (int i = 0; i < 13; ++i) h.moveW[i] = b->moveW[i];
@@ -1889,15 +2104,15 @@ int DevUpload(gomc_box *b, int64_t step0, int64_t nsteps, int cycles, bool trace
   h.sigSq = b->tSigSq;
   h.epsCn = b->tEpsCn;
   h.nHalf = b->tNHalf;
-  h.kx = b->kx;
-  h.ky = b->ky;
-  h.kz = b->kz;
-  h.pref = b->pref;
   h.sumR = b->sumRref;
   h.sumI = b->sumIref;
-  h.newR = b->sumRnew;
-  h.newI = b->sumInew;
-  h.kpack = d->kpack;
+  h.kpref = d->kpref;
+  h.npairs = d->npairs;
+  h.kCur = d->kbuf;
+  h.kNew = d->kbuf + 4 * size_t(d->npairs);
+  h.kcode = d->kcode;
+  h.kfirst = d->kfirst;
+  h.ksecond = d->ksecond;
   for (int a = 0; a < 3; ++a) h.nmax[a] = d->nmax[a];
   h.molStart = b->molStartDev;
   h.molKind = d->molKind;
@@ -1908,7 +2123,7 @@ int DevUpload(gomc_box *b, int64_t step0, int64_t nsteps, int cycles, bool trace
   h.team = d->team;
   h.rank = 0;
   h.k0 = 0;
-  h.k1 = b->ewald ? b->K : 0;
+  h.k1 = b->ewald ? d->npairs : 0;
   h.xchg = d->xchg;
   h.com = d->com;
   h.st = d->state;
@@ -2060,10 +2275,6 @@ int DevDownload(gomc_box *b) {
   HIP_TRY(b, hipMemcpyAsync(b->hy.data(), b->y, bytes, hipMemcpyDeviceToHost, b->stream));
   HIP_TRY(b, hipMemcpyAsync(b->hz.data(), b->z, bytes, hipMemcpyDeviceToHost, b->stream));
   HIP_TRY(b, hipStreamSynchronize(b->stream));
-  if (s.recipSwapped) {  // the box's structure factors ended in the other array
-    std::swap(b->sumRref, b->sumRnew);
-    std::swap(b->sumIref, b->sumInew);
-  }
   const int K = b->nkinds;
   b->mt.SetState(s.mt[s.mtCur], s.mtIdx);
   b->pot.inter = s.pot[0];
