@@ -502,6 +502,24 @@ int EnsurePartials(gomc_box *b, int nblocks) {
   return GOMC_OK;
 }
 
+// Host memory the device addresses, for what a call takes and returns besides
+// its few scalars (hostRes); at least n doubles.
+int EnsureStage(gomc_box *b, size_t n) {
+  if (n <= kStageBase && !b->stageCap) {  // the room behind hostRes
+    b->stage = b->hostRes + 16;
+    b->devStage = b->devRes + 16;
+    return GOMC_OK;
+  }
+  if (n <= b->stageCap) return GOMC_OK;
+  if (b->stageCap) (void)hipHostFree(b->stage);
+  b->stage = b->devStage = nullptr;
+  b->stageCap = 0;
+  HIP_TRY(b, hipHostMalloc(&b->stage, sizeof(double) * n, hipHostMallocMapped));
+  HIP_TRY(b, hipHostGetDevicePointer((void **)&b->devStage, b->stage, 0));
+  b->stageCap = n;
+  return GOMC_OK;
+}
+
 int Sync(gomc_box *b) {
   HIP_TRY(b, hipStreamSynchronize(b->stream));
   HIP_TRY(b, hipGetLastError());
@@ -880,7 +898,7 @@ static void FreeAll(gomc_box *b) {
   FreeMolCells(b->mc);
   MPFree(b);
   DevFree(b);
-  if (b->trialBuf) (void)hipFree(b->trialBuf);
+  if (b->stageCap) (void)hipHostFree(b->stage);
   if (b->virBuf) (void)hipFree(b->virBuf);
   if (b->sumPart) (void)hipFree(b->sumPart);
   b->sumPart = nullptr;
@@ -991,23 +1009,21 @@ int FlushPending(gomc_box *b) {
 // Energies of `n` trial positions of one atom against the live atoms
 // (CalculateEnergy::ParticleInter, src/CalculateEnergy.cpp:727-785), through
 // the trial cell table when 27 cells of it hold fewer slots than the box
-// has atoms; the trial staging buffer is the box's and grows only when `n`
-// does.
+// has atoms.
 int ParticleInterImpl(gomc_box *b, int atomType, double charge, int skipMol, int n,
                       const double *tx, const double *ty, const double *tz, double *en,
                       double *real, int32_t *overlap) {
-  if (n > b->trialCap) {
-    if (b->trialBuf) (void)hipFree(b->trialBuf);
-    b->trialBuf = nullptr;
-    b->trialCap = 0;
-    HIP_TRY(b, hipMalloc(&b->trialBuf, sizeof(double) * 6 * size_t(n)));
-    b->trialCap = n;
+  // positions and results through host memory the kernel addresses itself:
+  // copies of a few hundred bytes cost more than the kernel (16 trials of 1000
+  // methane / CO2 molecules: four copies took 22 of 59 us)
+  {
+    int rc = EnsureStage(b, 6 * size_t(n));
+    if (rc) return rc;
   }
-  double *buf = b->trialBuf;
-  const size_t nb = sizeof(double) * n;
-  HIP_TRY(b, hipMemcpyAsync(buf, tx, nb, hipMemcpyHostToDevice, b->stream));
-  HIP_TRY(b, hipMemcpyAsync(buf + n, ty, nb, hipMemcpyHostToDevice, b->stream));
-  HIP_TRY(b, hipMemcpyAsync(buf + 2 * n, tz, nb, hipMemcpyHostToDevice, b->stream));
+  std::copy(tx, tx + n, b->stage);
+  std::copy(ty, ty + n, b->stage + n);
+  std::copy(tz, tz + n, b->stage + 2 * size_t(n));
+  double *buf = b->devStage;
   ParticleArgs a;
   a.g = b->geom;
   a.x = b->x;
@@ -1053,10 +1069,9 @@ int ParticleInterImpl(gomc_box *b, int atomType, double charge, int skipMol, int
   else
     hipLaunchKernelGGL(ParticleInterKernel<0>, dim3(n), dim3(kBlock), 0, b->stream, a);
   HIP_TRY(b, hipGetLastError());
-  std::vector<double> host(3 * size_t(n));
-  HIP_TRY(b, hipMemcpyAsync(host.data(), buf + 3 * n, 3 * nb, hipMemcpyDeviceToHost, b->stream));
   int rc = Sync(b);
   if (rc) return rc;
+  const double *host = b->stage + 3 * size_t(n);
   for (int t = 0; t < n; ++t) {
     en[t] = host[t];
     real[t] = host[n + t];

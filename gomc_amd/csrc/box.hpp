@@ -126,6 +126,8 @@ __device__ inline bool FinishPartials(const Partial4 &mine, Partial4 *partials,
   return last;
 }
 
+constexpr size_t kStageBase = 1024;  // doubles of staging memory every box has
+
 // MultiParticle state (src/moves/MultiParticle.h:37-58 and the
 // MultiParticle members of src/MoveSettings.h): step sizes, interval
 // counters, and the device force sets [ref|trial].
@@ -140,7 +142,7 @@ struct MPState {
   double *aF[2][3] = {}, *aFR[2][3] = {};               // atom forces [set][xyz]
   double *mF[2][3] = {}, *mFR[2][3] = {}, *tq[2][3] = {};  // molecule terms
   double *tk[3] = {};                                   // t_k or r_k
-  int *inRange = nullptr, *fail = nullptr, *molStart = nullptr;
+  int *inRange = nullptr, *molStart = nullptr;
   double *wpart = nullptr;                              // per-block products
   unsigned *wcounter = nullptr;
 };
@@ -209,7 +211,7 @@ struct gomc_box {
   gomc::Partial4 *partials = nullptr;
   int maxPartials = 0;
   unsigned *counter = nullptr;
-  double *hostRes = nullptr, *devRes = nullptr;  // 16 doubles, host-mapped
+  double *hostRes = nullptr, *devRes = nullptr;  // 16 doubles (and kStageBase), host-mapped
   // a molecule whose accepted coordinates the next trial launch writes
   int pendingMol = -1;
   double pend[3][gomc::kMaxMolAtoms];
@@ -235,9 +237,12 @@ struct gomc_box {
   bool cached = false;
   double *cacheC = nullptr, *cacheS = nullptr, *stageC = nullptr, *stageS = nullptr;
   int stageMol = -1;
-  // staging for trial positions and their energies (ParticleInter)
-  double *trialBuf = nullptr;
-  int trialCap = 0;
+  // host memory the device addresses, for arrays a call takes or returns
+  // (trial positions and energies, forces, centres), one user at a time: room
+  // for kStageBase doubles lies behind hostRes, made with the box (an allocation
+  // costs about 60 us), more is allocated (stageCap)
+  double *stage = nullptr, *devStage = nullptr;
+  size_t stageCap = 0;
   // per-block partial sums of the virial kernels
   double *virBuf = nullptr;
   size_t virCap = 0;
@@ -301,6 +306,7 @@ int PairVirials(gomc_box *b, double *const com[3], const double **vpart, int *nb
 void FreeMolCells(MolCells &c);
 int EnsurePartials(gomc_box *b, int nblocks);
 int Sync(gomc_box *b);
+int EnsureStage(gomc_box *b, size_t n);
 int BuildCells(gomc_box *b);
 int FlushPending(gomc_box *b);
 // Trial cell table (box.hip).  Valid only after TrialCellsEnsure; any
@@ -317,9 +323,6 @@ int TrialCellsFlushEdits(gomc_box *b);
 int MPEnsure(gomc_box *b);
 void MPFree(gomc_box *b);
 int MPUploadCom(gomc_box *b);
-int MPPairForce(gomc_box *b, int set, double *lj, double *real);
-int MPRecipForce(gomc_box *b, int set);
-int MPMolTerms(gomc_box *b, int set, int comSet);
 int MPMove(gomc_box *b, uint64_t step, int &moveType, int &accepted, int &failed, double dE[3]);
 // GCMC pieces (gcmc.cpp / box.hip).
 int ParticleInterImpl(gomc_box *b, int atomType, double charge, int skipMol, int n,

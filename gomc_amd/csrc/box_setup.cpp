@@ -321,7 +321,7 @@ int gomc_box_create(const gomc_system_desc *d, int device, gomc_box **out) {
   ok &= hipMalloc(&b->atomCell, ni) == hipSuccess;
   ok &= hipMalloc(&b->nbr, sizeof(int) * b->ncell * 27) == hipSuccess;
   ok &= hipMalloc(&b->counter, sizeof(unsigned)) == hipSuccess;
-  ok &= hipHostMalloc(&b->hostRes, sizeof(double) * 16, hipHostMallocMapped) == hipSuccess;
+  ok &= hipHostMalloc(&b->hostRes, sizeof(double) * (16 + kStageBase), hipHostMallocMapped) == hipSuccess;
   if (!ok) return fail(GOMC_ERR_HIP, "device allocation failed");
   if (hipHostGetDevicePointer((void **)&b->devRes, b->hostRes, 0) != hipSuccess)
     return fail(GOMC_ERR_HIP, "mapped result pointer");

@@ -10,6 +10,7 @@
 // sum has a fixed order and a run is reproducible bit for bit.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "box.hpp"
 
@@ -148,7 +149,8 @@ struct TransformArgs {
   const int *molStart;
   const double *mF[3], *mFR[3], *tq[3];
   double *tk[3];
-  int *inRange, *fail;
+  int *inRange;
+  double *fail;  // host-mapped
 };
 
 // TransformMatrix::FromAxisAngle (src/TransformMatrix.h:186-214).
@@ -181,7 +183,7 @@ __global__ void __launch_bounds__(kBlock) TransformKernel(const TransformArgs a)
   a.inRange[m] = in ? 1 : 0;
   bool bad = !isfinite(sqrt(val[0] * val[0] + val[1] * val[1] + val[2] * val[2]));
   if (!a.rotate && (val[0] > a.g.half[0] || val[1] > a.g.half[1] || val[2] > a.g.half[2])) bad = true;
-  if (bad) atomicOr(a.fail, 1);
+  if (bad) *a.fail = 1.0;
 
   const int s = a.molStart[m], e = a.molStart[m + 1];
   const double c[3] = {a.cx[m], a.cy[m], a.cz[m]};
@@ -301,7 +303,7 @@ namespace gomc {
 
 void MPFree(gomc_box *b) {
   MPState &mp = b->mp;
-  std::vector<void *> ptrs = {mp.xn, mp.yn, mp.zn, mp.inRange, mp.fail, mp.wpart,
+  std::vector<void *> ptrs = {mp.xn, mp.yn, mp.zn, mp.inRange, mp.wpart,
                               mp.wcounter};
   for (int s = 0; s < 2; ++s)
     for (int d = 0; d < 3; ++d) {
@@ -338,8 +340,6 @@ int MPEnsure(gomc_box *b) {
     }
   for (int d = 0; d < 3; ++d) ok &= hipMalloc(&mp.tk[d], nm) == hipSuccess;
   ok &= hipMalloc(&mp.inRange, sizeof(int) * std::max(b->nmols, 1)) == hipSuccess;
-  ok &= hipMalloc(&mp.fail, sizeof(int)) == hipSuccess;
-
   ok &= hipMalloc(&mp.wpart, sizeof(double) * ((b->nmols + kBlock - 1) / kBlock + 1)) == hipSuccess;
   ok &= hipMalloc(&mp.wcounter, sizeof(unsigned)) == hipSuccess;
   if (!ok) {
@@ -352,33 +352,92 @@ int MPEnsure(gomc_box *b) {
   return GOMC_OK;
 }
 
-// The driver keeps the authoritative centres on the host; a MultiParticle
-// step starts from them.
-int MPUploadCom(gomc_box *b) {
-  const size_t bytes = sizeof(double) * b->nmols;
-  HIP_TRY(b, hipMemcpyAsync(b->mp.com[0][0], b->comx.data(), bytes, hipMemcpyHostToDevice, b->stream));
-  HIP_TRY(b, hipMemcpyAsync(b->mp.com[0][1], b->comy.data(), bytes, hipMemcpyHostToDevice, b->stream));
-  HIP_TRY(b, hipMemcpyAsync(b->mp.com[0][2], b->comz.data(), bytes, hipMemcpyHostToDevice, b->stream));
-  return Sync(b);
+constexpr int kFailSlot = 15;  // of hostRes: a transform failed
+
+// Arrays between the device and the box's staging memory, all of a call's in
+// one launch: a copy command an array costs about 10 us each way for pageable
+// memory, whatever its length (the 15 arrays and dozen waits of a force
+// evaluation took 340 of 453 us for 1000 waters).
+constexpr int kCopyMax = 6;
+struct CopyArgs {
+  const double *src[kCopyMax];
+  double *dst[kCopyMax];
+  int n[kCopyMax];
+};
+__global__ void __launch_bounds__(kBlock) CopyKernel(const CopyArgs a) {
+  const int v = blockIdx.y, n = a.n[v];
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+    a.dst[v][i] = a.src[v][i];
+}
+static hipError_t LaunchCopies(const CopyArgs &a, int count, hipStream_t s) {
+  int most = 1;
+  for (int v = 0; v < count; ++v) most = std::max(most, a.n[v]);
+  const int g = std::min((most + kBlock - 1) / kBlock, 256);
+  hipLaunchKernelGGL(CopyKernel, dim3(g, count), dim3(kBlock), 0, s, a);
+  return hipGetLastError();
 }
 
-// Pair forces of the current coordinates into force set `set`; energies out.
-int MPPairForce(gomc_box *b, int set, double *lj, double *real) {
-  int rc = PairForces(b, b->mp.aF[set]);
-  if (!rc) rc = Sync(b);
+// Device arrays to the host, one or two sets of three (a null destination is
+// passed over); ends with the call's wait.
+static int CopyOut(gomc_box *b, double *const *d0, double *const *s0, int n0,
+                   double *const *d1 = nullptr, double *const *s1 = nullptr, int n1 = 0) {
+  int rc = EnsureStage(b, 3 * (size_t(b->natoms) + 2 * size_t(b->nmols)));
   if (rc) return rc;
-  *lj = b->hostRes[0];
-  *real = b->hostRes[1];
+  CopyArgs a{};
+  double *to[kCopyMax], *at = b->devStage;
+  int count = 0;
+  auto add = [&](double *const *d, double *const *s, int n) {
+    for (int k = 0; k < 3; ++k)
+      if (d[k]) {
+        to[count] = d[k];
+        a.src[count] = s[k];
+        a.dst[count] = at;
+        a.n[count++] = n;
+        at += n;
+      }
+  };
+  add(d0, s0, n0);
+  if (d1) add(d1, s1, n1);
+  if (count) HIP_TRY(b, LaunchCopies(a, count, b->stream));
+  rc = Sync(b);
+  if (rc) return rc;
+  for (int v = 0; v < count; ++v)
+    std::memcpy(to[v], b->stage + (a.dst[v] - b->devStage), sizeof(double) * a.n[v]);
   return GOMC_OK;
 }
 
-// Reciprocal forces of the current coordinates from the "new" sums.
-int MPRecipForce(gomc_box *b, int set) {
+// The driver keeps the authoritative centres on the host; a MultiParticle
+// step starts from them.  Not waited for: their place in the staging memory is
+// behind what CopyOut returns, and every call that uploads them ends with a
+// wait.
+int MPUploadCom(gomc_box *b) {
+  const size_t n = b->nmols, off = 3 * (size_t(b->natoms) + n);
+  int rc = EnsureStage(b, off + 3 * n);
+  if (rc) return rc;
+  CopyArgs a{};
+  const std::vector<double> *com[3] = {&b->comx, &b->comy, &b->comz};
+  for (int d = 0; d < 3; ++d) {
+    std::copy(com[d]->begin(), com[d]->begin() + n, b->stage + off + d * n);
+    a.src[d] = b->devStage + off + d * n;
+    a.dst[d] = b->mp.com[0][d];
+    a.n[d] = b->nmols;
+  }
+  HIP_TRY(b, LaunchCopies(a, 3, b->stream));
+  return GOMC_OK;
+}
+
+// Pair forces of the current coordinates into force set `set`; their energies
+// are hostRes[0] and [1] after the caller's wait.
+static int MPPairForce(gomc_box *b, int set) { return PairForces(b, b->mp.aF[set]); }
+
+// Reciprocal forces of the current coordinates from the "new" sums; not waited
+// for.
+static int MPRecipForce(gomc_box *b, int set) {
   MPState &mp = b->mp;
   if (!b->ewald || !b->recipReady) {
     for (int d = 0; d < 3; ++d)
       HIP_TRY(b, hipMemsetAsync(mp.aFR[set][d], 0, sizeof(double) * b->natoms, b->stream));
-    return Sync(b);
+    return GOMC_OK;
   }
   RecipForceArgs a;
   int rc = RecipForceParts(b, b->sumRnew, b->sumInew, &a.k);
@@ -397,9 +456,10 @@ int MPRecipForce(gomc_box *b, int set) {
   hipLaunchKernelGGL(RecipForceKernel, dim3((b->natoms + kWave - 1) / kWave), dim3(kWave), 0,
                      b->stream, a);
   HIP_TRY(b, hipGetLastError());
-  return Sync(b);
+  return GOMC_OK;
 }
 
+// Not waited for.
 static int MolTerms(gomc_box *b, int set, int comSet, int mode) {
   MPState &mp = b->mp;
   MolTermsArgs a;
@@ -423,10 +483,8 @@ static int MolTerms(gomc_box *b, int set, int comSet, int mode) {
   const int g = std::max(1, (b->nmols + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(MolTermsKernel, dim3(g), dim3(kBlock), 0, b->stream, a);
   HIP_TRY(b, hipGetLastError());
-  return Sync(b);
+  return GOMC_OK;
 }
-
-int MPMolTerms(gomc_box *b, int set, int comSet) { return MolTerms(b, set, comSet, 7); }
 
 // Transform -> CalcEn -> GetCoeff (MultiParticle.h:332-511) on the
 // reference force set; out = {inter, real, recip, w_ratio, fail}.  On
@@ -436,7 +494,7 @@ static int MPTrial(gomc_box *b, int rotate, uint64_t step, double max, double ou
   MPState &mp = b->mp;
   const int R = mp.ref, N = 1 - mp.ref;
   b->stageMol = -1;
-  HIP_TRY(b, hipMemsetAsync(mp.fail, 0, sizeof(int), b->stream));
+  b->hostRes[kFailSlot] = 0.0;  // nothing of this box's runs: every call ends with a wait
   TransformArgs t;
   t.g = b->geom;
   t.nmols = b->nmols;
@@ -465,14 +523,13 @@ static int MPTrial(gomc_box *b, int rotate, uint64_t step, double max, double ou
     t.tk[d] = mp.tk[d];
   }
   t.inRange = mp.inRange;
-  t.fail = mp.fail;
+  t.fail = b->devRes + kFailSlot;
   const int g = std::max(1, (b->nmols + kBlock - 1) / kBlock);
   hipLaunchKernelGGL(TransformKernel, dim3(g), dim3(kBlock), 0, b->stream, t);
   HIP_TRY(b, hipGetLastError());
-  int fail = 0;
-  HIP_TRY(b, hipMemcpyAsync(&fail, mp.fail, sizeof(int), hipMemcpyDeviceToHost, b->stream));
   int rc = Sync(b);
   if (rc) return rc;
+  const bool fail = b->hostRes[kFailSlot] != 0.0;
   out[0] = b->pot.inter;
   out[1] = b->pot.real;
   out[2] = b->pot.recip;
@@ -488,7 +545,7 @@ static int MPTrial(gomc_box *b, int rotate, uint64_t step, double max, double ou
     rc = RecipSums(b, &out[2]);
     if (rc) return rc;
   }
-  rc = MPPairForce(b, N, &out[0], &out[1]);
+  rc = MPPairForce(b, N);
   if (!rc) rc = MPRecipForce(b, N);
   if (!rc) rc = MolTerms(b, N, 0, 7);
   if (rc) return rc;
@@ -514,6 +571,8 @@ static int MPTrial(gomc_box *b, int rotate, uint64_t step, double max, double ou
   HIP_TRY(b, hipGetLastError());
   rc = Sync(b);
   if (rc) return rc;
+  out[0] = b->hostRes[0];
+  out[1] = b->hostRes[1];
   double w = b->hostRes[4];
   out[3] = std::isfinite(w) ? w : 0.0;
   return GOMC_OK;
@@ -530,14 +589,10 @@ static int MPAccept(gomc_box *b, bool result, bool evaluated, const double e[3])
     mp.ref = 1 - mp.ref;
     TrialCellsInvalidate(b);  // every molecule moved
     if (b->ewald) gomc_recip_accept(b);
-    const size_t na = sizeof(double) * b->natoms, nm = sizeof(double) * b->nmols;
-    HIP_TRY(b, hipMemcpyAsync(b->hx.data(), b->x, na, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(b, hipMemcpyAsync(b->hy.data(), b->y, na, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(b, hipMemcpyAsync(b->hz.data(), b->z, na, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(b, hipMemcpyAsync(b->comx.data(), mp.com[0][0], nm, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(b, hipMemcpyAsync(b->comy.data(), mp.com[0][1], nm, hipMemcpyDeviceToHost, b->stream));
-    HIP_TRY(b, hipMemcpyAsync(b->comz.data(), mp.com[0][2], nm, hipMemcpyDeviceToHost, b->stream));
-    int rc = Sync(b);
+    double *dx[3] = {b->hx.data(), b->hy.data(), b->hz.data()},
+           *dc[3] = {b->comx.data(), b->comy.data(), b->comz.data()},
+           *sx[3] = {b->x, b->y, b->z};
+    int rc = CopyOut(b, dx, sx, b->natoms, dc, mp.com[0], b->nmols);
     // every molecule moved: EwaldCached::BoxReciprocalSums refilled the cache
     if (!rc && b->cached) rc = CacheBuild(b);
     return rc;
@@ -557,8 +612,7 @@ static int MPPrepForces(gomc_box *b) {
   int rc = GOMC_OK;
   if (b->ewald) rc = gomc_recip_copy_ref_to_new(b);
   if (!rc) rc = MPRecipForce(b, R);
-  double lj = 0, real = 0;
-  if (!rc) rc = MPPairForce(b, R, &lj, &real);
+  if (!rc) rc = MPPairForce(b, R);
   if (!rc) rc = MolTerms(b, R, 0, 7);
   if (!rc) b->pot.Total();
   return rc;
@@ -612,25 +666,21 @@ int MPMove(gomc_box *b, uint64_t step, int &moveType, int &accepted, int &failed
 // ====================================================================== C ABI
 extern "C" {
 
-static int CopyOut(gomc_box *b, double *const *dst, double *const *src, int n) {
-  for (int d = 0; d < 3; ++d)
-    if (dst[d]) HIP_TRY(b, hipMemcpyAsync(dst[d], src[d], sizeof(double) * n, hipMemcpyDeviceToHost, b->stream));
-  return Sync(b);
-}
-
 int gomc_box_force(gomc_box *b, double *lj, double *real, double *afx, double *afy, double *afz,
                    double *mfx, double *mfy, double *mfz) {
   if (!b || !lj || !real) return GOMC_ERR_ARG;
   (void)hipSetDevice(b->device);
   int rc = MPEnsure(b);
   if (!rc) rc = FlushPending(b);
-  if (!rc) rc = MPPairForce(b, b->mp.ref, lj, real);
+  if (!rc) rc = MPPairForce(b, b->mp.ref);
   if (!rc) rc = MolTerms(b, b->mp.ref, 0, 1);
   if (rc) return rc;
   double *da[3] = {afx, afy, afz}, *dm[3] = {mfx, mfy, mfz};
-  rc = CopyOut(b, da, b->mp.aF[b->mp.ref], b->natoms);
-  if (!rc) rc = CopyOut(b, dm, b->mp.mF[b->mp.ref], b->nmols);
-  return rc;
+  rc = CopyOut(b, da, b->mp.aF[b->mp.ref], b->natoms, dm, b->mp.mF[b->mp.ref], b->nmols);
+  if (rc) return rc;
+  *lj = b->hostRes[0];
+  *real = b->hostRes[1];
+  return GOMC_OK;
 }
 
 int gomc_box_force_recip(gomc_box *b, double *afx, double *afy, double *afz, double *mfx,
@@ -643,9 +693,7 @@ int gomc_box_force_recip(gomc_box *b, double *afx, double *afy, double *afz, dou
   if (!rc) rc = MolTerms(b, b->mp.ref, 0, 2);
   if (rc) return rc;
   double *da[3] = {afx, afy, afz}, *dm[3] = {mfx, mfy, mfz};
-  rc = CopyOut(b, da, b->mp.aFR[b->mp.ref], b->natoms);
-  if (!rc) rc = CopyOut(b, dm, b->mp.mFR[b->mp.ref], b->nmols);
-  return rc;
+  return CopyOut(b, da, b->mp.aFR[b->mp.ref], b->natoms, dm, b->mp.mFR[b->mp.ref], b->nmols);
 }
 
 int gomc_torque(gomc_box *b, double *tx, double *ty, double *tz) {
