@@ -72,130 +72,120 @@ struct TrialArgs {
 };
 static_assert(sizeof(TrialArgs) <= 4096, "trial arguments must fit the kernel argument buffer");
 
-// Atom j at (xj, yj, zj) against the molecule's old positions p with mask
-// bit p set (their energies subtracted) and new positions with bit
-// kNewBits + p set (added), p ascending, old before new
-// (CalculateEnergy.cpp:593-679).
+// Atom j at (xj, yj, zj) against atom p of the molecule: its old position (the
+// energy subtracted) where bit p of the mask is set, its new one (added) where
+// bit kNewBits + p is (CalculateEnergy.cpp:593-679).
 template <int P>
 __device__ __forceinline__ void TrialAtom(const TrialArgs &a, int j, double xj, double yj,
-                                          double zj, uint32_t mask, double &lj, double &real,
+                                          double zj, int p, uint32_t mask, double &lj, double &real,
                                           double &ov) {
-  const double qj = a.q[j];
-  const int tj = a.type[j];
-  for (int p = 0; p < a.mlen; ++p) {
-    const int idx = a.mtype[p] + tj * a.ntypes;
-    const double qiqj = a.mq[p] * qj * kQQFact;
-    if (mask >> p & 1u) {
-      const double d2 = DistSq(a.g, a.ox[p], a.oy[p], a.oz[p], xj, yj, zj);
-      if (a.g.rCutSq > d2) {
-        if (a.g.elect && qiqj != 0.0 && !(a.g.rCutCoulSq < d2)) real += -Coul<P>(a.g, d2, qiqj);
-        if (!(a.g.rCutLJSq < d2)) lj += -LJ<P>(d2, a.sigSq[idx], a.epsCn[idx], a.nHalf[idx]);
-      }
-    }
-    if (mask >> (kNewBits + p) & 1u) {
-      const double d2 = DistSq(a.g, a.nx[p], a.ny[p], a.nz[p], xj, yj, zj);
-      if (a.g.rCutSq > d2) {
-        if (d2 < a.g.rCutLowSq) ov = 1.0;
-        if (a.g.elect && qiqj != 0.0 && !(a.g.rCutCoulSq < d2)) real += Coul<P>(a.g, d2, qiqj);
-        if (!(a.g.rCutLJSq < d2)) lj += LJ<P>(d2, a.sigSq[idx], a.epsCn[idx], a.nHalf[idx]);
-      }
-    }
+  const Coefs coefs = GetCoefs();
+  const int idx = a.mtype[p] + a.type[j] * a.ntypes;
+  const double qiqj = a.mq[p] * a.q[j] * kQQFact;
+  const double sig = a.sigSq[idx], eps = a.epsCn[idx], nh = a.nHalf[idx];
+#pragma unroll 1
+  for (int side = 0; side < 2; ++side) {
+    if (!(mask >> (side ? kNewBits + p : p) & 1u)) continue;
+    const double d2 = side ? DistSq(a.g, a.nx[p], a.ny[p], a.nz[p], xj, yj, zj)
+                           : DistSq(a.g, a.ox[p], a.oy[p], a.oz[p], xj, yj, zj);
+    if (!(a.g.rCutSq > d2)) continue;
+    if (side && d2 < a.g.rCutLowSq) ov = 1.0;
+    PairTermsDev<P, true>(a.g, Fresh(coefs), d2, qiqj, sig, eps, nh, side ? 1.0 : -1.0, lj, real);
   }
 }
 
-// Blocks [0, nPairBlocks): the pair part.  Without a cell list one atom j
-// per thread against every old and new position; with one, one slot of a
-// listed cell per thread against the positions that cell neighbours
-// (CellList::EnumerateLocal, as MoleculeInter walks it), then one thread per
-// atom of the molecule accepted last (its cells are edited at the end of
-// this launch, so the walk skips it and takes it from the arguments).
-// Blocks after that: one k-vector per thread, the structure-factor delta and
-// the new per-k energy (Ewald.cpp:436-467).
+// Blocks [0, nPairBlocks): the pair part, block b for atom b % mlen of the
+// molecule and the b / mlen-th run of items.  Without a cell list an item is
+// one atom j; with one, one slot of a listed cell, against the positions that
+// cell neighbours (CellList::EnumerateLocal, as MoleculeInter walks it), then
+// one per atom of the molecule accepted last (its cells are edited at the end
+// of this launch, so the walk skips it and takes it from the arguments).
+// Blocks after that: two threads a k-vector, the even one for the new positions
+// and the odd one for the old, the structure-factor delta and the new per-k
+// energy (Ewald.cpp:436-467).
 // P = 1: pair terms and phases in FP32, sums in FP64 (the mixed mode).
+//
+// Bound by one thread's chain, not by the chip (a trial of 1000 waters is 100
+// blocks): an item a thread for one atom's two positions, one side's phases a
+// thread, pair terms without calls and one barrier a reduction took the kernel
+// from 14 us to 9.8 for 300 to 1000 waters; all of a molecule's positions
+// in one thread are six pair terms or sincos in a row.
+constexpr int kTrialK = kBlock / 2;  // k-vectors of a block
 template <int P>
 __global__ void __launch_bounds__(kBlock) TrialKernel(const TrialArgs a) {
-  __shared__ double red[kBlock / kWave];
-  Partial4 part{0, 0, 0, 0};
+  __shared__ double red[kBlock / kWave][4];
   const int tid = threadIdx.x;
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};  // lj, real, recip, overlap
   if (blockIdx.x == 0 && tid < a.clen) {
     a.wx[a.cstart + tid] = a.cx[tid];
     a.wy[a.cstart + tid] = a.cy[tid];
     a.wz[a.cstart + tid] = a.cz[tid];
   }
   if (int(blockIdx.x) < a.nPairBlocks) {
-    double lj = 0.0, real = 0.0, ov = 0.0;
-    const int t = blockIdx.x * kBlock + tid;
-    const uint32_t all = ~0u;
-    if (a.doPair && a.nlist == 0) {
-      const int j = t;
-      if (j < a.natoms && (j < a.mstart || j >= a.mstart + a.mlen) && a.mol[j] >= 0) {
-        const int cj = j - a.cstart;
-        if (cj >= 0 && cj < a.clen)
-          TrialAtom<P>(a, j, a.cx[cj], a.cy[cj], a.cz[cj], all, lj, real, ov);
-        else
-          TrialAtom<P>(a, j, a.x[j], a.y[j], a.z[j], all, lj, real, ov);
+    const int p = blockIdx.x % a.mlen, t = (blockIdx.x / a.mlen) * kBlock + tid;
+    // the item's atom (-1: none), whether its coordinates are the arguments'
+    int j = -1, cj = -1;
+    uint32_t mask = ~0u;
+    if (a.nlist == 0) {
+      if (t < a.natoms && a.mol[t] >= 0) {
+        j = t;
+        if (j >= a.cstart && j < a.cstart + a.clen) cj = j - a.cstart;
       }
-    } else if (a.doPair) {
+    } else {
       const int nslots = a.nlist * a.tcCap;
       if (t < nslots) {
         const int e = t / a.tcCap, s = t - e * a.tcCap;
         const int c = a.lcell[e];
-        if (s < a.tcCount[c]) {
-          const int j = a.tcSlots[c * a.tcCap + s];
-          const bool self = j >= a.mstart && j < a.mstart + a.mlen;
-          const bool pend = j >= a.cstart && j < a.cstart + a.clen;
-          if (!self && !pend) TrialAtom<P>(a, j, a.x[j], a.y[j], a.z[j], a.lmask[e], lj, real, ov);
-        }
+        mask = a.lmask[e];
+        if (s < a.tcCount[c]) j = a.tcSlots[c * a.tcCap + s];
+        if (j >= a.cstart && j < a.cstart + a.clen) j = -1;
       } else if (t - nslots < a.clen) {
-        const int cj = t - nslots, j = a.cstart + cj;
-        if ((j < a.mstart || j >= a.mstart + a.mlen) && a.mol[j] >= 0)
-          TrialAtom<P>(a, j, a.cx[cj], a.cy[cj], a.cz[cj], all, lj, real, ov);
+        cj = t - nslots;
+        j = a.cstart + cj;
+        if (a.mol[j] < 0) j = -1;
       }
     }
-    part.lj = BlockSum(lj, red);
-    part.real = BlockSum(real, red);
-    part.overlap = BlockSum(ov, red);
-  } else {
-    double e = 0.0;
-    const int k = (blockIdx.x - a.nPairBlocks) * kBlock + tid;
-    if (a.doRecip && k < a.K) {
-      const double kxk = a.kx[k], kyk = a.ky[k], kzk = a.kz[k];
-      double sRN = 0.0, sIN = 0.0, sRO = 0.0, sIO = 0.0;
-      if (a.oldC) {  // EwaldCached::MolReciprocal (EwaldCached.cpp:244-295)
-        for (int p = 0; p < a.mlen; ++p) {
-          if (fabs(a.mq[p]) < 0.000000001) continue;
-          double dNew = a.nx[p] * kxk + a.ny[p] * kyk + a.nz[p] * kzk;
-          double sn, cn;
-          Sincos<P>(dNew, &sn, &cn);
-          sRN += a.mq[p] * cn;
-          sIN += a.mq[p] * sn;
-        }
-        sRO = a.oldC[k];
-        sIO = a.oldS[k];
-        a.stC[k] = sRN;
-        a.stS[k] = sIN;
+    if (j >= 0 && (j < a.mstart || j >= a.mstart + a.mlen)) {
+      const double xj = cj >= 0 ? a.cx[cj] : a.x[j], yj = cj >= 0 ? a.cy[cj] : a.y[j],
+                   zj = cj >= 0 ? a.cz[cj] : a.z[j];
+      TrialAtom<P>(a, j, xj, yj, zj, p, mask, sum[0], sum[1], sum[3]);
+    }
+  } else if (a.doRecip) {
+    const int k = (blockIdx.x - a.nPairBlocks) * kTrialK + (tid >> 1);
+    const bool old = tid & 1, on = k < a.K;
+    double R = 0.0, I = 0.0;
+    if (on) {
+      if (old && a.oldC) {  // EwaldCached::MolReciprocal (EwaldCached.cpp:244-295)
+        R = a.oldC[k];
+        I = a.oldS[k];
       } else {
+        const double kxk = a.kx[k], kyk = a.ky[k], kzk = a.kz[k];
         for (int p = 0; p < a.mlen; ++p) {
           if (fabs(a.mq[p]) < 0.000000001) continue;
-          double dNew = a.nx[p] * kxk + a.ny[p] * kyk + a.nz[p] * kzk;
-          double dOld = a.ox[p] * kxk + a.oy[p] * kyk + a.oz[p] * kzk;
-          double sn, cn, so, co;
-          Sincos<P>(dNew, &sn, &cn);
-          Sincos<P>(dOld, &so, &co);
-          sRN += a.mq[p] * cn;
-          sIN += a.mq[p] * sn;
-          sRO += a.mq[p] * co;
-          sIO += a.mq[p] * so;
+          const double dot = old ? a.ox[p] * kxk + a.oy[p] * kyk + a.oz[p] * kzk
+                                 : a.nx[p] * kxk + a.ny[p] * kyk + a.nz[p] * kzk;
+          double sn, cs;
+          Sincos<P>(dot, &sn, &cs);
+          R += a.mq[p] * cs;
+          I += a.mq[p] * sn;
         }
       }
-      double R = a.sumRref[k] + (sRN - sRO);
-      double I = a.sumIref[k] + (sIN - sIO);
+    }
+    const double RO = __shfl_down(R, 1, kWave), IO = __shfl_down(I, 1, kWave);
+    if (on && !old) {
+      if (a.oldC) {
+        a.stC[k] = R;
+        a.stS[k] = I;
+      }
+      R = a.sumRref[k] + (R - RO);
+      I = a.sumIref[k] + (I - IO);
       a.sumRnew[k] = R;
       a.sumInew[k] = I;
-      e = (R * R + I * I) * a.pref[k];
+      sum[2] = (R * R + I * I) * a.pref[k];
     }
-    part.recip = BlockSum(e, red);
   }
+  BlockSum4(sum, red);
+  const Partial4 part{sum[0], sum[1], sum[2], sum[3]};
   // Every other block has published its partial, after its last read of
   // the cell table: the edits can no longer be seen by this launch.
   if (FinishPartials(part, a.partials, a.counter, a.result) && tid == 0)
@@ -439,32 +429,32 @@ struct ParticleArgs {
   int edge[3];
 };
 
+// Most threads have one slot or a few: a trial lasts as long as the chain from a
+// cell to its atoms' terms, five dependent loads, so one turn of 1024 threads
+// beats four of 256.  16 trials of 1000 methane / CO2 molecules: 13.9 -> 8.2 us.
+constexpr int kParticleBlock = 1024;
+
 template <int P>
 __device__ __forceinline__ void ParticleAtom(const ParticleArgs &a, int j, double px, double py,
                                              double pz, double &lj, double &real, double &ov) {
   const double d2 = DistSq(a.g, px, py, pz, a.x[j], a.y[j], a.z[j]);
   if (a.g.rCutSq > d2) {
     if (d2 < a.g.rCutLowSq) ov = 1.0;
-    if (!(a.g.rCutLJSq < d2)) {
-      const int idx = a.atype + a.type[j] * a.ntypes;
-      lj += LJ<P>(d2, a.sigSq[idx], a.epsCn[idx], a.nHalf[idx]);
-    }
-    if (a.g.elect) {
-      const double qiqj = a.q[j] * a.charge * kQQFact;
-      if (qiqj != 0.0 && !(a.g.rCutCoulSq < d2)) real += Coul<P>(a.g, d2, qiqj);
-    }
+    const int idx = a.atype + a.type[j] * a.ntypes;
+    PairTermsDev<P, true>(a.g, Fresh(GetCoefs()), d2, a.q[j] * a.charge * kQQFact, a.sigSq[idx],
+                    a.epsCn[idx], a.nHalf[idx], 1.0, lj, real);
   }
 }
 
 template <int P>
-__global__ void __launch_bounds__(kBlock) ParticleInterKernel(const ParticleArgs a) {
-  __shared__ double red[kBlock / kWave];
+__global__ void __launch_bounds__(kParticleBlock) ParticleInterKernel(const ParticleArgs a) {
+  __shared__ double red[kParticleBlock / kWave][4];
   const int t = blockIdx.x;
   const double px = a.tx[t], py = a.ty[t], pz = a.tz[t];
   double lj = 0.0, real = 0.0, ov = 0.0;
   if (a.tcCap > 0) {
     const int c0 = CellOf(px, py, pz, a.cs, a.edge);
-    for (int i = threadIdx.x; i < 27 * a.tcCap; i += kBlock) {
+    for (int i = threadIdx.x; i < 27 * a.tcCap; i += kParticleBlock) {
       const int n = i / a.tcCap, s = i - n * a.tcCap;
       const int c = a.nbr[c0 * 27 + n];
       if (s >= a.tcCount[c]) continue;
@@ -473,18 +463,17 @@ __global__ void __launch_bounds__(kBlock) ParticleInterKernel(const ParticleArgs
       ParticleAtom<P>(a, j, px, py, pz, lj, real, ov);
     }
   } else {
-    for (int j = threadIdx.x; j < a.natoms; j += kBlock) {
+    for (int j = threadIdx.x; j < a.natoms; j += kParticleBlock) {
       if (a.mol[j] == a.skipMol || a.mol[j] < 0) continue;
       ParticleAtom<P>(a, j, px, py, pz, lj, real, ov);
     }
   }
-  lj = BlockSum(lj, red);
-  real = BlockSum(real, red);
-  ov = BlockSum(ov, red);
+  double sum[4] = {lj, real, ov, 0.0};
+  BlockSum4(sum, red);
   if (threadIdx.x == 0) {
-    a.en[t] = lj;
-    a.real[t] = real;
-    a.overlap[t] = ov;
+    a.en[t] = sum[0];
+    a.real[t] = sum[1];
+    a.overlap[t] = sum[2];
   }
 }
 
@@ -682,7 +671,7 @@ int LaunchTrial(gomc_box *b, int m, const double *ox, const double *oy, const do
   }
   a.doPair = doPair;
   a.doRecip = doRecip && b->ewald;
-  const int nRecip = a.doRecip ? (b->K + kBlock - 1) / kBlock : 0;
+  const int nRecip = a.doRecip ? (b->K + kTrialK - 1) / kTrialK : 0;
   a.K = b->K;
   a.kx = b->kx;
   a.ky = b->ky;
@@ -764,8 +753,9 @@ int LaunchTrial(gomc_box *b, int m, const double *ox, const double *oy, const do
     }
   }
   if (doPair)
-    a.nPairBlocks = a.nlist > 0 ? int((size_t(a.nlist) * b->tcCap + a.clen + kBlock - 1) / kBlock)
-                                : (b->natoms + kBlock - 1) / kBlock;
+    a.nPairBlocks = len * (a.nlist > 0
+                               ? int((size_t(a.nlist) * b->tcCap + a.clen + kBlock - 1) / kBlock)
+                               : (b->natoms + kBlock - 1) / kBlock);
   else
     a.nPairBlocks = 0;
   int nblocks = a.nPairBlocks + nRecip;
@@ -1065,9 +1055,9 @@ int ParticleInterImpl(gomc_box *b, int atomType, double charge, int skipMol, int
     }
   }
   if (b->precision == 1)
-    hipLaunchKernelGGL(ParticleInterKernel<1>, dim3(n), dim3(kBlock), 0, b->stream, a);
+    hipLaunchKernelGGL(ParticleInterKernel<1>, dim3(n), dim3(kParticleBlock), 0, b->stream, a);
   else
-    hipLaunchKernelGGL(ParticleInterKernel<0>, dim3(n), dim3(kBlock), 0, b->stream, a);
+    hipLaunchKernelGGL(ParticleInterKernel<0>, dim3(n), dim3(kParticleBlock), 0, b->stream, a);
   HIP_TRY(b, hipGetLastError());
   int rc = Sync(b);
   if (rc) return rc;

@@ -92,7 +92,7 @@ struct Partial4 {
 __device__ inline bool FinishPartials(const Partial4 &mine, Partial4 *partials,
                                       unsigned *counter, double *result) {
   __shared__ bool last;
-  __shared__ double red[1024 / kWave];
+  __shared__ double red[1024 / kWave][4];
   if (threadIdx.x == 0) {
     partials[blockIdx.x] = mine;
     __threadfence();
@@ -102,23 +102,20 @@ __device__ inline bool FinishPartials(const Partial4 &mine, Partial4 *partials,
   __syncthreads();
   if (last) {
     __threadfence();
-    double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
     volatile Partial4 *vp = partials;
     for (unsigned i = threadIdx.x; i < gridDim.x; i += blockDim.x) {
-      s0 += vp[i].lj;
-      s1 += vp[i].real;
-      s2 += vp[i].recip;
-      s3 += vp[i].overlap;
+      s[0] += vp[i].lj;
+      s[1] += vp[i].real;
+      s[2] += vp[i].recip;
+      s[3] += vp[i].overlap;
     }
-    s0 = BlockSum(s0, red);
-    s1 = BlockSum(s1, red);
-    s2 = BlockSum(s2, red);
-    s3 = BlockSum(s3, red);
+    BlockSum4(s, red);
     if (threadIdx.x == 0) {
-      result[0] = s0;
-      result[1] = s1;
-      result[2] = s2;
-      result[3] = s3;
+      result[0] = s[0];
+      result[1] = s[1];
+      result[2] = s[2];
+      result[3] = s[3];
       *counter = 0u;
       __threadfence_system();
     }

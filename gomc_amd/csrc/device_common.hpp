@@ -65,26 +65,6 @@ __device__ __forceinline__ double DistSq(const BoxGeom &g, double ax, double ay,
   return dx * dx + dy * dy + dz * dz;
 }
 
-// FFParticle::CalcEn (src/FFParticle.cpp:295-325, lambda = 1):
-// eps_cn * ((sigma^2/r^2)^(n/2) - (sigma^2/r^2)^3).  For n = 12 the
-// repulsion is the attraction squared (pow(x, 6) within an ulp or two).
-__device__ __forceinline__ double LJEnergy(double distSq, double sigmaSq, double epsCn,
-                                           double nHalf) {
-  double rRat2 = sigmaSq / distSq;
-  double rRat4 = rRat2 * rRat2;
-  double attract = rRat4 * rRat2;
-  double repulse = (nHalf == 6.0) ? attract * attract : pow(rRat2, nHalf);
-  return epsCn * (repulse - attract);
-}
-
-// FFParticle::CalcCoulomb (src/FFParticle.cpp:387-399).
-__device__ __forceinline__ double CoulombEnergy(const BoxGeom &g, double distSq,
-                                                double qiqj) {
-  double dist = sqrt(distSq);
-  if (g.ewald) return qiqj * erfc(g.alpha * dist) / dist;
-  return qiqj / dist;
-}
-
 // Mixed precision (FP32 pair terms and phases, FP64 accumulation): the
 // same terms in FP32 from the FP64 squared distance.
 __device__ __forceinline__ double CoulombEnergyF32(const BoxGeom &g, double distSq, double qiqj) {
@@ -253,6 +233,60 @@ __device__ __forceinline__ double ExpNeg(Coefs c, double y) {
   return ldexp(p, int(n));
 }
 
+// Pair terms at precision P (FFParticle::CalcEn / CalcCoulomb,
+// src/FFParticle.cpp:295-399).  FP64: one reciprocal square root (a
+// Newton-refined estimate, then one correction each for r and 1 / r^2, to the
+// last place) stands for the root and the divisions, e^-x^2 and erfcx are
+// polynomials whose coefficients are scalar operands, and nothing is called:
+// a call would save and restore the registers of the pair loops.  LIBM: libm's
+// erfc, whose error is a tenth of the polynomial's 3e-15.
+template <int P, bool LIBM = false>
+__device__ __forceinline__ void PairTermsDev(const BoxGeom &g, Coefs cf, double d2, double qiqj,
+                                             double sigmaSq, double epsCn, double nHalf,
+                                             double sign, double &lj, double &real) {
+  const bool coul = g.elect && qiqj != 0.0 && !(g.rCutCoulSq < d2);
+  const bool inLJ = !(g.rCutLJSq < d2);
+  if (P) {
+    if (coul) real += sign * CoulombEnergyF32(g, d2, qiqj);
+    if (inLJ) lj += sign * LJEnergyF32(d2, sigmaSq, epsCn, nHalf);
+    return;
+  }
+  d2 = fmax(d2, 0x1p-1022);  // coincident atoms: huge, not 0 x inf
+  const double ir = Rsqrt64(d2);
+  double ir2 = ir * ir;
+  ir2 = fma(ir2, fma(-d2, ir2, 1.0), ir2);
+  if (coul) {
+    double e = qiqj * ir;
+    if (LIBM && g.ewald) {
+      double dist = d2 * ir;
+      dist = fma(fma(-dist, dist, d2), 0.5 * ir, dist);
+      e *= erfc(g.alpha * dist);
+    } else if (g.ewald) {
+      double dist = d2 * ir;
+      dist = fma(fma(-dist, dist, d2), 0.5 * ir, dist);
+      const double x = g.alpha * dist;
+      double ex;
+      if (x <= kErfcxUse) {
+        const double u = (x - kErfcxMid) * kErfcxInvHalf;
+        ex = cf[kExpDeg + 1];
+#pragma unroll
+        for (int k = 1; k <= kErfcxDeg; ++k) ex = FmaS(ex, u, cf[kExpDeg + 1 + k]);
+      } else {
+        ex = ErfcxTail(x);
+      }
+      e *= ExpNeg(cf, fmax(-(x * x), -700.0)) * ex;
+    }
+    real += sign * e;
+  }
+  if (inLJ) {
+    const double rRat2 = sigmaSq * ir2;
+    const double att = rRat2 * rRat2 * rRat2;
+    double rep = att * att;
+    if (nHalf != 6.0) rep = MiePow(rRat2, nHalf);
+    lj += sign * (epsCn * (rep - att));
+  }
+}
+
 // Sum over the wave in a fixed tree, valid in lane 63: four steps within rows
 // of 16 lanes, then the rows.  Lane moves are VALU operations here, a shuffle
 // through LDS is several times their latency.
@@ -276,14 +310,6 @@ __device__ __forceinline__ double WaveSumDpp(double v) {
 
 // The pair terms and phases at precision P: 0 is FP64 throughout, 1 the
 // FP32 forms above (sums stay FP64 in every caller).
-template <int P>
-__device__ __forceinline__ double Coul(const BoxGeom &g, double d2, double qiqj) {
-  return P ? CoulombEnergyF32(g, d2, qiqj) : CoulombEnergy(g, d2, qiqj);
-}
-template <int P>
-__device__ __forceinline__ double LJ(double d2, double sig, double eps, double nh) {
-  return P ? LJEnergyF32(d2, sig, eps, nh) : LJEnergy(d2, sig, eps, nh);
-}
 template <int P>
 __device__ __forceinline__ void Sincos(double ang, double *s, double *c) {
   if (P)
@@ -315,6 +341,26 @@ __device__ __forceinline__ T BlockSum(T v, T *lds) {
     for (int w = 0; w < nwaves; ++w) r += lds[w];
   __syncthreads();
   return r;
+}
+
+// Four sums over the workgroup with one barrier, valid in every lane of the
+// first wave: each wave's by lane moves, then one value a lane.
+__device__ __forceinline__ void BlockSum4(double (&v)[4], double (*lds)[4]) {
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int nwaves = blockDim.x / kWave;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = WaveSumDpp(v[i]);
+  if (lane == kWave - 1)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) lds[wave][i] = v[i];
+  __syncthreads();
+  if (wave == 0) {
+    double r = (lane >> 2) < nwaves ? lds[lane >> 2][lane & 3] : 0.0;
+#pragma unroll
+    for (int off = kWave / 2; off >= 4; off >>= 1) r += __shfl_down(r, off, kWave);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __shfl(r, i, kWave);
+  }
 }
 
 }  // namespace gomc

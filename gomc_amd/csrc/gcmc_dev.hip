@@ -573,55 +573,6 @@ NOINLINE __device__ void CellPlace(const DevBox &B, Ctl &c, int a, double x, dou
 }
 
 // ------------------------------------------------- workgroup energy phases --
-// Pair terms at precision P (FFParticle::CalcEn / CalcCoulomb,
-// src/FFParticle.cpp:295-399).  FP64: one reciprocal square root (a
-// Newton-refined estimate, then one correction each for r and 1 / r^2, to the
-// last place) stands for the root and the divisions, e^-x^2 and erfcx are
-// polynomials whose coefficients are scalar operands, and nothing is called:
-// a call would save and restore the registers of the pair loops.
-template <int P>
-__device__ __forceinline__ void PairTermsDev(const BoxGeom &g, Coefs cf, double d2, double qiqj,
-                                             double sigmaSq, double epsCn, double nHalf,
-                                             double sign, double &lj, double &real) {
-  const bool coul = g.elect && qiqj != 0.0 && !(g.rCutCoulSq < d2);
-  const bool inLJ = !(g.rCutLJSq < d2);
-  if (P) {
-    if (coul) real += sign * CoulombEnergyF32(g, d2, qiqj);
-    if (inLJ) lj += sign * LJEnergyF32(d2, sigmaSq, epsCn, nHalf);
-    return;
-  }
-  d2 = fmax(d2, 0x1p-1022);  // coincident atoms: huge, not 0 x inf
-  const double ir = Rsqrt64(d2);
-  double ir2 = ir * ir;
-  ir2 = fma(ir2, fma(-d2, ir2, 1.0), ir2);
-  if (coul) {
-    double e = qiqj * ir;
-    if (g.ewald) {
-      double dist = d2 * ir;
-      dist = fma(fma(-dist, dist, d2), 0.5 * ir, dist);
-      const double x = g.alpha * dist;
-      double ex;
-      if (x <= kErfcxUse) {
-        const double u = (x - kErfcxMid) * kErfcxInvHalf;
-        ex = cf[kExpDeg + 1];
-#pragma unroll
-        for (int k = 1; k <= kErfcxDeg; ++k) ex = FmaS(ex, u, cf[kExpDeg + 1 + k]);
-      } else {
-        ex = ErfcxTail(x);
-      }
-      e *= ExpNeg(cf, fmax(-(x * x), -700.0)) * ex;
-    }
-    real += sign * e;
-  }
-  if (inLJ) {
-    const double rRat2 = sigmaSq * ir2;
-    const double att = rRat2 * rRat2 * rRat2;
-    double rep = att * att;
-    if (nHalf != 6.0) rep = MiePow(rRat2, nHalf);
-    lj += sign * (epsCn * (rep - att));
-  }
-}
-
 // FP64 phases e^{i k.r} of a trial's positions as products of per-axis
 // tables e^{i (2 pi n / L_a) r_a}, |n| <= nmax_a: position p of a trial is its
 // new one of atom p, or its old one of atom p - kDevKindAtoms,
