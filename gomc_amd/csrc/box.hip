@@ -409,6 +409,37 @@ __global__ void __launch_bounds__(kBlock) CacheBuildKernel(const CacheArgs a) {
   }
 }
 
+// Intramolecular Ewald correction of every molecule in the box.
+struct CorrArgs {
+  BoxGeom g;
+  const double *x, *y, *z, *q;
+  const int *mol, *molStart;
+  int nmols;
+  Partial4 *partials;
+  unsigned *counter;
+  double *result;
+};
+
+__global__ void __launch_bounds__(kWave) CorrectionKernel(const CorrArgs a) {
+  __shared__ double red[1][4];
+  const int m = blockIdx.x * kWave + threadIdx.x;
+  double c = 0.0;
+  if (m < a.nmols) {
+    const int s = a.molStart[m], e = a.molStart[m + 1];
+    if (s < e && a.mol[s] >= 0)
+      for (int i = s; i < e; ++i) {
+        if (fabs(a.q[i]) < 0.000000001) continue;
+        for (int j = i + 1; j < e; ++j) {
+          const double dist = sqrt(DistSq(a.g, a.x[i], a.y[i], a.z[i], a.x[j], a.y[j], a.z[j]));
+          c += a.q[i] * a.q[j] * erf(a.g.alpha * dist) / dist;
+        }
+      }
+  }
+  double sum[4] = {0.0, 0.0, -kQQFact * c, 0.0};
+  BlockSum4(sum, red);
+  FinishPartials(Partial4{sum[0], sum[1], sum[2], sum[3]}, a.partials, a.counter, a.result);
+}
+
 // Trial positions of one atom against the live atoms
 // (CalculateEnergy.cpp:741-783): one workgroup per trial.  With the trial
 // cell table (tcCap > 0) a workgroup walks the 27 cells around its
@@ -826,18 +857,33 @@ int BuildCells(gomc_box *b) {
   return GOMC_OK;
 }
 
-static double BoxHostMinImage(double d, int axis, const gomc_box *b) {
-  const double ax = b->geom.L[axis], half = b->geom.half[axis];
-  if (d > half)
-    d -= ax;
-  else if (d < -half)
-    d += ax;
-  return d;
+// Ewald::MolCorrection (src/Ewald.cpp:1236-1265) summed over the box's
+// molecules, a molecule a thread; hostRes[kCorrSlot] once the stream is done.
+// On the host the error functions took 0.13 of the 0.32 ms of a total of 2197
+// waters.
+int LaunchCorrection(gomc_box *b) {
+  CorrArgs a;
+  a.g = b->geom;
+  a.x = b->x;
+  a.y = b->y;
+  a.z = b->z;
+  a.q = b->q;
+  a.mol = b->mol;
+  a.molStart = b->molStartDev;
+  a.nmols = b->nmols;
+  const int nblocks = std::max(1, (b->nmols + kWave - 1) / kWave);
+  int rc = EnsurePartials(b, nblocks);
+  if (rc) return rc;
+  a.partials = b->partials;
+  a.counter = b->counter;
+  a.result = b->devRes + kCorrSlot - 2;
+  hipLaunchKernelGGL(CorrectionKernel, dim3(nblocks), dim3(kWave), 0, b->stream, a);
+  HIP_TRY(b, hipGetLastError());
+  return GOMC_OK;
 }
 
-// Ewald::BoxSelf, MolCorrection summed over molecules, and
-// CalculateEnergy::EnergyCorrection, from the host copy (O(molecules)).
-void HostCorrectionSelfLRC(gomc_box *b, double &self, double &corr, double &lrc) {
+// Ewald::BoxSelf and CalculateEnergy::EnergyCorrection (O(kinds)).
+void HostSelfLRC(gomc_box *b, double &self, double &lrc) {
   self = 0.0;
   for (int k = 0; k < b->nkinds; ++k) {
     double molSelf = 0.0;
@@ -845,23 +891,6 @@ void HostCorrectionSelfLRC(gomc_box *b, double &self, double &corr, double &lrc)
     self += (molSelf * unsigned(b->kindCount[k]));
   }
   self *= -1.0 * b->alpha * kQQFact * M_2_SQRTPI * 0.5;
-  corr = 0.0;
-  for (int m = 0; m < b->nmols; ++m) {
-    if (!b->molBox.empty() && b->molBox[m] != 0) continue;
-    const int s = b->molStart[m], len = b->molLen[m], kind = b->molKind[m];
-    double c = 0.0;
-    for (int i = 0; i < len; ++i) {
-      if (std::fabs(b->kindCharge[kind][i]) < 0.000000001) continue;
-      for (int j = i + 1; j < len; ++j) {
-        double dx = BoxHostMinImage(b->hx[s + i] - b->hx[s + j], 0, b);
-        double dy = BoxHostMinImage(b->hy[s + i] - b->hy[s + j], 1, b);
-        double dz = BoxHostMinImage(b->hz[s + i] - b->hz[s + j], 2, b);
-        double dist = std::sqrt(dx * dx + dy * dy + dz * dz);
-        c += (b->kindCharge[kind][i] * b->kindCharge[kind][j] * std::erf(b->alpha * dist) / dist);
-      }
-    }
-    corr += -1.0 * kQQFact * c * 1.0 * 1.0;
-  }
   lrc = 0.0;
   for (int i = 0; i < b->nkinds; ++i)
     for (int j = 0; j < b->nkinds; ++j)

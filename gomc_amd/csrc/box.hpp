@@ -289,7 +289,9 @@ int HipFail(gomc_box *b, hipError_t e, const char *what);
 int LaunchTrial(gomc_box *b, int mol, const double *ox, const double *oy, const double *oz,
                 const double *nx, const double *ny, const double *nz, bool doPair,
                 bool doRecip, double out[4]);
-void HostCorrectionSelfLRC(gomc_box *b, double &self, double &corr, double &lrc);
+constexpr int kCorrSlot = 10;  // of hostRes: LaunchCorrection's sum
+int LaunchCorrection(gomc_box *b);
+void HostSelfLRC(gomc_box *b, double &self, double &lrc);
 int RecipSums(gomc_box *b, double *erecip);
 // The k list's columns and work units (after the k-vectors change).
 int BuildKPlan(gomc_box *b, const std::vector<double> &kx, const std::vector<double> &ky,

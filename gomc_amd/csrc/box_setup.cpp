@@ -359,13 +359,15 @@ int gomc_box_create(const gomc_system_desc *d, int device, gomc_box **out) {
     }
   }
   double lj = 0, real = 0;
-  int rc = BoxInter(b, &lj, &real);
+  int rc = b->ewald ? LaunchCorrection(b) : GOMC_OK;
+  if (!rc) rc = BoxInter(b, &lj, &real);
   if (rc) {
     gomc_box_destroy(b);
     return rc;
   }
   double self = 0, corr = 0, lrc = 0;
-  HostCorrectionSelfLRC(b, self, corr, lrc);
+  HostSelfLRC(b, self, lrc);
+  if (b->ewald) corr = b->hostRes[kCorrSlot];
   b->pot.inter = lj;
   b->pot.real = real;
   b->pot.recip = erecip;
@@ -469,10 +471,12 @@ int gomc_system_total(gomc_box *b, double out[7]) {
     if (rc) return rc;
   }
   double lj = 0, real = 0;
-  rc = BoxInter(b, &lj, &real);
+  if (b->ewald) rc = LaunchCorrection(b);
+  if (!rc) rc = BoxInter(b, &lj, &real);
   if (rc) return rc;
   double self = 0, corr = 0, lrc = 0;
-  HostCorrectionSelfLRC(b, self, corr, lrc);
+  HostSelfLRC(b, self, lrc);
+  if (b->ewald) corr = b->hostRes[kCorrSlot];
   Energies e;
   e.inter = lj;
   e.tc = b->lrc ? lrc : 0.0;
