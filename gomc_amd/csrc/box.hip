@@ -42,7 +42,7 @@ struct TrialArgs {
   const int *type, *mol;
   const double *sigSq, *epsCn, *nHalf;
   int ntypes, natoms, mstart, mlen;
-  int nPairBlocks, doPair, doRecip, K;
+  int nPairBlocks, doPair, doRecip, K, kRuns;
   double ox[kMaxMolAtoms], oy[kMaxMolAtoms], oz[kMaxMolAtoms];
   double nx[kMaxMolAtoms], ny[kMaxMolAtoms], nz[kMaxMolAtoms];
   double mq[kMaxMolAtoms];
@@ -110,7 +110,12 @@ __device__ __forceinline__ void TrialAtom(const TrialArgs &a, int j, double xj, 
 // thread, pair terms without calls and one barrier a reduction took the kernel
 // from 14 us to 9.8 for 300 to 1000 waters; all of a molecule's positions
 // in one thread are six pair terms or sincos in a row.
-constexpr int kTrialK = kBlock / 2;  // k-vectors of a block
+constexpr int kTrialK = kBlock / 2;  // k-vectors of a block's run
+// A block takes as many runs as keep the reciprocal blocks to this: each block
+// costs the last one's counter and sums a little, and from 16384 k-vectors on
+// that outweighs the shorter chain (8000 waters, 25,000 k-vectors, mixed: call
+// 35.2 us with one run a block, as before the split; 33.4 with two).
+constexpr int kTrialRecipBlocks = 128;
 template <int P>
 __global__ void __launch_bounds__(kBlock) TrialKernel(const TrialArgs a) {
   __shared__ double red[kBlock / kWave][4];
@@ -151,37 +156,41 @@ __global__ void __launch_bounds__(kBlock) TrialKernel(const TrialArgs a) {
       TrialAtom<P>(a, j, xj, yj, zj, p, mask, sum[0], sum[1], sum[3]);
     }
   } else if (a.doRecip) {
-    const int k = (blockIdx.x - a.nPairBlocks) * kTrialK + (tid >> 1);
-    const bool old = tid & 1, on = k < a.K;
-    double R = 0.0, I = 0.0;
-    if (on) {
-      if (old && a.oldC) {  // EwaldCached::MolReciprocal (EwaldCached.cpp:244-295)
-        R = a.oldC[k];
-        I = a.oldS[k];
-      } else {
-        const double kxk = a.kx[k], kyk = a.ky[k], kzk = a.kz[k];
-        for (int p = 0; p < a.mlen; ++p) {
-          if (fabs(a.mq[p]) < 0.000000001) continue;
-          const double dot = old ? a.ox[p] * kxk + a.oy[p] * kyk + a.oz[p] * kzk
-                                 : a.nx[p] * kxk + a.ny[p] * kyk + a.nz[p] * kzk;
-          double sn, cs;
-          Sincos<P>(dot, &sn, &cs);
-          R += a.mq[p] * cs;
-          I += a.mq[p] * sn;
+    const bool old = tid & 1;
+    const int first = (blockIdx.x - a.nPairBlocks) * a.kRuns * kTrialK;
+    for (int k0 = first; k0 < min(first + a.kRuns * kTrialK, a.K); k0 += kTrialK) {
+      const int k = k0 + (tid >> 1);
+      const bool on = k < a.K;
+      double R = 0.0, I = 0.0;
+      if (on) {
+        if (old && a.oldC) {  // EwaldCached::MolReciprocal (EwaldCached.cpp:244-295)
+          R = a.oldC[k];
+          I = a.oldS[k];
+        } else {
+          const double kxk = a.kx[k], kyk = a.ky[k], kzk = a.kz[k];
+          for (int p = 0; p < a.mlen; ++p) {
+            if (fabs(a.mq[p]) < 0.000000001) continue;
+            const double dot = old ? a.ox[p] * kxk + a.oy[p] * kyk + a.oz[p] * kzk
+                                   : a.nx[p] * kxk + a.ny[p] * kyk + a.nz[p] * kzk;
+            double sn, cs;
+            Sincos<P>(dot, &sn, &cs);
+            R += a.mq[p] * cs;
+            I += a.mq[p] * sn;
+          }
         }
       }
-    }
-    const double RO = __shfl_down(R, 1, kWave), IO = __shfl_down(I, 1, kWave);
-    if (on && !old) {
-      if (a.oldC) {
-        a.stC[k] = R;
-        a.stS[k] = I;
+      const double RO = __shfl_down(R, 1, kWave), IO = __shfl_down(I, 1, kWave);
+      if (on && !old) {
+        if (a.oldC) {
+          a.stC[k] = R;
+          a.stS[k] = I;
+        }
+        R = a.sumRref[k] + (R - RO);
+        I = a.sumIref[k] + (I - IO);
+        a.sumRnew[k] = R;
+        a.sumInew[k] = I;
+        sum[2] += (R * R + I * I) * a.pref[k];
       }
-      R = a.sumRref[k] + (R - RO);
-      I = a.sumIref[k] + (I - IO);
-      a.sumRnew[k] = R;
-      a.sumInew[k] = I;
-      sum[2] = (R * R + I * I) * a.pref[k];
     }
   }
   BlockSum4(sum, red);
@@ -702,7 +711,9 @@ int LaunchTrial(gomc_box *b, int m, const double *ox, const double *oy, const do
   }
   a.doPair = doPair;
   a.doRecip = doRecip && b->ewald;
-  const int nRecip = a.doRecip ? (b->K + kTrialK - 1) / kTrialK : 0;
+  const int runs = (b->K + kTrialK - 1) / kTrialK;
+  a.kRuns = std::max(1, (runs + kTrialRecipBlocks - 1) / kTrialRecipBlocks);
+  const int nRecip = a.doRecip ? (runs + a.kRuns - 1) / a.kRuns : 0;
   a.K = b->K;
   a.kx = b->kx;
   a.ky = b->ky;
