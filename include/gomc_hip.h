@@ -174,7 +174,7 @@ int gomc_recip_sums(gomc_box *b, double *erecip);
 /* gomc_recip_sums without allocating: no counterpart in the reference; for
  * callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops).  Same kernels and results; the scratch
- * (per-chunk sums, block partials, counter) lives in one 32.1 MiB
+ * (per-chunk sums, block partials, counter) lives in one 32.5 MiB
  * file-scope device array per GPU, held until the process ends, so calls
  * that overlap on one GPU race.  Refuses boxes of more than 2^20 k-vectors
  * (GOMC_ERR_ARG).  The box must have been set up by gomc_recip_init. */
