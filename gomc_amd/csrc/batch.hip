@@ -494,7 +494,8 @@ __device__ __forceinline__ void PairPhase(const LMEM BatchBox *sb, const LMEM Co
   LMEM int *list[2] = {nearList + wave * 2 * kNearListLen, nearList + (wave * 2 + 1) * kNearListLen};
   const uint64_t below = (uint64_t(1) << lane) - 1;
   const bool cull = __builtin_amdgcn_readfirstlane(sb->cull) != 0;
-  const double rCutSq = Uniform(sb->rCutSq), rLowSq = Uniform(sb->rCutLowSq);
+  // an overlap is a pair inside the cutoff as well, however large RcutLow
+  const double rCutSq = Uniform(sb->rCutSq), rLowSq = fmin(Uniform(sb->rCutLowSq), rCutSq);
   const uint32_t liveBits = __builtin_amdgcn_readfirstlane(uint32_t(sb->live));
   const int mol[2] = {__builtin_amdgcn_readfirstlane(mv[0].mol),
                       __builtin_amdgcn_readfirstlane(mv[1].mol)};
