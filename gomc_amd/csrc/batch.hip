@@ -32,8 +32,8 @@
 //   2454, team of 2            10.7 /  8.4, was 13.7 / 12.2
 //   3950, team of 8             8.2 /  6.3, was 11.0 / 10.3
 #include "batch.hpp"
+#include "coul_table.hpp"
 #include "device_common.hpp"
-#include "erfcx_poly.hpp"
 
 namespace gomc {
 namespace {
@@ -292,92 +292,15 @@ struct LjReal {
   double lj, real;
 };
 
-// The Coulomb factor erfc(alpha r) / r (1 / r without Ewald) as a function of
-// r^2, a polynomial of degree 7 in each 64th of an octave of r^2 from 1 to 256
-// A^2: row and offset come from the bits of r^2, and seven multiply-adds stand
-// for the reciprocal square root, the exponential and the 28th-degree erfcx
-// (75 instructions).  Made per box from libm's erfc at the rows' Chebyshev
-// nodes, as differences from the row's middle so that nothing cancels: within
-// a few 1e-16 of erfc(alpha r) / r at small alpha r and a few 1e-15 at alpha r
-// = 3.4 (the fit had 3e-15 throughout), where erfc itself is 1e-6.  The terms
-// beyond r^2 = 256 or below 1 are computed directly.
-constexpr int kTabBits = 6, kTabOctaves = 8, kTabRows = kTabOctaves << kTabBits, kTabDeg = 7;
-constexpr int kTabShift = 20 - kTabBits, kTabBase = 0x3ff << kTabBits;
+// The box's Coulomb table (coul_table.hpp), copied to LDS when its run starts.
 struct alignas(16) CoulTab {
-  double c[kTabRows * (kTabDeg + 1)];
+  double c[kTabWords];
 };
-// Where coefficient k of a row lies: pairs of coefficients (16 bytes) change
-// places from row to row, so that one pair of many rows is spread over all LDS
-// banks (a row is a quarter of them).
-__device__ __forceinline__ int TabAt(int row, int k) {
-  return row * (kTabDeg + 1) + (k ^ ((row >> 1) & 6));
-}
 
-// Coefficients of the interpolating polynomial from its values at the eight
-// Chebyshev nodes of [-1, 1]: m[k][j] multiplies value j in the coefficient of
-// s^k (the Lagrange polynomials, expanded).
-struct Lagrange8 {
-  double node[8], m[8][8];
-};
-constexpr Lagrange8 MakeLagrange8() {
-  Lagrange8 l{};
-  const double n[4] = {0.98078528040323044913, 0.83146961230254523708, 0.55557023301960222474,
-                       0.19509032201612826785};  // cos((2 j + 1) pi / 16)
-  for (int j = 0; j < 8; ++j) l.node[j] = j < 4 ? n[j] : -n[7 - j];
-  for (int j = 0; j < 8; ++j) {
-    double p[8] = {1.0, 0, 0, 0, 0, 0, 0, 0}, den = 1.0;
-    int deg = 0;
-    for (int i = 0; i < 8; ++i) {
-      if (i == j) continue;
-      den *= l.node[j] - l.node[i];
-      ++deg;
-      for (int k = deg; k >= 0; --k)
-        p[k] = (k > 0 ? p[k - 1] : 0.0) - l.node[i] * (k < deg ? p[k] : 0.0);
-    }
-    for (int k = 0; k < 8; ++k) l.m[k][j] = p[k] / den;
-  }
-  return l;
-}
-static __constant__ Lagrange8 lagrange8 = MakeLagrange8();
-
+// The same factor below the table's first octave.
 __device__ __noinline__ double CoulFactor(const LMEM BatchBox *sb, double d2) {
   const double r = sqrt(d2);
   return sb->ewald ? erfc(sb->alpha * r) / r : 1.0 / r;
-}
-
-// Middle and half width of a row.
-__device__ __forceinline__ void TabRow(int row, double *mid, double *half) {
-  const uint32_t hi = (uint32_t(row + kTabBase) << kTabShift) | (1u << (kTabShift - 1));
-  *mid = __builtin_bit_cast(double, uint64_t(hi) << 32);
-  *half = ldexp(1.0, (row >> kTabBits) - kTabBits - 1);
-}
-
-__device__ __noinline__ void BuildCoulTab(const LMEM BatchBox *sb, LMEM CoulTab *tab) {
-  for (int i = threadIdx.x; i < kTabRows * 8; i += kBatchThreads) {
-    double mid, half;
-    TabRow(i / 8, &mid, &half);
-    tab->c[TabAt(i / 8, i % 8)] = CoulFactor(sb, fma(half, lagrange8.node[i % 8], mid));
-  }
-  __syncthreads();
-  for (int row = threadIdx.x; row < kTabRows; row += kBatchThreads) {
-    double mid, half, g[8], c[8];
-    TabRow(row, &mid, &half);
-    const double f0 = CoulFactor(sb, mid);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) g[j] = tab->c[TabAt(row, j)] - f0;
-    double scale = 1.0;
-    const double inv = 1.0 / half;  // a power of two
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      double v = 0.0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v = fma(lagrange8.m[k][j], g[j], v);
-      c[k] = k == 0 ? f0 + v : v * scale;
-      scale *= inv;
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) tab->c[TabAt(row, k)] = c[k];
-  }
 }
 
 // Energy terms of one pair (FFParticle::CalcEn / CalcCoulomb,
@@ -392,26 +315,11 @@ __device__ __forceinline__ LjReal PairTerm(const LMEM BatchBox *sb, const LMEM C
   const double qiqj = sb->qq[pq], eps = sb->epsCn[pq];
   if constexpr (sizeof(T) == 8) {
     if (sb->elect && qiqj != 0.0 && !(sb->rCutCoulSq < d2)) {
-      const uint64_t u = __builtin_bit_cast(uint64_t, d2);
-      const int row = int(uint32_t(u >> 32) >> kTabShift) - kTabBase;
-      double f;
-      if (uint32_t(row) < uint32_t(kTabRows)) {
-        const uint32_t mid = (uint32_t(u >> 32) & ~((1u << kTabShift) - 1)) | (1u << (kTabShift - 1));
-        const double t = d2 - __builtin_bit_cast(double, uint64_t(mid) << 32);
-        typedef double v2d __attribute__((ext_vector_type(2)));
-        const LMEM v2d *c = (const LMEM v2d *)(tab->c + row * (kTabDeg + 1));
-        const int x = (row >> 2) & 3;
-        const v2d c6 = c[3 ^ x], c4 = c[2 ^ x], c2 = c[1 ^ x], c0 = c[x];
-        f = fma(c6.y, t, c6.x);
-        f = fma(f, t, c4.y);
-        f = fma(f, t, c4.x);
-        f = fma(f, t, c2.y);
-        f = fma(f, t, c2.x);
-        f = fma(f, t, c0.y);
-        f = fma(f, t, c0.x);
-      } else {
-        f = CoulFactor(sb, d2);
-      }
+      double t;
+      const int row = TabRow(d2, sb->tabBase, &t);
+      const double f = uint32_t(row) < uint32_t(kTabRows)
+                           ? TabValue((const LMEM TabPair *)tab->c, (const LMEM double *)tab->c, row, t)
+                           : CoulFactor(sb, d2);
       out.real = (sign * qiqj) * f;
     }
     if (eps != 0.0 && !(sb->rCutLJSq < d2)) {
@@ -1405,8 +1313,11 @@ __global__ void __launch_bounds__(kBatchThreads) McBatchKernel(const BatchArgs a
           Lp(ldsCom)[a.ldsMols + i] = float(r.CYg[i]);
           Lp(ldsCom)[2 * a.ldsMols + i] = float(r.CZg[i]);
         }
-      if (PREC == 0 && sb->elect) BuildCoulTab(sb, Lp(&ctabS));
-      // the tables and centres are read after the programs' first barrier
+      if (PREC == 0 && sb->elect) {
+        const GMEM TabPair *src = (const GMEM TabPair *)(a.coulTab + size_t(b) * kTabWords);
+        for (int i = tid; i < kTabWords / 2; i += kBatchThreads) ((LMEM TabPair *)Lp(ctabS.c))[i] = src[i];
+      }
+      // the table and centres are read after the programs' first barrier
       Cursor c;
       switch (len) {
         case 1:

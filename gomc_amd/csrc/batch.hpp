@@ -6,10 +6,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <memory>
 #include <string>
 #include <vector>
 
 #include "../../include/gomc_hip.h"
+#include "coul_table.hpp"
 #include "host_rng.hpp"
 
 namespace gomc {
@@ -64,6 +66,7 @@ struct BatchBox {
   int cull;  // 1: cull far molecules by their centres before atom pairs
   float nearCutSqF;  // (rc + 2 r_max + margin)^2: centres farther apart than this hold
                      // no pair inside the cutoff; the margin covers FP32 centres
+  int tabBase;       // of its Coulomb table
   int wide;          // 1: half of every edge exceeds the cutoff and the molecule's radius
   int team;  // workgroups running the box (1, 2, 4, 8)
   int live;  // bit p * kBatchMaxAtoms + q: atoms p, q interact (charge or LJ)
@@ -112,6 +115,7 @@ struct BatchArgs {
   double *sumR, *sumI;        // reference structure factors
   double *dR, *dI;            // structure-factor change of a pass's first move
   double *dR2, *dI2;          // and of its second; null: one move per pass
+  const double *coulTab;      // [nboxes][kTabWords] Coulomb tables (FP64)
   const int64_t *moves;       // [nboxes] moves to make in this launch
   int ldsMols;                // per-box centre capacity of dynamic LDS
   BatchTrace trace;
@@ -134,6 +138,9 @@ struct gomc_batch {
   int32_t *kn = nullptr;
   double *pref = nullptr, *sumR = nullptr, *sumI = nullptr, *dR = nullptr, *dI = nullptr;
   double *dR2 = nullptr, *dI2 = nullptr;
+  double *coulTab = nullptr;  // FP64 only
+  // the table of the box packed last: boxes of one alpha and cutoff share it
+  std::shared_ptr<const gomc::CoulTable> table;
   int64_t *moves = nullptr;
   // workgroup task lists (device) and their capacity; team exchange blocks
   gomc::BatchTask *tasks = nullptr;
@@ -181,6 +188,7 @@ struct PackedBox {
   BatchState S;
   std::vector<double> x, y, z, cx, cy, cz, pref, sr, si;
   std::vector<int32_t> kn;
+  std::shared_ptr<const CoulTable> table;  // FP64 with electrostatics
 };
 // Builds the box once through the plain path (initial energies, structure
 // factors, centres) and packs it at the given offsets; errors go to bt->err.

@@ -26,7 +26,7 @@ int BFail(gomc_batch *bt, int code, const std::string &msg) {
 
 void FreeBatch(gomc_batch *bt) {
   void *ptrs[] = {bt->boxes, bt->state, bt->x,    bt->y,    bt->z,    bt->cx,         bt->cy,
-                  bt->cz,    bt->kn,    bt->pref, bt->sumR, bt->sumI, bt->dR, bt->dI, bt->dR2, bt->dI2, bt->moves,      bt->trace.acc,
+                  bt->cz,    bt->kn,    bt->pref, bt->sumR, bt->sumI, bt->dR, bt->dI, bt->dR2, bt->dI2, bt->coulTab, bt->moves, bt->trace.acc,
                   bt->trace.dlj, bt->trace.dreal, bt->trace.drecip, bt->tasks, bt->wgTask,
                   bt->xchg, bt->errFlag, bt->boxTicks};
   for (void *p : ptrs)
@@ -142,6 +142,17 @@ int PackBox(gomc_batch *bt, const gomc_system_desc &d, int64_t atomOff, int64_t 
     return BFail(bt, GOMC_ERR_ARG, "box too large for the batched item indexing");
   P.ewald = b->ewald;
   P.elect = b->elect;
+  out.table.reset();
+  if (bt->precision == 0 && b->elect) {
+    const CoulTable *t = bt->table.get();
+    if (!t || t->alpha != b->alpha || t->ewald != b->ewald || t->base != TabBase(P.rCutCoulSq)) {
+      auto made = std::make_shared<CoulTable>();
+      MakeCoulTable(b->alpha, b->ewald, P.rCutCoulSq, made.get());
+      bt->table = std::move(made);
+    }
+    out.table = bt->table;
+    P.tabBase = out.table->base;
+  }
   out.x = b->hx;
   out.y = b->hy;
   out.z = b->hz;
@@ -249,6 +260,7 @@ BatchArgs MakeArgs(const gomc_batch *bt) {
   a.dI = bt->dI;
   a.dR2 = bt->dR2;
   a.dI2 = bt->dI2;
+  a.coulTab = bt->coulTab;
   a.moves = bt->moves;
   a.tasks = bt->tasks;
   a.wgTask = bt->wgTask;
@@ -286,6 +298,8 @@ int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t 
     ok &= alloc((void **)&bt->dR2, sizeof(double) * kvec);
     ok &= alloc((void **)&bt->dI2, sizeof(double) * kvec);
   }
+  if (bt->precision == 0)
+    ok &= alloc((void **)&bt->coulTab, sizeof(double) * kTabWords * size_t(nboxes));
   // one workgroup per compute unit: the kernel's 1024 threads at 128
   // registers fill a CU, and team members must all be resident at once
   int cus = 0;
@@ -332,6 +346,8 @@ int UploadBox(gomc_batch *bt, int slot, const PackedBox &pb) {
     BHIP(bt, up(bt->cy + mo, pb.cy.data(), sizeof(double) * pb.cy.size()));
     BHIP(bt, up(bt->cz + mo, pb.cz.data(), sizeof(double) * pb.cz.size()));
   }
+  if (pb.table)
+    BHIP(bt, up(bt->coulTab + size_t(slot) * kTabWords, pb.table->c.data(), sizeof(double) * kTabWords));
   BHIP(bt, up(bt->kn + P.kOff, pb.kn.data(), sizeof(int32_t) * pb.kn.size()));
   BHIP(bt, up(bt->pref + P.kOff, pb.pref.data(), sizeof(double) * pb.pref.size()));
   BHIP(bt, up(bt->sumR + P.kOff, pb.sr.data(), sizeof(double) * pb.sr.size()));

@@ -163,6 +163,7 @@ struct gomc_server {
   double kernelSec = 0.0;
   bool stop = false;
   std::string err;
+  std::shared_ptr<const CoulTable> table;  // of the job packed last
   std::thread loop;
   std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
   // GCMC lane
@@ -236,6 +237,7 @@ void Admit(gomc_server *sv, std::unique_lock<std::mutex> &lk) {
     j->pb.kn.clear();
     j->pb.sr.clear();
     j->pb.si.clear();
+    j->pb.table.reset();
   }
 }
 
@@ -582,7 +584,12 @@ int gomc_server_submit(gomc_server *sv, const gomc_system_desc *d, int64_t moves
   // the caller's thread, while the loop keeps the device busy
   gomc_batch scratch;  // holds the packing error, not shared with the loop
   scratch.device = sv->device;
+  scratch.precision = sv->precision;
   scratch.teams = false;
+  {
+    std::lock_guard<std::mutex> g(sv->mu);
+    scratch.table = sv->table;
+  }
   int rc = PackBox(&scratch, *d, 0, 0, 0, j->pb);
   if (rc) {
     std::lock_guard<std::mutex> g(sv->mu);
@@ -597,6 +604,7 @@ int gomc_server_submit(gomc_server *sv, const gomc_system_desc *d, int64_t moves
   // per-move cost of the batched kernel at this size, FP64, microseconds
   j->costUs = 10.0 + 0.006 * double(j->pb.P.nmols);
   std::lock_guard<std::mutex> g(sv->mu);
+  if (scratch.table) sv->table = scratch.table;
   j->id = sv->nextId++;
   j->tSubmit = Now(sv->t0);
   *job_id = j->id;
