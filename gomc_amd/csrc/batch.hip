@@ -940,7 +940,7 @@ __device__ __forceinline__ void Settle(LMEM BatchState *st, bool accept, double 
 // 0), so a pass waits for one exponential.  Then lane 0 settles the moves.
 __device__ __noinline__ void Decide(const LMEM BatchBox *sb, LMEM BatchState *st,
                                     LMEM MoveShared *ms, const LMEM double *uA,
-                                    const LMEM double *uB, int has, const BatchTrace *trace,
+                                    const LMEM double *uB, int has, const LMEM BatchTrace *trace,
                                     int64_t at) {
   const int lane = int(threadIdx.x) & (kWave - 1);
   const LMEM double *s = ms->tot;
@@ -994,6 +994,9 @@ __device__ __noinline__ void Decide(const LMEM BatchBox *sb, LMEM BatchState *st
 // draws are made): called once a box, so the phases' many registers are saved
 // once, not once a pass.  Which moves a pass holds follows from the draws and
 // the step alone, so every wave finds it for itself.
+// A run's pointers lie in LDS, one copy a workgroup: in a lane's private memory
+// they were 300 bytes of scratch stored by each of 1024 lanes, and the trace's
+// address took the kernel's arguments there too, 21 us of every launch.
 template <typename T>
 struct BoxRun {
   const LMEM BatchBox *sb;
@@ -1012,10 +1015,11 @@ struct BoxRun {
   DeltaPtrs delta;
   GMEM uint64_t *xb;
   GMEM int *err;
-  const BatchTrace *trace;  // null: another box's
+  BatchTrace trace;
   int64_t step, end;
   uint64_t pass;
   int rank, team, pairs;    // pairs: passes of two moves
+  int traced;               // 1: this member writes the trace
 };
 
 // Where a box's run stands, the same in every wave.  An even step A and the
@@ -1083,20 +1087,19 @@ __device__ __forceinline__ void WaveFence() {
 
 // Totals, decisions and commit of a pass, by wave 0.
 template <typename T>
-__device__ __noinline__ void FinishPass(const BoxRun<T> *rp, int uA, int uB, int has, uint64_t pass,
+__device__ __noinline__ void FinishPass(const LMEM BoxRun<T> *r, int uA, int uB, int has, uint64_t pass,
                                         int64_t at, int pw, int waves, int len) {
-  const BoxRun<T> &r = *rp;
-  LMEM MoveShared *ms = r.ms;
+  LMEM MoveShared *ms = r->ms;
   const LMEM double *red = &ms->red[0][0];
   const int tid = threadIdx.x, i = tid % kXchgVals;
   // value i comes from the pair waves, the reciprocal waves or the last pair wave
   const int w0 = i < kRecA ? 0 : (i < kXLj0 ? pw : pw - 1);
-  const int w1 = i < kRecA ? pw : (i < kXLj0 ? waves : (r.rank == 0 ? pw : pw - 1));
+  const int w1 = i < kRecA ? pw : (i < kXLj0 ? waves : (r->rank == 0 ? pw : pw - 1));
   double v = 0.0;
   for (int w = w0; w < w1; ++w) v += red[w * kXchgVals + i];
   if (i >= kNumSums) v = 0.0;
-  if (r.team > 1) {
-    const TeamValue t = TeamSum(r.xb, r.team, r.rank, pass + 1, v, r.err);
+  if (r->team > 1) {
+    const TeamValue t = TeamSum(r->xb, r->team, r->rank, pass + 1, v, r->err);
     v = t.v;
     if (!t.ok) {
       if (tid == 0) ms->abort = 1;
@@ -1105,7 +1108,7 @@ __device__ __noinline__ void FinishPass(const BoxRun<T> *rp, int uA, int uB, int
   }
   if (tid < kXchgVals) ms->tot[tid] = v;
   WaveFence();
-  Decide(r.sb, r.st, ms, r.draws[uA], r.draws[uB], has, r.trace, at);
+  Decide(r->sb, r->st, ms, r->draws[uA], r->draws[uB], has, r->traced ? &r->trace : nullptr, at);
   WaveFence();
   // S(k) follows in the next pass's reciprocal phase
   const int mvI = tid / 32, p = tid % 32;
@@ -1114,18 +1117,18 @@ __device__ __noinline__ void FinishPass(const BoxRun<T> *rp, int uA, int uB, int
     const int m = mv->mol;
     if (p < len) {
       const int64_t ai = int64_t(m) * len + p;
-      r.X[ai] = mv->newp[0][p];
-      r.Y[ai] = mv->newp[1][p];
-      r.Z[ai] = mv->newp[2][p];
+      r->X[ai] = mv->newp[0][p];
+      r->Y[ai] = mv->newp[1][p];
+      r->Z[ai] = mv->newp[2][p];
     }
     if (p == 0 && mv->type == 0) {
-      r.CXg[m] = mv->com[1][0];
-      r.CYg[m] = mv->com[1][1];
-      r.CZg[m] = mv->com[1][2];
-      if (r.CX) {
-        r.CX[m] = float(mv->com[1][0]);
-        r.CY[m] = float(mv->com[1][1]);
-        r.CZ[m] = float(mv->com[1][2]);
+      r->CXg[m] = mv->com[1][0];
+      r->CYg[m] = mv->com[1][1];
+      r->CZg[m] = mv->com[1][2];
+      if (r->CX) {
+        r->CX[m] = float(mv->com[1][0]);
+        r->CY[m] = float(mv->com[1][1]);
+        r->CZ[m] = float(mv->com[1][2]);
       }
     }
   }
@@ -1133,8 +1136,8 @@ __device__ __noinline__ void FinishPass(const BoxRun<T> *rp, int uA, int uB, int
 
 // The pair waves' program; wave 0 also proposes, decides and commits.
 template <typename T, int LEN, typename ComPtr>
-__device__ __noinline__ Cursor PairProgram(const BoxRun<T> *rp, ComPtr CX, ComPtr CY, ComPtr CZ) {
-  BoxRun<T> r = *rp;
+__device__ __noinline__ Cursor PairProgram(const LMEM BoxRun<T> *rp, ComPtr CX, ComPtr CY, ComPtr CZ) {
+  BoxRun<T> r = *(const BoxRun<T> *)rp;
   r.X = UniformPtr(r.X);
   r.Y = UniformPtr(r.Y);
   r.Z = UniformPtr(r.Z);
@@ -1181,8 +1184,8 @@ __device__ __noinline__ Cursor PairProgram(const BoxRun<T> *rp, ComPtr CX, ComPt
 
 // The reciprocal waves' program.
 template <typename T, int S, int LEN>
-__device__ __noinline__ Cursor RecipProgram(const BoxRun<T> *rp) {
-  const BoxRun<T> r = *rp;
+__device__ __noinline__ Cursor RecipProgram(const LMEM BoxRun<T> *rp) {
+  const BoxRun<T> r = *(const BoxRun<T> *)rp;
   const LMEM BatchBox *sb = r.sb;
   LMEM double *red = &r.ms->red[0][0];
   const int nmols = __builtin_amdgcn_readfirstlane(sb->nmols);
@@ -1210,7 +1213,7 @@ __device__ __noinline__ Cursor RecipProgram(const BoxRun<T> *rp) {
 }
 
 template <typename T, int LEN>
-__device__ __forceinline__ Cursor RunBox(const BoxRun<T> *r, int wave) {
+__device__ __forceinline__ Cursor RunBox(const LMEM BoxRun<T> *r, int wave) {
   if (wave < __builtin_amdgcn_readfirstlane(r->sb->pairWaves)) {
     if (r->CX) return PairProgram<T, LEN>(r, r->CX, r->CY, r->CZ);
     return PairProgram<T, LEN>(r, r->CXg, r->CYg, r->CZg);
@@ -1238,6 +1241,7 @@ __global__ void __launch_bounds__(kBatchThreads) McBatchKernel(const BatchArgs a
   __shared__ PairQueue queuesS[kPairWavesMax];
   __shared__ int nearListS[kPairWavesMax * 2 * kNearListLen];
   __shared__ CoulTab ctabS;
+  __shared__ BoxRun<T> runS;
   extern __shared__ float ldsCom[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -1254,64 +1258,66 @@ __global__ void __launch_bounds__(kBatchThreads) McBatchKernel(const BatchArgs a
       msS.abort = 0;
       stS = a.state[b];
     }
+    if (tid == kWave) {
+      const BatchBox &box = a.boxes[b];
+      const int64_t aoff = box.atomOff, moff = box.molOff, koff = box.kOff;
+      BoxRun<T> &r = runS;
+      r.sb = Lp(&sbS);
+      r.st = Lp(&stS);
+      r.ms = Lp(&msS);
+      r.tab = Lp(tabS);
+      r.ctab = Lp(&ctabS);
+      r.queues = Lp(queuesS);
+      r.nearList = Lp(nearListS);
+      r.draws = Lp(drawsS);
+      // The box's molecule centres, rounded to FP32, live in LDS for the launch
+      // when they fit (a.ldsMols per workgroup): the cull reads them there.
+      r.CX = box.nmols <= a.ldsMols ? Lp(ldsCom) : nullptr;
+      r.CY = r.CX + a.ldsMols;
+      r.CZ = r.CX + 2 * a.ldsMols;
+      // Team members share the box's coordinates and centres.  Every member
+      // writes the same accepted values at the same point of a pass, after the
+      // exchange that needs all members' pair phases of that pass, and reads
+      // them only after its own write and a barrier: a read sees its own
+      // member's write or another's identical one.
+      r.X = Gp(a.x + aoff);
+      r.Y = Gp(a.y + aoff);
+      r.Z = Gp(a.z + aoff);
+      r.CXg = Gp(a.cx + moff);
+      r.CYg = Gp(a.cy + moff);
+      r.CZg = Gp(a.cz + moff);
+      r.kn = Gp(a.kn + koff);
+      r.pref = Gp(a.pref + koff);
+      r.sumR = Gp(a.sumR + koff);
+      r.sumI = Gp(a.sumI + koff);
+      r.delta = DeltaPtrs{{Gp(a.dR + koff), Gp(a.dR2 ? a.dR2 + koff : a.dR + koff)},
+                          {Gp(a.dI + koff), Gp(a.dI2 ? a.dI2 + koff : a.dI + koff)}};
+      r.xb = Gp(a.xchg + int64_t(b) * kXchgWords);
+      r.err = Gp(a.err);
+      r.trace = a.trace;
+      r.traced = rank == 0 && b == a.trace.box;
+      r.step = a.state[b].step;
+      r.end = r.step + a.moves[b];
+      r.pass = uint64_t(a.state[b].passes);
+      r.rank = rank;
+      r.team = box.team > 1 ? box.team : 1;
+      r.pairs = a.dR2 != nullptr;
+    }
     __syncthreads();
     const LMEM BatchBox *sb = Lp(&sbS);
+    const LMEM BoxRun<T> *r = Lp(&runS);
     const int len = __builtin_amdgcn_readfirstlane(sb->molLen);
     const int nmols = __builtin_amdgcn_readfirstlane(sb->nmols);
-    const int team = __builtin_amdgcn_readfirstlane(sb->team > 1 ? sb->team : 1);
-    // Team members share the box's coordinates and centres.  Every member
-    // writes the same accepted values at the same point of a pass, after the
-    // exchange that needs all members' pair phases of that pass, and reads
-    // them only after its own write and a barrier: a read sees its own
-    // member's write or another's identical one.
-    const int64_t aoff = UniformI64(sb->atomOff);
-    const int64_t moff = UniformI64(sb->molOff);
-    const int64_t koff = UniformI64(sb->kOff);
-    const int64_t moves = UniformI64(a.moves[b]);
+    const int64_t moves = UniformI64(r->end - r->step);
     const bool ewald = __builtin_amdgcn_readfirstlane(sb->ewald) != 0;
-    // The box's molecule centres, rounded to FP32, live in LDS for the launch
-    // when they fit (a.ldsMols per workgroup): the cull reads them there.
     const bool inLds = nmols <= a.ldsMols;
-    BoxRun<T> r;
-    r.sb = sb;
-    r.st = Lp(&stS);
-    r.ms = Lp(&msS);
-    r.tab = Lp(tabS);
-    r.ctab = Lp(&ctabS);
-    r.queues = Lp(queuesS);
-    r.nearList = Lp(nearListS);
-    r.draws = Lp(drawsS);
-    r.CX = inLds ? Lp(ldsCom) : nullptr;
-    r.CY = r.CX + a.ldsMols;
-    r.CZ = r.CX + 2 * a.ldsMols;
-    r.X = Gp(a.x + aoff);
-    r.Y = Gp(a.y + aoff);
-    r.Z = Gp(a.z + aoff);
-    r.CXg = Gp(a.cx + moff);
-    r.CYg = Gp(a.cy + moff);
-    r.CZg = Gp(a.cz + moff);
-    r.kn = Gp(a.kn + koff);
-    r.pref = Gp(a.pref + koff);
-    r.sumR = Gp(a.sumR + koff);
-    r.sumI = Gp(a.sumI + koff);
-    r.delta = DeltaPtrs{{Gp(a.dR + koff), Gp(a.dR2 ? a.dR2 + koff : a.dR + koff)},
-                        {Gp(a.dI + koff), Gp(a.dI2 ? a.dI2 + koff : a.dI + koff)}};
-    r.xb = Gp(a.xchg + int64_t(b) * kXchgWords);
-    r.err = Gp(a.err);
-    r.trace = rank == 0 && b == a.trace.box ? &a.trace : nullptr;
-    r.step = UniformI64(a.state[b].step);
-    r.end = r.step + moves;
-    r.pass = uint64_t(UniformI64(a.state[b].passes));
-    r.rank = rank;
-    r.team = team;
-    r.pairs = a.dR2 != nullptr;
     const uint64_t t0 = wall_clock64();
     if (moves > 0) {
       if (inLds)
         for (int i = tid; i < nmols; i += kBatchThreads) {
-          Lp(ldsCom)[i] = float(r.CXg[i]);
-          Lp(ldsCom)[a.ldsMols + i] = float(r.CYg[i]);
-          Lp(ldsCom)[2 * a.ldsMols + i] = float(r.CZg[i]);
+          Lp(ldsCom)[i] = float(r->CXg[i]);
+          Lp(ldsCom)[a.ldsMols + i] = float(r->CYg[i]);
+          Lp(ldsCom)[2 * a.ldsMols + i] = float(r->CZg[i]);
         }
       if (PREC == 0 && sb->elect) {
         const GMEM TabPair *src = (const GMEM TabPair *)(a.coulTab + size_t(b) * kTabWords);
@@ -1321,18 +1327,21 @@ __global__ void __launch_bounds__(kBatchThreads) McBatchKernel(const BatchArgs a
       Cursor c;
       switch (len) {
         case 1:
-          c = RunBox<T, 1>(&r, wave);
+          c = RunBox<T, 1>(r, wave);
           break;
         case 2:
-          c = RunBox<T, 2>(&r, wave);
+          c = RunBox<T, 2>(r, wave);
           break;
         case 3:
-          c = RunBox<T, 3>(&r, wave);
+          c = RunBox<T, 3>(r, wave);
           break;
         default:
-          c = RunBox<T, 4>(&r, wave);
+          c = RunBox<T, 4>(r, wave);
       }
-      if (c.pend && ewald) RecipFold(sb, rank, team, r.kn, r.sumR, r.sumI, r.delta, c.pend);
+      if (c.pend && ewald) {
+        const BoxRun<T> &g = runS;
+        RecipFold(sb, rank, g.team, g.kn, g.sumR, g.sumI, g.delta, c.pend);
+      }
       if (tid == 0 && rank == 0) {
         stS.step = c.step;
         stS.passes = int64_t(c.pass);
