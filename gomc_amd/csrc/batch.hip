@@ -1252,7 +1252,21 @@ __global__ void __launch_bounds__(kBatchThreads) McBatchKernel(const BatchArgs a
     {
       const uint64_t *src = reinterpret_cast<const uint64_t *>(&a.boxes[b]);
       uint64_t *dst = reinterpret_cast<uint64_t *>(&sbS);
+      // the Coulomb table's loads run beside the description's
+      constexpr int kPer = (kTabWords / 2 + kBatchThreads - 1) / kBatchThreads;
+      TabPair row[kPer];
+      if (PREC == 0) {
+        const GMEM TabPair *t = (const GMEM TabPair *)(a.coulTab + size_t(a.boxes[b].tab) * kTabWords);
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) row[i] = t[min(tid + i * kBatchThreads, kTabWords / 2 - 1)];
+      }
       for (int i = tid; i < int(sizeof(BatchBox) / 8); i += kBatchThreads) dst[i] = src[i];
+      if (PREC == 0) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+          if (tid + i * kBatchThreads < kTabWords / 2)
+            ((LMEM TabPair *)Lp(ctabS.c))[tid + i * kBatchThreads] = row[i];
+      }
     }
     if (tid == 0) {
       msS.abort = 0;
@@ -1319,11 +1333,7 @@ __global__ void __launch_bounds__(kBatchThreads) McBatchKernel(const BatchArgs a
           Lp(ldsCom)[a.ldsMols + i] = float(r->CYg[i]);
           Lp(ldsCom)[2 * a.ldsMols + i] = float(r->CZg[i]);
         }
-      if (PREC == 0 && sb->elect) {
-        const GMEM TabPair *src = (const GMEM TabPair *)(a.coulTab + size_t(b) * kTabWords);
-        for (int i = tid; i < kTabWords / 2; i += kBatchThreads) ((LMEM TabPair *)Lp(ctabS.c))[i] = src[i];
-      }
-      // the table and centres are read after the programs' first barrier
+      // the centres are read after the programs' first barrier
       Cursor c;
       switch (len) {
         case 1:

@@ -66,7 +66,7 @@ struct BatchBox {
   int cull;  // 1: cull far molecules by their centres before atom pairs
   float nearCutSqF;  // (rc + 2 r_max + margin)^2: centres farther apart than this hold
                      // no pair inside the cutoff; the margin covers FP32 centres
-  int tabBase;       // of its Coulomb table
+  int tab, tabBase;  // its Coulomb table and that table's base
   int wide;          // 1: half of every edge exceeds the cutoff and the molecule's radius
   int team;  // workgroups running the box (1, 2, 4, 8)
   int live;  // bit p * kBatchMaxAtoms + q: atoms p, q interact (charge or LJ)
@@ -115,7 +115,7 @@ struct BatchArgs {
   double *sumR, *sumI;        // reference structure factors
   double *dR, *dI;            // structure-factor change of a pass's first move
   double *dR2, *dI2;          // and of its second; null: one move per pass
-  const double *coulTab;      // [nboxes][kTabWords] Coulomb tables (FP64)
+  const double *coulTab;      // [][kTabWords] Coulomb tables (FP64), at least one
   const int64_t *moves;       // [nboxes] moves to make in this launch
   int ldsMols;                // per-box centre capacity of dynamic LDS
   BatchTrace trace;
@@ -195,8 +195,10 @@ struct PackedBox {
 int PackBox(gomc_batch *bt, const gomc_system_desc &d, int64_t atomOff, int64_t molOff,
             int64_t kOff, PackedBox &out);
 // Device buffers for `nboxes` boxes and the given flat-array lengths; pairs:
-// with the second change of S(k) that passes of two moves need.
-int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec, bool pairs);
+// with the second change of S(k) that passes of two moves need; room for this
+// many Coulomb tables (FP64).
+int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec, bool pairs,
+               int tables);
 // Team size of a box of n molecules (a function of n alone, so a box's
 // results do not depend on the other boxes of its batch).
 int TeamSize(const gomc_batch *bt, int nmols);

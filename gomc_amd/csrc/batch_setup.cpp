@@ -273,7 +273,7 @@ BatchArgs MakeArgs(const gomc_batch *bt) {
 }
 
 int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t kvec,
-               bool pairs) {
+               bool pairs, int tables) {
   BHIP(bt, hipSetDevice(bt->device));
   auto alloc = [&](void **p, size_t bytes) { return hipMalloc(p, std::max<size_t>(bytes, 8)) == hipSuccess; };
   bool ok = hipStreamCreateWithFlags(&bt->stream, hipStreamNonBlocking) == hipSuccess;
@@ -299,7 +299,7 @@ int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t 
     ok &= alloc((void **)&bt->dI2, sizeof(double) * kvec);
   }
   if (bt->precision == 0)
-    ok &= alloc((void **)&bt->coulTab, sizeof(double) * kTabWords * size_t(nboxes));
+    ok &= alloc((void **)&bt->coulTab, sizeof(double) * kTabWords * size_t(std::max(tables, 1)));
   // one workgroup per compute unit: the kernel's 1024 threads at 128
   // registers fill a CU, and team members must all be resident at once
   int cus = 0;
@@ -347,7 +347,7 @@ int UploadBox(gomc_batch *bt, int slot, const PackedBox &pb) {
     BHIP(bt, up(bt->cz + mo, pb.cz.data(), sizeof(double) * pb.cz.size()));
   }
   if (pb.table)
-    BHIP(bt, up(bt->coulTab + size_t(slot) * kTabWords, pb.table->c.data(), sizeof(double) * kTabWords));
+    BHIP(bt, up(bt->coulTab + size_t(P.tab) * kTabWords, pb.table->c.data(), sizeof(double) * kTabWords));
   BHIP(bt, up(bt->kn + P.kOff, pb.kn.data(), sizeof(int32_t) * pb.kn.size()));
   BHIP(bt, up(bt->pref + P.kOff, pb.pref.data(), sizeof(double) * pb.pref.size()));
   BHIP(bt, up(bt->sumR + P.kOff, pb.sr.data(), sizeof(double) * pb.sr.size()));
@@ -566,7 +566,19 @@ int gomc_batch_create_tuned(const gomc_system_desc *descs, int nboxes, int devic
     for (auto &pb : packed) teams = teams || pb.P.team > 1;
     if (teams && int64_t(perCU) * cus < gridCap) return fail(GOMC_ERR_STATE);
   }
-  int rc = AllocBatch(bt, nboxes, atoms, mols, kvec, true);
+  // boxes of one alpha and cutoff share a Coulomb table
+  std::vector<const CoulTable *> tables;
+  for (auto &pb : packed) {
+    const CoulTable *t = pb.table.get();
+    if (!t) continue;
+    const auto at = std::find(tables.begin(), tables.end(), t);
+    pb.P.tab = int(at - tables.begin());
+    if (at == tables.end())
+      tables.push_back(t);
+    else
+      pb.table.reset();  // uploaded with the first of them
+  }
+  int rc = AllocBatch(bt, nboxes, atoms, mols, kvec, true, int(tables.size()));
   if (rc) return fail(rc);
   bt->hboxes.resize(nboxes);
   for (int i = 0; i < nboxes; ++i) {

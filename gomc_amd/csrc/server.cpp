@@ -210,6 +210,7 @@ void Admit(gomc_server *sv, std::unique_lock<std::mutex> &lk) {
     j->pb.P.atomOff = a;
     j->pb.P.molOff = m;
     j->pb.P.kOff = k;
+    j->pb.P.tab = slot;
     sv->slotJob[slot] = j;
     sv->bytesUsed += JobBytes(*j);
     sv->bytesPeak = std::max(sv->bytesPeak, sv->bytesUsed);
@@ -534,7 +535,7 @@ int gomc_server_create(int device, int precision, int slots, int64_t budget_byte
   // passes of two moves keep 16 more bytes a k-vector slot: where the budget
   // has room for them beside the arenas
   const bool pairs = arena + 16.0 * double(sv->kCap) <= double(budget_bytes);
-  int rc = AllocBatch(bt, slots, sv->atomCap, sv->molCap, sv->kCap, pairs);
+  int rc = AllocBatch(bt, slots, sv->atomCap, sv->molCap, sv->kCap, pairs, slots);
   if (!rc) {
     std::vector<BatchState> zs(slots);
     std::memset(zs.data(), 0, sizeof(BatchState) * slots);
