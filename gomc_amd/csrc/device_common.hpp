@@ -233,13 +233,24 @@ __device__ __forceinline__ double ExpNeg(Coefs c, double y) {
   return ldexp(p, int(n));
 }
 
+// sigma^2 / d2 to the last place from ir = 1 / sqrt(d2): powers of it multiply
+// its error, so one correction is spent on it rather than on 1 / d2.
+__device__ __forceinline__ double LJRatio(double sigmaSq, double d2, double ir) {
+  const double ir2 = ir * ir, x = sigmaSq * ir2;
+  return fma(fma(-d2, x, sigmaSq), ir2, x);
+}
+
+// The Mie repulsion for exponents other than 12, out of line where its
+// registers would weigh on a pair loop.
+static __device__ __noinline__ double PowOutOfLine(double x, double h) { return pow(x, h); }
+
 // Pair terms at precision P (FFParticle::CalcEn / CalcCoulomb,
 // src/FFParticle.cpp:295-399).  FP64: one reciprocal square root (a
-// Newton-refined estimate, then one correction each for r and 1 / r^2, to the
-// last place) stands for the root and the divisions, e^-x^2 and erfcx are
-// polynomials whose coefficients are scalar operands, and nothing is called:
-// a call would save and restore the registers of the pair loops.  LIBM: libm's
-// erfc, whose error is a tenth of the polynomial's 3e-15.
+// Newton-refined estimate, then one correction each for r and sigma^2 / r^2, to
+// the last place) stands for the root and the divisions, e^-x^2 and erfcx are
+// polynomials whose coefficients are scalar operands, and for the exponent 12
+// nothing is called: a call would save and restore the registers of the pair
+// loops.  LIBM: libm's erfc, whose error is a tenth of the polynomial's 3e-15.
 template <int P, bool LIBM = false>
 __device__ __forceinline__ void PairTermsDev(const BoxGeom &g, Coefs cf, double d2, double qiqj,
                                              double sigmaSq, double epsCn, double nHalf,
@@ -253,8 +264,6 @@ __device__ __forceinline__ void PairTermsDev(const BoxGeom &g, Coefs cf, double 
   }
   d2 = fmax(d2, 0x1p-1022);  // coincident atoms: huge, not 0 x inf
   const double ir = Rsqrt64(d2);
-  double ir2 = ir * ir;
-  ir2 = fma(ir2, fma(-d2, ir2, 1.0), ir2);
   if (coul) {
     double e = qiqj * ir;
     if (LIBM && g.ewald) {
@@ -279,10 +288,10 @@ __device__ __forceinline__ void PairTermsDev(const BoxGeom &g, Coefs cf, double 
     real += sign * e;
   }
   if (inLJ) {
-    const double rRat2 = sigmaSq * ir2;
+    const double rRat2 = LJRatio(sigmaSq, d2, ir);
     const double att = rRat2 * rRat2 * rRat2;
     double rep = att * att;
-    if (nHalf != 6.0) rep = MiePow(rRat2, nHalf);
+    if (nHalf != 6.0) rep = LIBM ? pow(rRat2, nHalf) : PowOutOfLine(rRat2, nHalf);
     lj += sign * (epsCn * (rep - att));
   }
 }
