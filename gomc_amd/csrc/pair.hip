@@ -185,45 +185,53 @@ struct PairTerms {
 // Energies and virial factors F.r / r^2 of one pair inside the box cutoff
 // (FFParticle::CalcCoulomb / CalcCoulombVir, src/FFParticle.cpp:387-446,
 // CalcEn / CalcVir 295-359): one reciprocal square root (a Newton-refined
-// estimate, then one correction each for r and 1 / r^2, to the last place)
+// estimate, then corrections for r, sigma^2 / r^2 and 1 / r^2, to the last place)
 // stands for every root and division, and one exponential for erfc's and the
-// virial's Gaussian.
+// virial's Gaussian.  The energy alone takes libm's erfc and pow: the
+// polynomial is 4e-16 too small in the mean, which a sum over all pairs keeps
+// (Coulomb energy of 300 to 2197 waters within 3e-16 of 64-bit sums, by the
+// polynomial within 4e-15).
 template <bool E, bool F, bool MIE>  // MIE: some repulsion exponent is not 12
 __device__ __forceinline__ PairTerms PairEval(const BoxGeom &g, Coefs c, double d2, double qiqj,
                                               const PairType &t) {
+  constexpr bool libm = E && !F;
   PairTerms p{0.0, 0.0, 0.0, 0.0};
   d2 = fmax(d2, 0x1p-1022);  // coincident atoms: huge, not 0 x inf
   const double ir = Rsqrt64(d2);
   double ir2 = ir * ir;
-  ir2 = fma(ir2, fma(-d2, ir2, 1.0), ir2);
+  if (F) ir2 = fma(ir2, fma(-d2, ir2, 1.0), ir2);
   if (g.elect && qiqj != 0.0 && !(g.rCutCoulSq < d2)) {
     if (g.ewald) {
       double dist = d2 * ir;
       dist = fma(fma(-dist, dist, d2), 0.5 * ir, dist);
       const double x = g.alpha * dist;
-      const double gauss = ExpNeg(c, -(x * x));
-      double ex;
-      if (x <= kErfcxUse) {
-        const double u = (x - kErfcxMid) * kErfcxInvHalf;
-        ex = c[kExpDeg + 1];
-#pragma unroll
-        for (int k = 1; k <= kErfcxDeg; ++k) ex = FmaS(ex, u, c[kExpDeg + 1 + k]);
+      if (libm) {
+        p.eReal = qiqj * (erfc(x) * ir);
       } else {
-        ex = ErfcxTail(x);
+        const double gauss = ExpNeg(c, -(x * x));
+        double ex;
+        if (x <= kErfcxUse) {
+          const double u = (x - kErfcxMid) * kErfcxInvHalf;
+          ex = c[kExpDeg + 1];
+#pragma unroll
+          for (int k = 1; k <= kErfcxDeg; ++k) ex = FmaS(ex, u, c[kExpDeg + 1 + k]);
+        } else {
+          ex = ErfcxTail(x);
+        }
+        const double ec = gauss * ex * ir;
+        if (E) p.eReal = qiqj * ec;
+        p.vReal = qiqj * (ec + g.alpha * M_2_SQRTPI * gauss) * ir2;
       }
-      const double ec = gauss * ex * ir;
-      if (E) p.eReal = qiqj * ec;
-      if (F) p.vReal = qiqj * (ec + g.alpha * M_2_SQRTPI * gauss) * ir2;
     } else {
       if (E) p.eReal = qiqj * ir;
       if (F) p.vReal = qiqj * (ir2 * ir);
     }
   }
   if (t.eps6 != 0.0 && !(g.rCutLJSq < d2)) {
-    const double rRat2 = t.sig * ir2;
+    const double rRat2 = E ? LJRatio(t.sig, d2, ir) : t.sig * ir2;
     const double att = rRat2 * rRat2 * rRat2;
     double rep = att * att;
-    if (MIE && t.nh != 6.0) rep = MiePow(rRat2, t.nh);
+    if (MIE && t.nh != 6.0) rep = libm ? pow(rRat2, t.nh) : MiePow(rRat2, t.nh);
     if (E) p.eLJ = t.eps * (rep - att);
     if (F) p.vLJ = t.eps6 * (t.nov6 * rep - att) * ir2;
   }
