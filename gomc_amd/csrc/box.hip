@@ -112,10 +112,15 @@ __device__ __forceinline__ void TrialAtom(const TrialArgs &a, int j, double xj, 
 // in one thread are six pair terms or sincos in a row.
 constexpr int kTrialK = kBlock / 2;  // k-vectors of a block's run
 // A block takes as many runs as keep the reciprocal blocks to this: each block
-// costs the last one's counter and sums a little, and from 16384 k-vectors on
-// that outweighs the shorter chain (8000 waters, 25,000 k-vectors, mixed: call
-// 35.2 us with one run a block, as before the split; 33.4 with two).
-constexpr int kTrialRecipBlocks = 128;
+// costs the last one's counter and sums about 17 ns, each more run a block a
+// chain of one sincos an atom, 0.5 us for one atom, 1.4 for three, 2.9 for
+// eight.  Microseconds a call with at most 128 / 256 / 512 / any number of
+// blocks (one thread a k-vector and any number of blocks: last), FP64:
+// 3 atoms, 43,500 k-vectors 34.6 / 33.6 / 36.1 / 36.2 (35.8), 226,500 50.2 /
+// 43.2 / 43.9 / 70.9 (49.8); 8 atoms, 94,100 49.1 / 42.8 / 42.6 / 48.0 (46.1),
+// 226,500 72.9 / 55.1 / 52.4 / 73.8 (58.0); 16 atoms, 94,100 64.1 / 51.3 / 49.0
+// / 53.1 (56.2), 226,500 108 / 73.8 / 67.3 / 82.3 (60.1).
+constexpr int TrialRecipBlocks(int atoms) { return atoms <= 4 ? 256 : 512; }
 template <int P>
 __global__ void __launch_bounds__(kBlock) TrialKernel(const TrialArgs a) {
   __shared__ double red[kBlock / kWave][4];
@@ -712,7 +717,8 @@ int LaunchTrial(gomc_box *b, int m, const double *ox, const double *oy, const do
   a.doPair = doPair;
   a.doRecip = doRecip && b->ewald;
   const int runs = (b->K + kTrialK - 1) / kTrialK;
-  a.kRuns = std::max(1, (runs + kTrialRecipBlocks - 1) / kTrialRecipBlocks);
+  const int most = TrialRecipBlocks(len);
+  a.kRuns = std::max(1, (runs + most - 1) / most);
   const int nRecip = a.doRecip ? (runs + a.kRuns - 1) / a.kRuns : 0;
   a.K = b->K;
   a.kx = b->kx;
