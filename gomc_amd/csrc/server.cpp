@@ -86,6 +86,7 @@ constexpr int kGcmcBuilders = 4;  // threads building GCMC jobs' device boxes
 constexpr int64_t kAtomBytes = 3 * sizeof(double);                          // x, y, z
 constexpr int64_t kMolBytes = 3 * sizeof(double);                           // centres
 constexpr int64_t kKBytes = sizeof(int32_t) + 5 * sizeof(double);           // kn, pref, S, dS
+constexpr int64_t kPairBytes = 2 * sizeof(double);  // a pass's second dS, where it fits
 
 // A descriptor deep-copied at submission, for jobs that are built later
 // (the caller's arrays may be gone by then).
@@ -152,6 +153,7 @@ struct gomc_server {
   int device = 0, precision = 0, nslots = 0;
   double tickMs = 20.0;
   int64_t budget = 0, atomCap = 0, molCap = 0, kCap = 0, bytesUsed = 0, bytesPeak = 0;
+  int64_t slotBytes = kKBytes;  // of a k-vector slot
   gomc_batch *bt = nullptr;
   Arena atoms, mols, kvec;
   std::mutex mu;
@@ -178,8 +180,8 @@ struct gomc_server {
 
 namespace {
 
-int64_t JobBytes(const Job &j) {
-  return j.pb.P.natoms * kAtomBytes + j.pb.P.nmols * kMolBytes + int64_t(j.pb.P.K) * kKBytes;
+int64_t JobBytes(const gomc_server *sv, const Job &j) {
+  return j.pb.P.natoms * kAtomBytes + j.pb.P.nmols * kMolBytes + int64_t(j.pb.P.K) * sv->slotBytes;
 }
 
 // Admits queued jobs in arrival order while a slot and memory are free.
@@ -212,7 +214,7 @@ void Admit(gomc_server *sv, std::unique_lock<std::mutex> &lk) {
     j->pb.P.kOff = k;
     j->pb.P.tab = slot;
     sv->slotJob[slot] = j;
-    sv->bytesUsed += JobBytes(*j);
+    sv->bytesUsed += JobBytes(sv, *j);
     sv->bytesPeak = std::max(sv->bytesPeak, sv->bytesUsed);
     lk.unlock();
     int rc = UploadBox(sv->bt, slot, j->pb);
@@ -280,7 +282,7 @@ void Loop(gomc_server *sv) {
           sv->atoms.Release(j->atomOff, j->pb.P.natoms);
           sv->mols.Release(j->molOff, j->pb.P.nmols);
           sv->kvec.Release(j->kOff, j->pb.P.K);
-          sv->bytesUsed -= JobBytes(*j);
+          sv->bytesUsed -= JobBytes(sv, *j);
           sv->slotJob[s] = nullptr;
           --sv->outstanding;
         }
@@ -303,7 +305,7 @@ void Loop(gomc_server *sv) {
       sv->atoms.Release(j->atomOff, j->pb.P.natoms);
       sv->mols.Release(j->molOff, j->pb.P.nmols);
       sv->kvec.Release(j->kOff, j->pb.P.K);
-      sv->bytesUsed -= JobBytes(*j);
+      sv->bytesUsed -= JobBytes(sv, *j);
       sv->slotJob[s] = nullptr;
       // an empty slot makes no moves and reads nothing
       BatchBox empty;
@@ -534,7 +536,8 @@ int gomc_server_create(int device, int precision, int slots, int64_t budget_byte
   std::memset(bt->hboxes.data(), 0, sizeof(BatchBox) * slots);
   // passes of two moves keep 16 more bytes a k-vector slot: where the budget
   // has room for them beside the arenas
-  const bool pairs = arena + 16.0 * double(sv->kCap) <= double(budget_bytes);
+  const bool pairs = arena + double(kPairBytes) * double(sv->kCap) <= double(budget_bytes);
+  if (pairs) sv->slotBytes += kPairBytes;
   int rc = AllocBatch(bt, slots, sv->atomCap, sv->molCap, sv->kCap, pairs, slots);
   if (!rc) {
     std::vector<BatchState> zs(slots);

@@ -408,7 +408,9 @@ int gomc_batch_last_kernel_ms(const gomc_batch *bt, double *ms);
  * workgroup slots; submitted jobs (NVT boxes as for gomc_batch_create) are
  * admitted in arrival order when a slot is free and their coordinates,
  * centres, k-vectors and structure factors fit the `budget_bytes` device
- * arenas (the NVT lane's arenas take the budget up to 64 MiB per slot);
+ * arenas (the NVT lane's arenas take the budget up to 64 MiB per slot; a
+ * slot's description and, in FP64, its Coulomb table, 38 KB in all, come
+ * beside the budget);
  * every launch advances each resident job by the moves that cost about
  * `tick_ms`; finished jobs release their slot and memory.  A job's result
  * does not depend on the other jobs in the batch. */

@@ -1,0 +1,33 @@
+"""The memory a server reports for its jobs covers what it keeps for them: every
+array of a k-vector slot, the second change of S(k) included where the budget has
+room for passes of two moves.
+"""
+import pytest
+
+from gomc_amd import systems
+from gomc_amd.api import Batch, Box
+from gomc_amd.serve import Server
+
+pytestmark = pytest.mark.gpu
+
+# kn 4 bytes; pref, S(k) and its change 40; a pass's second change 16
+SLOT, PAIRS = 44, 16
+
+
+@pytest.mark.parametrize("budget,pairs", [(64 << 20, False), (96 << 20, True)])
+def test_peak_covers_a_job(budget, pairs):
+    s = systems.water_box(300, seed=2)
+    b = Box(s)
+    width = 256 if b.nkvec <= 3072 else 512
+    b.close()
+    bt = Batch([s], tuning="default")
+    lay = bt.layout(0)
+    bt.close()
+    need = 24 * s.natoms + 24 * s.nmols + \
+        lay["kseg"] * lay["rounds"] * width * (SLOT + (PAIRS if pairs else 0))
+    sv = Server(slots=1, budget_bytes=budget, tick_ms=2.0)
+    sv.submit(s, 200)
+    sv.drain(60)
+    peak = sv.stats()["peak_bytes"]
+    sv.close()
+    assert peak == need
