@@ -319,8 +319,10 @@ void Loop(gomc_server *sv) {
 }
 
 // Device bytes of a GCMC job on the plain path: coordinates, charges,
-// kinds, cell list, forces are not built; k-vector arrays (index triple,
-// prefactor, two structure-factor pairs) and per-molecule data.
+// kinds, cell list, forces are not built; k-vector arrays (components and
+// prefactor, two structure-factor pairs: 64 bytes; the device loop's pairs of
+// k-vectors: 8 structure-factor values, prefactor, index triple and two places
+// a pair, 42 bytes a k-vector) and per-molecule data.
 int64_t GcmcBytes(const gomc_system_desc &d) {
   int64_t natoms = 0;
   for (int m = 0; m < d.n_mols; ++m) natoms += d.kind_natoms[d.mol_kind[m]];
@@ -330,7 +332,7 @@ int64_t GcmcBytes(const gomc_system_desc &d) {
   // k-vectors in the half sphere |k| < kc: (2/3) pi (kc L / 2 pi)^3
   double kv = 2.0 / 3.0 * M_PI;
   for (int i = 0; i < 3; ++i) kv *= kc * d.box[i] / (2.0 * M_PI);
-  return natoms * 96 + int64_t(d.n_mols) * 64 + int64_t(kv) * 64 + (int64_t(1) << 20);
+  return natoms * 96 + int64_t(d.n_mols) * 64 + int64_t(kv) * 106 + (int64_t(1) << 20);
 }
 
 // Builder of the GCMC lane: takes queued GCMC jobs in arrival order while

@@ -31,3 +31,18 @@ def test_peak_covers_a_job(budget, pairs):
     peak = sv.stats()["peak_bytes"]
     sv.close()
     assert peak == need
+
+
+def test_peak_covers_a_gcmc_job():
+    """Its k-vector arrays, the device loop's among them, and its coordinates."""
+    s = systems.gcmc_mixture(5, 5, 75.0, fugacity_bar=(1e-3, 1e-3), reservoir=40, seed=3)
+    b = Box(s)
+    need = b.nkvec * (4 * 8 + 4 * 8 + (8 * 8 + 8 + 3 * 4) // 2) + s.natoms * 24
+    b.close()
+    assert need > 4 << 20
+    sv = Server(slots=1, budget_bytes=256 << 20, tick_ms=2.0)
+    sv.submit(s, 50)
+    sv.drain(60)
+    peak = sv.stats()["peak_bytes"]
+    sv.close()
+    assert need <= peak <= 1.5 * need
