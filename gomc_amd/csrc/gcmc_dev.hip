@@ -1920,61 +1920,71 @@ int DevCheck(gomc_box *b) {
   return GOMC_OK;
 }
 
+// What a box's device move loop keeps from its k-vectors and kinds.
+int DevCreate(gomc_box *b) {
+  b->dev = new DevDriver();
+  DevDriver *d = b->dev;
+  HIP_TRY(b, hipMalloc(&d->state, sizeof(DevState)));
+  HIP_TRY(b, hipMalloc(&d->molKind, sizeof(int) * std::max(1, b->nmols)));
+  HIP_TRY(b, hipMalloc(&d->molBox, sizeof(int) * std::max(1, b->nmols)));
+  HIP_TRY(b, hipMalloc(&d->com, sizeof(double) * 3 * std::max(1, b->nmols)));
+  HIP_TRY(b, hipMalloc(&d->xchg, sizeof(uint64_t) * kDevXchgWords));
+  HIP_TRY(b, hipMemcpy(d->molKind, b->molKind.data(), sizeof(int) * b->nmols, hipMemcpyHostToDevice));
+  // index triples of the box's k-vectors, in their order
+  std::vector<double> kx, ky, kz, pref;
+  std::vector<int32_t> packed;
+  KVectorsOrth(b->geom.L, b->alpha * b->alpha, b->recipRcut, b->volume, kx, ky, kz, pref, &packed);
+  if (b->ewald && int(packed.size()) != b->K)
+    return Fail(b, GOMC_ERR_STATE, "device move loop: k-vector count mismatch");
+  for (int32_t code : packed) {
+    d->nmax[0] = std::max(d->nmax[0], code & 0xff);
+    d->nmax[1] = std::max(d->nmax[1], std::abs(((code >> 8) & 0xff) - 128));
+    d->nmax[2] = std::max(d->nmax[2], std::abs(((code >> 16) & 0xff) - 128));
+  }
+  if (d->nmax[0] > kDevNMax || d->nmax[1] > kDevNMax || d->nmax[2] > kDevNMax)
+    return Fail(b, GOMC_ERR_ARG, "device move loop: more than 40 k-vectors per axis");
+  // each with its mirror in z, where the half space holds that too
+  std::vector<int32_t> code, first, second;
+  std::vector<double> kpref;
+  code.reserve(packed.size());
+  first.reserve(packed.size());
+  second.reserve(packed.size());
+  kpref.reserve(packed.size());
+  for (size_t k = 0; k < packed.size(); ++k) {
+    const int nz = ((packed[k] >> 16) & 0xff) - 128;
+    // the k-vectors of one (nx, ny) stand in rising nz
+    const int64_t m = int64_t(k) - 2 * nz;
+    const int other = m >= 0 && m < int64_t(packed.size()) &&
+                              packed[m] == ((packed[k] & 0xffff) | ((128 - nz) << 16))
+                          ? int(m)
+                          : int(k);
+    if (nz < 0 && other != int(k)) continue;  // listed with its mirror
+    code.push_back(packed[k] | (other == int(k) ? INT32_MIN : 0));
+    kpref.push_back(pref[k]);
+    first.push_back(int(k));
+    second.push_back(other);
+  }
+  d->npairs = int(code.size());
+  HIP_TRY(b, hipMalloc(&d->kbuf, sizeof(double) * std::max<size_t>(1, 8 * code.size())));
+  HIP_TRY(b, hipMalloc(&d->kpref, sizeof(double) * std::max<size_t>(1, kpref.size())));
+  if (!kpref.empty())
+    HIP_TRY(b, hipMemcpy(d->kpref, kpref.data(), sizeof(double) * kpref.size(), hipMemcpyHostToDevice));
+  for (auto [dst, src] : {std::pair<int32_t **, std::vector<int32_t> *>{&d->kcode, &code},
+                          {&d->kfirst, &first},
+                          {&d->ksecond, &second}}) {
+    HIP_TRY(b, hipMalloc(dst, sizeof(int32_t) * std::max<size_t>(1, src->size())));
+    if (!src->empty())
+      HIP_TRY(b, hipMemcpy(*dst, src->data(), sizeof(int32_t) * src->size(), hipMemcpyHostToDevice));
+  }
+  return GOMC_OK;
+}
+
 int DevEnsure(gomc_box *b, int64_t traceMoves) {
   if (!b->dev) {
-    b->dev = new DevDriver();
-    DevDriver *d = b->dev;
-    HIP_TRY(b, hipMalloc(&d->state, sizeof(DevState)));
-    HIP_TRY(b, hipMalloc(&d->molKind, sizeof(int) * std::max(1, b->nmols)));
-    HIP_TRY(b, hipMalloc(&d->molBox, sizeof(int) * std::max(1, b->nmols)));
-    HIP_TRY(b, hipMalloc(&d->com, sizeof(double) * 3 * std::max(1, b->nmols)));
-    HIP_TRY(b, hipMalloc(&d->xchg, sizeof(uint64_t) * kDevXchgWords));
-    HIP_TRY(b, hipMemcpy(d->molKind, b->molKind.data(), sizeof(int) * b->nmols, hipMemcpyHostToDevice));
-    // index triples of the box's k-vectors, in their order
-    std::vector<double> kx, ky, kz, pref;
-    std::vector<int32_t> packed;
-    KVectorsOrth(b->geom.L, b->alpha * b->alpha, b->recipRcut, b->volume, kx, ky, kz, pref, &packed);
-    if (b->ewald && int(packed.size()) != b->K)
-      return Fail(b, GOMC_ERR_STATE, "device move loop: k-vector count mismatch");
-    for (int32_t code : packed) {
-      d->nmax[0] = std::max(d->nmax[0], code & 0xff);
-      d->nmax[1] = std::max(d->nmax[1], std::abs(((code >> 8) & 0xff) - 128));
-      d->nmax[2] = std::max(d->nmax[2], std::abs(((code >> 16) & 0xff) - 128));
-    }
-    if (d->nmax[0] > kDevNMax || d->nmax[1] > kDevNMax || d->nmax[2] > kDevNMax)
-      return Fail(b, GOMC_ERR_ARG, "device move loop: more than 40 k-vectors per axis");
-    // each with its mirror in z, where the half space holds that too
-    std::vector<int32_t> code, first, second;
-    std::vector<double> kpref;
-    code.reserve(packed.size());
-    first.reserve(packed.size());
-    second.reserve(packed.size());
-    kpref.reserve(packed.size());
-    for (size_t k = 0; k < packed.size(); ++k) {
-      const int nz = ((packed[k] >> 16) & 0xff) - 128;
-      // the k-vectors of one (nx, ny) stand in rising nz
-      const int64_t m = int64_t(k) - 2 * nz;
-      const int other = m >= 0 && m < int64_t(packed.size()) &&
-                                packed[m] == ((packed[k] & 0xffff) | ((128 - nz) << 16))
-                            ? int(m)
-                            : int(k);
-      if (nz < 0 && other != int(k)) continue;  // listed with its mirror
-      code.push_back(packed[k] | (other == int(k) ? INT32_MIN : 0));
-      kpref.push_back(pref[k]);
-      first.push_back(int(k));
-      second.push_back(other);
-    }
-    d->npairs = int(code.size());
-    HIP_TRY(b, hipMalloc(&d->kbuf, sizeof(double) * std::max<size_t>(1, 8 * code.size())));
-    HIP_TRY(b, hipMalloc(&d->kpref, sizeof(double) * std::max<size_t>(1, kpref.size())));
-    if (!kpref.empty())
-      HIP_TRY(b, hipMemcpy(d->kpref, kpref.data(), sizeof(double) * kpref.size(), hipMemcpyHostToDevice));
-    for (auto [dst, src] : {std::pair<int32_t **, std::vector<int32_t> *>{&d->kcode, &code},
-                            {&d->kfirst, &first},
-                            {&d->ksecond, &second}}) {
-      HIP_TRY(b, hipMalloc(dst, sizeof(int32_t) * std::max<size_t>(1, src->size())));
-      if (!src->empty())
-        HIP_TRY(b, hipMemcpy(*dst, src->data(), sizeof(int32_t) * src->size(), hipMemcpyHostToDevice));
+    const int rc = DevCreate(b);
+    if (rc) {  // a later call must not find it half made
+      DevFree(b);
+      return rc;
     }
   }
   DevDriver *d = b->dev;
