@@ -530,6 +530,7 @@ int EnsurePartials(gomc_box *b, int nblocks) {
   if (nblocks <= b->maxPartials) return GOMC_OK;
   if (b->partials) (void)hipFree(b->partials);
   b->partials = nullptr;
+  b->maxPartials = 0;
   int n = std::max(nblocks, 1024);
   HIP_TRY(b, hipMalloc(&b->partials, sizeof(Partial4) * n));
   b->maxPartials = n;
