@@ -21,10 +21,11 @@
 // every sum is fixed by the positions.  Energies and virials: the partner
 // must come later in the cell order, so each pair is met once.
 //
-// Bound by FP64 issue and, at four waves a SIMD, the tail of the last round.
-// 10,000 waters, rc 12 A: forces 336 us (with atom cells, tiles and sorted
-// hit lists 733), virial 170 us (606), energy 173 us (950); 1000 waters, rc
-// 10 A: forces 64 us (154).
+// Bound by FP64 issue and the tail of the last round of home molecules (128
+// VGPRs, four waves a SIMD, of which three are there on average).
+// 10,000 waters, rc 12 A: forces 333 us (with atom cells, tiles and sorted
+// hit lists 733), virial 166 us (606), energy 185 us (950); 1000 waters, rc
+// 10 A: forces 62 us (154).
 #include <algorithm>
 #include <cmath>
 

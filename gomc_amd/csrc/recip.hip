@@ -104,7 +104,7 @@ struct SumsArgs {
 // against up to 8 MFMAs).  A tile is padded to whole steps of 4 atoms by
 // charge 0.  Bound by the matrix cores and the table builds between them:
 // 10,000 waters (30,000 atoms, K = 30,902, 5.8 GFLOP with the padding of
-// 16-column, 8-nz tiles) 168 us, 34 TFLOP/s; 620 us as one rotating phase
+// 16-column, 8-nz tiles) 159 us, 36 TFLOP/s; 620 us as one rotating phase
 // per (atom, k-vector) on the vector units.
 template <bool direct>  // no x and y tables: a very long box
 __global__ void __launch_bounds__(kMmThreads, 4) RecipSumsPartKernel(const SumsArgs a) {
@@ -312,9 +312,9 @@ struct ForceArgs {
 // sorted by length, so the waves' shares are alike).  B operands, the z
 // phases of the atoms, and the x and y phases sit in LDS; an A operand is
 // one 8-byte read per lane for NT MFMAs.  Bound by the matrix cores on a
-// large box: 10,000 waters (8.3 GFLOP with the padding) 187 us, 45 TFLOP/s;
+// large box: 188 us on 10,000 waters (8.3 GFLOP with the padding), 44 TFLOP/s;
 // 635 us as six multiply-adds and a complex product per (atom, k-vector) on
-// the vector units.  1000 waters 10.7 us, before 16.4.
+// the vector units.  1000 waters 9.8 us, before 16.4.
 template <int NT, bool XY>  // XY: x and y phases from tables
 __global__ void __launch_bounds__(kMmThreads, 4) RecipForcePartKernel(const ForceArgs a) {
   constexpr int A = 16 * NT;
@@ -509,11 +509,11 @@ void FreeKPlan(KPlan &p) {
 }
 
 // ------------------------------------------------------ structure factors --
-constexpr int kSumsTabBytes = 48 * 1024;  // phase tables of a tile: three workgroups a CU
-constexpr int kSumsWorkgroups = 512;      // two a CU
+constexpr int kSumsTabBytes = 48 * 1024;  // phase tables of a tile
+constexpr int kSumsWorkgroups = 512;      // two a CU, what their registers allow
 
 // Atom chunks of the first pass: about kSumsWorkgroups workgroups, chunks of
-// at least 32 atoms, chunks x K within kSumsPartCap doubles / 2.
+// at least 32 atoms, chunks x K within kSumsPartCap (pairs of doubles).
 static int SumsChunks(const gomc_box *b) {
   int c = (kSumsWorkgroups + b->kp.nB - 1) / std::max(1, b->kp.nB);
   c = std::min(c, (b->natoms + 31) / 32);
@@ -675,8 +675,15 @@ int RecipSumsNoAlloc(gomc_box *b, double *erecip) {
 
 // ------------------------------------------------------------------ force --
 constexpr int kForceWorkgroups = 512;    // two a CU
-constexpr int kForceTabBytes = 76 * 1024;  // their tables: two workgroups a CU
 constexpr int kForceZMax = 32;           // steps of a z window when the tables do not fit
+// Tables of a workgroup of 16 nt atoms that leave room for a second one on the
+// CU (160 KiB, less the static part).  Measured on cubic water boxes, rc 12 A,
+// tolerance 1e-6, microseconds a call with this limit and with 6 KiB more, where
+// 64 atoms run alone on a CU instead of 32 and 32 at n = 22 to 24 k-vectors an
+// axis: n = 21 113.6 / 113.3, 22 143.0 / 167.2, 23 191.1 / 190.0, 24 215.8 /
+// 205.8; 64 atoms alone also at 25 275 / 314, 26 309 / 345, 28 430 / 418, 32 901 /
+// 974.
+constexpr int ForceTabBytes(int nt) { return 80 * 1024 - int(sizeof(double)) * kMmWaves * 3 * 16 * nt; }
 
 // The k-space force of every atom over the sums (sumR, sumI), as per-chunk
 // parts; launched on the box's stream, not waited for.
@@ -729,9 +736,9 @@ int RecipForceParts(gomc_box *b, const double *sumR, const double *sumI, RecipPa
            size_t(4) * a.zSteps * A * sizeof(double);
   };
   int nt = 4;
-  while (nt > 1 && bytes(16 * nt) > size_t(kForceTabBytes)) nt /= 2;
-  if (bytes(16 * nt) > size_t(kForceTabBytes)) a.zSteps = std::min(a.zSteps, kForceZMax);
-  if (bytes(16 * nt) > size_t(kForceTabBytes)) xy = false;
+  while (nt > 1 && bytes(16 * nt) > size_t(ForceTabBytes(nt))) nt /= 2;
+  if (bytes(16 * nt) > size_t(ForceTabBytes(nt))) a.zSteps = std::min(a.zSteps, kForceZMax);
+  if (bytes(16 * nt) > size_t(ForceTabBytes(nt))) xy = false;
   const int blocks = (b->natoms + 16 * nt - 1) / (16 * nt);
   const int most = std::max(1, (p.ngrp + kMmWaves - 1) / kMmWaves);
   a.chunks = std::max(1, std::min(most, (kForceWorkgroups + blocks / 2) / std::max(1, blocks)));
