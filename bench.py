@@ -40,10 +40,11 @@ METRIC = ("MC trial moves/s (1 GPU), batched+served vs plain at ≤1e-6 rel ΔE;
           "p99 latency")
 FP64_PEAK_TFLOPS = 78.6   # MI355X FP64 vector (and matrix) peak
 HBM_PEAK_GBS = 8000.0     # MI355X HBM3E
-# HBM bytes per launch of McBatchKernel<0> on the default 256-box workload,
-# from rocprofv3 FETCH_SIZE / WRITE_SIZE scaled by a known-size copy
+# Bytes beyond the L2 per launch of McBatchKernel<0> on the default 256-box
+# workload (the memory-side cache holds an unknown part of them), from rocprofv3
+# FETCH_SIZE / WRITE_SIZE scaled by a known-size copy
 # (profiles/McBatchKernel_water256_fp64_hbm.md); reported for that workload.
-PROFILED_TRAFFIC = {"bytes": 239.1e9, "source": "profiles/McBatchKernel_water256_fp64_hbm.md"}
+PROFILED_TRAFFIC = {"bytes": 221.0e9, "source": "profiles/McBatchKernel_water256_fp64_hbm.md"}
 # Fixed per-term FLOP weights of the algorithmic work model: distance +
 # minimum image 12, erfc-Coulomb 30, LJ 15, sincos + 2 FMA 24, per-k energy 6.
 W_DIST, W_COUL, W_LJ, W_SINCOS, W_KENERGY = 12, 30, 15, 24, 6

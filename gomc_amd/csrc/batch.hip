@@ -22,15 +22,21 @@
 // n = 0..nmax, built each pass for the moving molecules' old and new
 // positions (one sincos per table entry), and advanced along nz.
 //
-// What bounds it: instruction issue of the CU's four SIMDs in both phases, FP64
-// at a quarter rate, and then the passes' barriers.  Measured on MI355X, rigid
-// 3-site water, microseconds a move of one box alone, FP64 / mixed, against
-// one move a pass, libm-free erfc by polynomial and FP64 centre tests:
-//   202 waters, 1 workgroup     8.1 /  7.5, was 10.4 /  9.4
-//   985                        10.5 / 10.0, was 14.4 / 12.9
-//   1700                       12.1 / 10.7, was 16.1 / 14.1
-//   2454, team of 2            10.7 /  8.4, was 13.7 / 12.2
-//   3950, team of 8             8.2 /  6.3, was 11.0 / 10.3
+// What bounds it: over a cycle of 256 boxes a SIMD issues a vector instruction in
+// 38 % of its cycles and a wave waits two thirds of its own, at the passes'
+// barriers and for memory; within the pair and reciprocal phases fewer
+// instructions are fewer microseconds.  Measured on MI355X, rigid 3-site water,
+// microseconds a move of one box alone, FP64 / mixed, against one move a pass,
+// libm-free erfc by polynomial and FP64 centre tests:
+//   202 waters, 1 workgroup     7.9 /  7.3, was 10.4 /  9.4
+//   500                         8.9 /  8.2, was 13.3 / 12.3
+//   985                         9.8 /  8.8, was 14.4 / 12.9
+//   1700                       11.6 / 10.4, was 16.1 / 14.1
+//   2454, team of 2             9.8 /  8.0, was 13.7 / 12.2
+//   3950, team of 8             8.1 /  6.3, was 11.0 / 10.3
+// A launch costs more than it did: a workgroup loads its box's pointers, Coulomb
+// table and two programs (one box of 300 waters, 1 / 4 / 40 moves 92 / 120 / 493
+// us a call, was 81 / 116 / 540).
 #include "batch.hpp"
 #include "coul_table.hpp"
 #include "device_common.hpp"
@@ -991,8 +997,10 @@ __device__ __noinline__ void Decide(const LMEM BatchBox *sb, LMEM BatchState *st
 // ------------------------------------------------------------- programs --
 // The pair waves and the reciprocal waves of a workgroup run a program each,
 // a loop over the box's passes with the same four barriers a pass (five where
-// draws are made): called once a box, so the phases' many registers are saved
-// once, not once a pass.  Which moves a pass holds follows from the draws and
+// draws are made): called once a box, so the callee-saved registers of the
+// phases (60 stores a lane in FP64) are saved once, not once a pass, which holds
+// 7 spill stores and 18 loads of its own and the small frames of the
+// out-of-line steps.  Which moves a pass holds follows from the draws and
 // the step alone, so every wave finds it for itself.
 // A run's pointers lie in LDS, one copy a workgroup: in a lane's private memory
 // they were 300 bytes of scratch stored by each of 1024 lanes, and the trace's

@@ -33,8 +33,8 @@ constexpr int kXchgWords = 2 * kTeamMax * kXchgVals;
 // Polls of a member's counter before a team gives up and flags an error.
 constexpr int64_t kTeamSpinLimit = int64_t(1) << 22;
 // Molecules whose FP32 centres are kept in LDS beside the static tables
-// (phase tables of two moves, pair queues, near lists; 78 of the 160 KiB of a
-// CU): 4096 x 12 B.
+// (phase tables of two moves, Coulomb table, pair queues, near lists: 113,752 B
+// in FP64, 101,080 in mixed precision, of a CU's 163,840): 4096 x 12 B.
 constexpr int kBatchLdsMolCap = 4096;
 // Boxes of more molecules skip the centre cull.
 constexpr int kBatchNearCap = 4096;

@@ -98,12 +98,13 @@ int PackBox(gomc_batch *bt, const gomc_system_desc &d, int64_t atomOff, int64_t 
   {
     // Waves for the pair phase; the rest run the reciprocal phase beside
     // it.  Measured on MI355X (water, one workgroup, microseconds a move with
-    // 8 / 12 pair waves, FP64 and mixed): 202 molecules 9.4 / 8.1 and 8.9 /
-    // 7.6, 500 10.0 / 9.0 and 9.5 / 8.5, 985 (3047 k-vectors) 10.5 / 10.1 and
-    // 10.0 / 9.1, 1300 (4021) 12.0 / 12.1 and 10.4 / 10.6, 1700 12.0 / 13.1:
-    // 12 up to 3072 k-vectors, 12 for each thread of the four reciprocal waves.
-    // Teams split the k-vectors and the molecules alike and are fastest with 8
-    // (2454 on two: 8 10.7, 12 11.9; 3950 on eight: 8.2, 8.4).
+    // 8 / 12 pair waves, FP64 and mixed): 202 molecules 9.4 / 8.0 and 8.8 /
+    // 7.3, 500 10.0 / 8.8 and 9.5 / 8.2, 985 (3047 k-vectors) 10.3 / 9.8 and
+    // 9.8 / 8.8, 1300 (4021) 11.2 / 11.7 and 10.2 / 10.4, 1700 11.6 / 12.7 and
+    // 10.4 / 11.4: 12 up to 3072 k-vectors, 12 for each thread of the four
+    // reciprocal waves.  Teams split the k-vectors and the molecules alike and
+    // were fastest with 8 (2454 on two: 8 10.7, 12 11.9; 3950 on eight: 8.2,
+    // 8.4, before the run's pointers moved to LDS).
     const int T = bt->teams ? TeamSize(bt, b->nmols) : 1;
     const int kper = b->ewald ? b->K : 0;
     P.pairWaves = (T == 1 && kper <= bt->tune.pair12_max_k) ? 12 : 8;
@@ -359,13 +360,13 @@ int UploadBox(gomc_batch *bt, int slot, const PackedBox &pb) {
 
 int TeamSize(const gomc_batch *bt, int nmols) {
   // Measured on MI355X (water, microseconds a move in FP64 on 1 / 2 / 4 / 8
-  // workgroups): 1700 molecules 12.2 / 9.9 / 8.2 / 7.9, 2454 16.5 / 10.8 / 8.4
-  // / 7.9, 3300 16.6 / 11.8 / 9.8 / 8.2, 3950 19.9 / 13.3 / 9.9 / 8.3: a member
+  // workgroups): 1700 molecules 11.6 / 9.4 / 8.1 / 7.5, 2454 16.0 / 9.9 / 8.1
+  // / 7.5, 3300 16.0 / 11.5 / 9.5 / 8.2, 3950 19.4 / 13.0 / 9.5 / 8.1: a member
   // repeats about 7 us (draws, trial coordinates, tables, the exchange) and the
   // rest is split.  A cycle ends with its longest box, so the longest get the
   // larger teams; with the default thresholds {1800, 2700, 3500} a 256-box
-  // cycle takes 42 ms, and moving any of them by 100 changes it by less than
-  // 2 % or makes it longer.
+  // cycle takes 38 ms; the best of the autotuner's 29 shapes, {1800, 2900, 3400},
+  // is 1 % shorter, and its others are up to 30 % longer.
   const int32_t *t = bt->tune.team_min;
   if (t[2] > 0 && nmols >= t[2]) return 8;
   if (t[1] > 0 && nmols >= t[1]) return 4;

@@ -107,8 +107,8 @@ __device__ __forceinline__ void TrialAtom(const TrialArgs &a, int j, double xj, 
 //
 // Bound by one thread's chain, not by the chip (a trial of 1000 waters is 100
 // blocks): an item a thread for one atom's two positions, one side's phases a
-// thread, pair terms without calls and one barrier a reduction took the kernel
-// from 14 us to 9.8 for 300 to 1000 waters; all of a molecule's positions
+// thread and one barrier a reduction took the kernel from 14 us to 9 for 300 to
+// 1000 waters; all of a molecule's positions
 // in one thread are six pair terms or sincos in a row.
 constexpr int kTrialK = kBlock / 2;  // k-vectors of a block's run
 // A block takes as many runs as keep the reciprocal blocks to this: each block
@@ -476,7 +476,7 @@ struct ParticleArgs {
 
 // Most threads have one slot or a few: a trial lasts as long as the chain from a
 // cell to its atoms' terms, five dependent loads, so one turn of 1024 threads
-// beats four of 256.  16 trials of 1000 methane / CO2 molecules: 13.9 -> 8.2 us.
+// beats four of 256.  16 trials of 1000 methane / CO2 molecules: 13.9 -> 7.9 us.
 constexpr int kParticleBlock = 1024;
 
 template <int P>

@@ -17,7 +17,9 @@
 //                       molecule, and every k-vector's structure-factor delta,
 //                       reduced in one pass;
 //   CBMC stage          (trial position, atom) pairs spread over the waves,
-//                       each wave summing one pair over every atom;
+//                       each wave summing one pair over the live atoms of the
+//                       27 cells around it (over all live atoms in a small or
+//                       dilute box);
 //   swap reciprocal     every k-vector's new structure factor.
 // Energies are summed in a fixed order, so a run does not depend on timing.
 //
@@ -25,7 +27,7 @@
 // instruction issue and LDS reads, the rest by thread 0's chain of LDS and
 // global loads and by what the 64 KiB instruction cache cannot hold (the loop is
 // 70 KiB).  Microseconds a move in FP64 on MI355X: 1000 methane / CO2 molecules
-// in 40 A 42.8 -> 29 (pair terms without calls or divisions, the neighbour walk
+// in 40 A 42.7 -> 29.5 (pair terms without calls or divisions, the neighbour walk
 // without searches, two k-vectors a set of phases, trials picked by a wave).
 #include <algorithm>
 #include <cmath>

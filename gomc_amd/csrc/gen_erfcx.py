@@ -1,5 +1,5 @@
-"""Generates erfcx_poly.hpp: the polynomial used by the batched kernel's
-FP64 erfc, erfc(x) = exp(-x^2) * erfcx(x) for 0 <= x <= 4.
+"""Generates erfcx_poly.hpp: the polynomial of the FP64 erfc in the
+whole-box forces and virial and in the device move loop, erfc(x) = exp(-x^2) * erfcx(x) for 0 <= x <= 4.
 
 erfcx(x) = exp(x^2) erfc(x) is smooth; it is sampled at 6000 Chebyshev
 nodes of [0, 4.1] (scipy.special.erfcx as the reference values), fitted by a

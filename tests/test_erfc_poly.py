@@ -1,8 +1,8 @@
-"""The batched kernel's FP64 erfc on [0, 4]: exp(-x^2) times a fitted
+"""The FP64 erfc of the force and virial kernels and the device move loop on [0, 4]: exp(-x^2) times a fitted
 polynomial for erfcx (gomc_amd/csrc/erfcx_poly.hpp).  Pinned against
 scipy.special.erfc on a dense grid (relative error below 5e-15), at
 erfc(0) = 1 and against the series erfc(x) = 1 - 2x/sqrt(pi) + 2x^3/(3
-sqrt(pi)) - ... near 0.  The kernel evaluates the same Horner form in
+sqrt(pi)) - ... near 0.  The kernels evaluate the same Horner form in
 double precision."""
 import math
 import re
