@@ -34,9 +34,10 @@
 //   1700                       11.6 / 10.4, was 16.1 / 14.1
 //   2454, team of 2             9.8 /  8.0, was 13.7 / 12.2
 //   3950, team of 8             8.1 /  6.3, was 11.0 / 10.3
-// A launch costs more than it did: a workgroup loads its box's pointers, Coulomb
-// table and two programs (one box of 300 waters, 1 / 4 / 40 moves 92 / 120 / 493
-// us a call, was 81 / 116 / 540).
+// A launch itself costs 10 us more in the kernel: a workgroup loads its box's
+// pointers, Coulomb table and two programs.  The calls are shorter all the same
+// (one box of 300 waters, 1 / 4 / 40 moves 76 / 104 / 479 us, was 80 / 115 / 540):
+// the host copies and waits less.
 #include "batch.hpp"
 #include "coul_table.hpp"
 #include "device_common.hpp"

@@ -142,11 +142,11 @@ struct gomc_batch {
   // the table of the box packed last: boxes of one alpha and cutoff share it
   std::shared_ptr<const gomc::CoulTable> table;
   int64_t *moves = nullptr;
-  // workgroup task lists (device) and their capacity; team exchange blocks
+  // behind `moves`: the lists' starts and the workgroups' task lists
   gomc::BatchTask *tasks = nullptr;
   int *wgTask = nullptr;
-  uint64_t *xchg = nullptr;
-  int *errFlag = nullptr;
+  uint64_t *xchg = nullptr;  // team exchange blocks
+  int *errFlag = nullptr;  // the word behind boxTicks
   int grid = 0;        // workgroups per launch
   int gridCap = 0;     // workgroups that fit on the device at once
   bool teams = true;   // false: every box runs on one workgroup (serving)
@@ -202,7 +202,7 @@ int AllocBatch(gomc_batch *bt, int nboxes, int64_t atoms, int64_t mols, int64_t 
 // Team size of a box of n molecules (a function of n alone, so a box's
 // results do not depend on the other boxes of its batch).
 int TeamSize(const gomc_batch *bt, int nmols);
-// Builds and uploads the workgroup task lists for the given move counts.
+// Builds the workgroup task lists for the given move counts and uploads both.
 int BuildTasks(gomc_batch *bt, const std::vector<int64_t> &moves);
 // Uploads a packed box: parameters and state at index `slot`, arrays at
 // the box's offsets.
